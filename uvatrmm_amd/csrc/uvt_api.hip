@@ -36,7 +36,7 @@ struct PartSum {
 
 // PARTS: the records are LaunchTiles (some write partial tiles); else plain
 // uvt_tiles, every one writing C.
-template <int TM, int TN, bool VEC, bool PARTS>
+template <int TM, int TN, bool PARTS>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__ A, int64_t lda,
@@ -49,12 +49,12 @@ void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__
         const LaunchTile lt = static_cast<const LaunchTile*>(tiles)[blockIdx.x];
         const uvt_tile& t = lt.t;
         UVT_GLOBAL double* part = lt.part >= 0 ? gbl(parts) + (int64_t)lt.part * (TM * TN) : nullptr;
-        f64_tile<TM, TN, VEC, W::M, W::N>(t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags, gbl(A), lda,
-                                          gbl(B), ldb, gbl(C), ldc, m, smem, -1, part);
+        f64_tile<TM, TN, W::M, W::N>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
+                                     ldb, gbl(C), ldc, m, smem, -1, part);
     } else {
         const uvt_tile t = static_cast<const uvt_tile*>(tiles)[blockIdx.x];
-        f64_tile<TM, TN, VEC, W::M, W::N>(t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags, gbl(A), lda,
-                                          gbl(B), ldb, gbl(C), ldc, m, smem);
+        f64_tile<TM, TN, W::M, W::N>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
+                                     ldb, gbl(C), ldc, m, smem);
     }
 }
 
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void k_add_parts(const PartSum* __restrict__ s
 
 // The trapezoid walk without a tile list: workgroup b takes row tile
 // nrt-1-b/nct (longest reduction first) and column tile b%nct.
-template <int TM, int TN, bool VEC>
+template <int TM, int TN>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, const double* __restrict__ A,
@@ -91,8 +91,8 @@ void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, const double* 
     const int rt = nrt - 1 - (int)(blockIdx.x / nct), ct = (int)(blockIdx.x % nct);
     const int r0 = rt * TM;
     const int rows = (int)(n - r0 < TM ? n - r0 : TM);
-    f64_tile<TM, TN, VEC, W::M, W::N>(r0, rows, ct * TN, 0, r0 + rows, kTileLower, gbl(A), lda,
-                                      gbl(B), ldb, gbl(C), ldc, m, smem);
+    f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, ct * TN, 0, r0 + rows, kTileLower}, gbl(A), lda, gbl(B), ldb,
+                                 gbl(C), ldc, m, smem);
 }
 
 // The trapezoid walk split stream-K (uvt_sk.hpp): workgroup w of group
@@ -100,15 +100,16 @@ void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, const double* 
 // another, in column tile w % ncg of each piece's row tile when the launch
 // runs column groups; its first piece writes partial tile w if it starts
 // inside its tile, every other piece starts at k = 0 and writes C.
-template <int TM, int TN, bool VEC>
+template <int TM, int TN>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_trmm_sk_f64(SkGeo g, const double* __restrict__ A, int64_t lda, const double* __restrict__ B,
                    int64_t ldb, double* __restrict__ C, int64_t ldc, double* __restrict__ parts)
 {
     using W = TileWaves<TM, TN>;
-    static_assert(F64Cfg<TM, TN, W::M, W::N>::BK == kSkPanel, "stream-K panels are the kernel's k panels");
-    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N>::SMEM_DOUBLES];
+    using Opt = TileOpt<true, false, kTriALe, false, false, false>;
+    static_assert(kTileK == kSkPanel, "stream-K panels are the kernel's k panels");
+    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
     // The piece arithmetic (64-bit divisions) runs in vector registers; its
     // results are the same in every lane and go back to scalar registers, so
     // they do not take vector registers from the tile.
@@ -134,9 +135,9 @@ void k_trmm_sk_f64(SkGeo g, const double* __restrict__ A, int64_t lda, const dou
         // the piece loop
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
-        f64_tile<TM, TN, VEC, W::M, W::N, kSkPanel, false>(uni(s.r0), uni(s.rows), uni(s.c0 + cx), uni(s.k_lo), uni(s.k_hi),
-                                          kTileLower, gbl(A), lda, gbl(B), ldb, gbl(C), ldc, g.m, smem,
-                                          tid, uni(s.p0 > 0) ? part : nullptr);
+        const TileArgs t{uni(s.r0), uni(s.rows), uni(s.c0 + cx), uni(s.k_lo), uni(s.k_hi), kTileLower};
+        f64_tile<TM, TN, W::M, W::N, Opt>(t, gbl(A), lda, gbl(B), ldb, gbl(C), ldc, g.m, smem, tid,
+                                          uni(s.p0 > 0) ? part : nullptr);
         first = false;
         x = uni64(s.next);
     }
@@ -504,26 +505,16 @@ static uvt_status plan_upload(uvt_handle h, uvt_plan plan)
 
 // parts == nullptr: dtiles holds uvt_tiles; else LaunchTiles.
 template <int TM, int TN>
-static void launch_tiles(const void* dtiles, int64_t ntiles, bool vec, const double* A,
-                         int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc,
-                         int64_t m, double* parts, hipStream_t s)
+static void launch_tiles(const void* dtiles, int64_t ntiles, const double* A, int64_t lda, const double* B,
+                         int64_t ldb, double* C, int64_t ldc, int64_t m, double* parts, hipStream_t s)
 {
-    dim3 grid((unsigned)ntiles), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    if (parts) {
-        if (vec)
-            hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, true, true>), grid, block, 0, s, dtiles, A, lda,
-                               B, ldb, C, ldc, m, parts);
-        else
-            hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, false, true>), grid, block, 0, s, dtiles, A, lda,
-                               B, ldb, C, ldc, m, parts);
-    } else {
-        if (vec)
-            hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, true, false>), grid, block, 0, s, dtiles, A, lda,
-                               B, ldb, C, ldc, m, parts);
-        else
-            hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, false, false>), grid, block, 0, s, dtiles, A, lda,
-                               B, ldb, C, ldc, m, parts);
-    }
+    const dim3 grid((unsigned)ntiles), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
+    if (parts)
+        hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, true>), grid, block, 0, s, dtiles, A, lda, B, ldb, C, ldc, m,
+                           parts);
+    else
+        hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, false>), grid, block, 0, s, dtiles, A, lda, B, ldb, C, ldc, m,
+                           parts);
 }
 
 static uvt_status launch_tiles_f64(int32_t cfg, const void* dtiles, int64_t ntiles,
@@ -532,45 +523,29 @@ static uvt_status launch_tiles_f64(int32_t cfg, const void* dtiles, int64_t ntil
 {
     if (ntiles <= 0) return UVT_OK;
     if (ntiles > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && lda % 2 == 0 &&
-                     ldb % 2 == 0;
-    if (cfg == UVT_CFG_256x128)
-        launch_tiles<256, 128>(dtiles, ntiles, vec, A, lda, B, ldb, C, ldc, m, parts, s);
-    else if (cfg == UVT_CFG_64x64)
-        launch_tiles<64, 64>(dtiles, ntiles, vec, A, lda, B, ldb, C, ldc, m, parts, s);
-    else if (cfg == UVT_CFG_128x32)
-        launch_tiles<128, 32>(dtiles, ntiles, vec, A, lda, B, ldb, C, ldc, m, parts, s);
-    else
-        launch_tiles<128, 128>(dtiles, ntiles, vec, A, lda, B, ldb, C, ldc, m, parts, s);
+    if (cfg == UVT_CFG_256x128) launch_tiles<256, 128>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+    else if (cfg == UVT_CFG_64x64) launch_tiles<64, 64>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+    else if (cfg == UVT_CFG_128x32) launch_tiles<128, 32>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+    else launch_tiles<128, 128>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }
 
 template <int TM, int TN>
-static void launch_trapezoid(bool vec, int64_t n, int64_t m, const double* A, int64_t lda,
-                             const double* B, int64_t ldb, double* C, int64_t ldc, hipStream_t s)
+static void launch_trapezoid(int64_t n, int64_t m, const double* A, int64_t lda, const double* B, int64_t ldb,
+                             double* C, int64_t ldc, hipStream_t s)
 {
     const int nrt = (int)((n + TM - 1) / TM), nct = (int)((m + TN - 1) / TN);
     const dim3 grid((unsigned)((int64_t)nrt * nct)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    if (vec)
-        hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN, true>), grid, block, 0, s, n, m, nrt, nct, A,
-                           lda, B, ldb, C, ldc);
-    else
-        hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN, false>), grid, block, 0, s, n, m, nrt, nct,
-                           A, lda, B, ldb, C, ldc);
+    hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN>), grid, block, 0, s, n, m, nrt, nct, A, lda, B, ldb, C, ldc);
 }
 
 template <int TM, int TN>
-static void launch_trapezoid_sk(bool vec, const SkGeo& g, const double* A, int64_t lda, const double* B,
-                                int64_t ldb, double* C, int64_t ldc, double* parts, hipStream_t s)
+static void launch_trapezoid_sk(const SkGeo& g, const double* A, int64_t lda, const double* B, int64_t ldb,
+                                double* C, int64_t ldc, double* parts, hipStream_t s)
 {
     const dim3 grid((unsigned)sk_launch(g)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    if (vec)
-        hipLaunchKernelGGL((k_trmm_sk_f64<TM, TN, true>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc,
-                           parts);
-    else
-        hipLaunchKernelGGL((k_trmm_sk_f64<TM, TN, false>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc,
-                           parts);
+    hipLaunchKernelGGL((k_trmm_sk_f64<TM, TN>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc, parts);
     hipLaunchKernelGGL((k_sk_fixup<TM, TN>), dim3((unsigned)sk_launch(g), 4), dim3(256), 0, s, g, parts, C, ldc);
 }
 
@@ -645,11 +620,9 @@ uvt_status uvt_launch_trapezoid_sk_f64(int32_t cfg, int64_t n, int64_t m, const 
     if (cfg == UVT_CFG_256x128) return UVT_ERR_ARG;  // stream-K runs 128x128 tiles (uvt_sk_workgroups)
     if (n > 0x3FFFFFFF || m > 0x3FFFFFFF || workgroups > 0x7FFFFFFF) return UVT_ERR_SIZE;
     const SkGeo g = sk_geometry(n, m, uvt_cfg_tile_m(cfg), uvt_cfg_tile_n(cfg), workgroups, kSkGroupCols);
-    const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && lda % 2 == 0 &&
-                     ldb % 2 == 0;
-    if (cfg == UVT_CFG_64x64) launch_trapezoid_sk<64, 64>(vec, g, A, lda, B, ldb, C, ldc, parts, s);
-    else if (cfg == UVT_CFG_128x32) launch_trapezoid_sk<128, 32>(vec, g, A, lda, B, ldb, C, ldc, parts, s);
-    else launch_trapezoid_sk<128, 128>(vec, g, A, lda, B, ldb, C, ldc, parts, s);
+    if (cfg == UVT_CFG_64x64) launch_trapezoid_sk<64, 64>(g, A, lda, B, ldb, C, ldc, parts, s);
+    else if (cfg == UVT_CFG_128x32) launch_trapezoid_sk<128, 32>(g, A, lda, B, ldb, C, ldc, parts, s);
+    else launch_trapezoid_sk<128, 128>(g, A, lda, B, ldb, C, ldc, parts, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }
@@ -662,12 +635,10 @@ uvt_status uvt_launch_trapezoid_f64(int32_t cfg, int64_t n, int64_t m, const dou
     if (n > 0x3FFFFFFF || m > 0x3FFFFFFF) return UVT_ERR_SIZE;
     const int64_t tm = uvt_cfg_tile_m(cfg), tn = uvt_cfg_tile_n(cfg);
     if (((n + tm - 1) / tm) * ((m + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && lda % 2 == 0 &&
-                     ldb % 2 == 0;
-    if (cfg == UVT_CFG_256x128) launch_trapezoid<256, 128>(vec, n, m, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_64x64) launch_trapezoid<64, 64>(vec, n, m, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_128x32) launch_trapezoid<128, 32>(vec, n, m, A, lda, B, ldb, C, ldc, s);
-    else launch_trapezoid<128, 128>(vec, n, m, A, lda, B, ldb, C, ldc, s);
+    if (cfg == UVT_CFG_256x128) launch_trapezoid<256, 128>(n, m, A, lda, B, ldb, C, ldc, s);
+    else if (cfg == UVT_CFG_64x64) launch_trapezoid<64, 64>(n, m, A, lda, B, ldb, C, ldc, s);
+    else if (cfg == UVT_CFG_128x32) launch_trapezoid<128, 32>(n, m, A, lda, B, ldb, C, ldc, s);
+    else launch_trapezoid<128, 128>(n, m, A, lda, B, ldb, C, ldc, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }

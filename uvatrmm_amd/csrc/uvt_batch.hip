@@ -64,12 +64,12 @@ struct BatchProb {
 // depend on the wave layout, so a tile gives the same bits as the
 // single-problem kernels' tiles of the same shape.
 constexpr int kBatchThreads = 512;
-template <bool VEC>
 __global__ __launch_bounds__(kBatchThreads, 4)
 void k_batch_f64(const BatchTile* __restrict__ tiles, int ntiles, const BatchProb* __restrict__ probs,
                  int* __restrict__ counter)
 {
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES];
+    using Opt = TileOpt<true, false, kTriALe, false, false, true, true>;
     static_assert(F64Cfg<64, 64, 2, 4>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 64, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 32, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES,
@@ -78,7 +78,7 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, int ntiles, const BatchPro
     for (;;) {
         if (threadIdx.x == 0) next = atomicAdd(counter, 1);
         __syncthreads();
-        const int t = next;
+        const int t = __builtin_amdgcn_readfirstlane(next);  // uniform: its records load into scalar registers
         __syncthreads();  // every thread has read `next` before it is overwritten
         if (t >= ntiles) break;
         const BatchTile bt = tiles[t];
@@ -86,18 +86,21 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, int ntiles, const BatchPro
         // p.pad is always 0, but loaded per tile: the thread index built from
         // it keeps each shape's offset arithmetic inside its own branch
         const int tid = (int)threadIdx.x + p.pad;
-        if (bt.cfg == UVT_CFG_64x64)
-            f64_tile<64, 64, VEC, 2, 4, 16, true, true>(bt.r0, bt.rows, bt.c0, bt.k_lo, bt.k_hi, kTileLower, gbl(p.A),
-                                        p.lda, gbl(p.B), p.ldb, gbl(p.C), p.ldc, p.m, smem, tid);
-        else if (bt.cfg == UVT_CFG_128x64)
-            f64_tile<128, 64, VEC, 4, 2, 16, true, true>(bt.r0, bt.rows, bt.c0, bt.k_lo, bt.k_hi, kTileLower, gbl(p.A),
-                                         p.lda, gbl(p.B), p.ldb, gbl(p.C), p.ldc, p.m, smem, tid);
-        else if (bt.cfg == UVT_CFG_128x32)
-            f64_tile<128, 32, VEC, 4, 2, 16, true, true>(bt.r0, bt.rows, bt.c0, bt.k_lo, bt.k_hi, kTileLower, gbl(p.A),
-                                         p.lda, gbl(p.B), p.ldb, gbl(p.C), p.ldc, p.m, smem, tid);
-        else
-            f64_tile<128, 128, VEC, 4, 2, 16, true, true>(bt.r0, bt.rows, bt.c0, bt.k_lo, bt.k_hi, kTileLower, gbl(p.A),
-                                          p.lda, gbl(p.B), p.ldb, gbl(p.C), p.ldc, p.m, smem, tid);
+        const TileArgs ta{bt.r0, bt.rows, bt.c0, bt.k_lo, bt.k_hi, kTileLower};
+        auto run = [&](auto tm, auto tn, auto wm, auto wn) {
+            f64_tile<tm(), tn(), wm(), wn(), Opt>(ta, gbl(p.A), p.lda, gbl(p.B), p.ldb, gbl(p.C), p.ldc, p.m, smem,
+                                                  tid);
+        };
+        using std::integral_constant;
+        constexpr integral_constant<int, 2> i2{};
+        constexpr integral_constant<int, 4> i4{};
+        constexpr integral_constant<int, 32> i32{};
+        constexpr integral_constant<int, 64> i64{};
+        constexpr integral_constant<int, 128> i128{};
+        if (bt.cfg == UVT_CFG_64x64) run(i64, i64, i2, i4);
+        else if (bt.cfg == UVT_CFG_128x64) run(i128, i64, i4, i2);
+        else if (bt.cfg == UVT_CFG_128x32) run(i128, i32, i4, i2);
+        else run(i128, i128, i4, i2);
         __syncthreads();  // the LDS tile is reused by the next tile
     }
 }
@@ -112,7 +115,7 @@ __global__ void k_zero_ints(int* p, int n)
 int persistent_grid(int cus)
 {
     int b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_batch_f64<true>, kBatchThreads, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_batch_f64, kBatchThreads, 0) != hipSuccess ||
         b < 1) {
         (void)hipGetLastError();
         b = 1;
@@ -120,12 +123,11 @@ int persistent_grid(int cus)
     return cus * b;
 }
 
-void launch_persistent(bool vec, int grid, const BatchTile* tiles, int ntiles, const BatchProb* probs,
+void launch_persistent(int grid, const BatchTile* tiles, int ntiles, const BatchProb* probs,
                        int* counter, hipStream_t s)
 {
     const dim3 g((unsigned)std::max(1, std::min(grid, ntiles))), block(kBatchThreads);
-    if (vec) hipLaunchKernelGGL(k_batch_f64<true>, g, block, 0, s, tiles, ntiles, probs, counter);
-    else hipLaunchKernelGGL(k_batch_f64<false>, g, block, 0, s, tiles, ntiles, probs, counter);
+    hipLaunchKernelGGL(k_batch_f64, g, block, 0, s, tiles, ntiles, probs, counter);
 }
 
 // ---- tuning table ------------------------------------------------------------
@@ -243,9 +245,8 @@ struct uvt_batch_s {
     // FP64 part
     std::vector<int> f64_index;        // problem -> slot in the FP64 table
     std::vector<BatchProb> f64_probs;  // host image
-    // one queue of every tile shape per 16-byte load path: index vec
-    std::vector<BatchTile> tiles[2];
-    BatchTile* d_tiles[2] = {nullptr, nullptr};
+    std::vector<BatchTile> tiles;  // one queue of every tile shape
+    BatchTile* d_tiles = nullptr;
     BatchProb* d_probs = nullptr;
     int* d_counters = nullptr;
     // split part (problems that run the integer stages)
@@ -276,8 +277,7 @@ static void batch_free(uvt_batch b)
     if (b->join) (void)hipEventDestroy(b->join);
     if (b->cap) (void)hipStreamDestroy(b->cap);
     if (b->side) (void)hipStreamDestroy(b->side);
-    for (auto& p : b->d_tiles)
-        if (p) (void)hipFree(p);
+    if (b->d_tiles) (void)hipFree(b->d_tiles);
     if (b->d_probs) (void)hipFree(b->d_probs);
     if (b->d_counters) (void)hipFree(b->d_counters);
     if (b->d_split_work) (void)hipFree(b->d_split_work);
@@ -369,14 +369,13 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         b->f64_probs.push_back(f64_desc(p));
         const int cfg = table.empty() ? uvt_default_cfg(p.n, p.m) : uvt_tune_pick(table, p.n, p.m);
         const bool use_int8 = routes_to_int8(p, slices);
-        trapezoid_tiles(slot, p.n, p.m, cfg, b->tiles[b->f64_probs.back().vec], use_int8);
+        trapezoid_tiles(slot, p.n, p.m, cfg, b->tiles, use_int8);
         b->int8.push_back(use_int8);
         if (use_int8) b->int8_flops += (double)p.m * (double)p.n * (double)p.n;
         if (use_int8) b->sp.push_back(uvt_split_problem{p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.n, p.m});
     }
-    for (auto& v : b->tiles) sort_longest_first(v);
-    for (auto& v : b->tiles)
-        if (v.size() > 0x7FFFFFFF) st = UVT_ERR_SIZE;
+    sort_longest_first(b->tiles);
+    if (b->tiles.size() > 0x7FFFFFFF) st = UVT_ERR_SIZE;
     if (st != UVT_OK) {
         batch_free(b);
         return st;
@@ -390,12 +389,10 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         }                                \
     } while (0)
     // FP64 buffers
-    for (int c = 0; c < 2; ++c)
-        if (!b->tiles[c].empty()) {
-            BATCH_HIP(hipMalloc(&b->d_tiles[c], b->tiles[c].size() * sizeof(BatchTile)));
-            BATCH_HIP(hipMemcpy(b->d_tiles[c], b->tiles[c].data(), b->tiles[c].size() * sizeof(BatchTile),
-                                hipMemcpyHostToDevice));
-        }
+    if (!b->tiles.empty()) {
+        BATCH_HIP(hipMalloc(&b->d_tiles, b->tiles.size() * sizeof(BatchTile)));
+        BATCH_HIP(hipMemcpy(b->d_tiles, b->tiles.data(), b->tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
+    }
     if (!b->f64_probs.empty()) {
         BATCH_HIP(hipMalloc(&b->d_probs, b->f64_probs.size() * sizeof(BatchProb)));
         BATCH_HIP(hipMemcpy(b->d_probs, b->f64_probs.data(), b->f64_probs.size() * sizeof(BatchProb),
@@ -445,10 +442,8 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         st = uvt_split_batch_launch(b->sp.data(), (int)b->sp.size(), slices, b->d_split_work,
                                     b->d_split_desc, b->d_split_lut, b->split_totals, b->split_lut_off,
                                     b->side, UVT_SPLIT_GEMM);
-    for (int q = 0; q < 2; ++q)
-        if (!b->tiles[q].empty())
-            launch_persistent(q == 1, grid, b->d_tiles[q], (int)b->tiles[q].size(), b->d_probs,
-                              b->d_counters + 16 * q, b->cap);
+    if (!b->tiles.empty())
+        launch_persistent(grid, b->d_tiles, (int)b->tiles.size(), b->d_probs, b->d_counters, b->cap);
     BATCH_HIP(hipEventRecord(b->join, b->side));
     BATCH_HIP(hipStreamWaitEvent(b->cap, b->join, 0));
     // the reconstruction adds to the diagonal blocks the FP64 queue stored
@@ -485,7 +480,7 @@ extern "C" uvt_status uvt_batch_update(uvt_batch b, const uvt_problem* probs, in
         if (p.n != q.n || p.m != q.m || p.prec != q.prec || p.route != q.route) return UVT_ERR_ARG;
         uvt_status st = check(p);
         if (st != UVT_OK) return st;
-        // the 16-byte load path was fixed at capture time
+        // operands keep the alignment they were planned with
         if (f64_desc(p).vec != b->f64_probs[b->f64_index[i]].vec) return UVT_ERR_ARG;
     }
     UVT_HIP(hipSetDevice(b->h->device));
@@ -509,11 +504,7 @@ extern "C" uvt_status uvt_batch_info(uvt_batch b, double* flops, double* int8_fl
     if (!b) return UVT_ERR_ARG;
     if (flops) *flops = b->flops;
     if (int8_flops) *int8_flops = b->int8_flops;
-    if (fp64_tiles) {
-        int64_t t = 0;
-        for (auto& v : b->tiles) t += (int64_t)v.size();
-        *fp64_tiles = t;
-    }
+    if (fp64_tiles) *fp64_tiles = (int64_t)b->tiles.size();
     if (graph_nodes) *graph_nodes = (int32_t)b->nodes;
     return UVT_OK;
 }
@@ -626,7 +617,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
                 for (int rep = 0; rep < 4; ++rep) {
                     hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, counter, 16);
                     (void)hipEventRecord(e0, s);
-                    launch_persistent(true, grid, dtiles, (int)tiles.size(), dprobs, counter, s);
+                    launch_persistent(grid, dtiles, (int)tiles.size(), dprobs, counter, s);
                     (void)hipEventRecord(e1, s);
                     float ms_ = 0.f;
                     if (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms_, e0, e1) != hipSuccess) {

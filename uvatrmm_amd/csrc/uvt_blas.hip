@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void k_axpby(int64_t rows, int64_t cols, doubl
 }
 
 // Rectangle C[0:M, 0:N] = A[0:M, 0:K] * B[0:K, 0:N] on the FP64 tile.
-template <int TM, int TN, bool VEC>
+template <int TM, int TN>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_gemm_f64(int64_t M, int64_t N, int K, int nct, const double* __restrict__ A, int64_t lda,
@@ -121,26 +121,20 @@ void k_gemm_f64(int64_t M, int64_t N, int K, int nct, const double* __restrict__
     const int rt = (int)(blockIdx.x / nct), ct = (int)(blockIdx.x % nct);
     const int r0 = rt * TM;
     const int rows = (int)(M - r0 < TM ? M - r0 : TM);
-    f64_tile<TM, TN, VEC, W::M, W::N>(r0, rows, ct * TN, 0, K, 0, gbl(A), lda, gbl(B), ldb, gbl(C),
-                                      ldc, N, smem);
+    f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, ct * TN, 0, K, 0}, gbl(A), lda, gbl(B), ldb, gbl(C), ldc, N,
+                                 smem);
 }
 
 template <int TM, int TN>
-void launch_gemm(bool vec, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda,
-                 const double* B, int64_t ldb, double* C, int64_t ldc, hipStream_t s)
+void launch_gemm(int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, const double* B, int64_t ldb,
+                 double* C, int64_t ldc, hipStream_t s)
 {
     const int nrt = (int)((M + TM - 1) / TM), nct = (int)((N + TN - 1) / TN);
     const dim3 grid((unsigned)((int64_t)nrt * nct));
     const dim3 block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    if (vec)
-        hipLaunchKernelGGL((k_gemm_f64<TM, TN, true>), grid, block, 0, s, M, N, (int)K, nct, A, lda,
-                           B, ldb, C, ldc);
-    else
-        hipLaunchKernelGGL((k_gemm_f64<TM, TN, false>), grid, block, 0, s, M, N, (int)K, nct, A,
-                           lda, B, ldb, C, ldc);
+    hipLaunchKernelGGL((k_gemm_f64<TM, TN>), grid, block, 0, s, M, N, (int)K, nct, A, lda, B, ldb, C, ldc);
 }
 
-bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 int64_t even(int64_t x) { return x + (x & 1); }
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -176,10 +170,9 @@ uvt_status uvt_launch_gemm_f64(int32_t cfg, int64_t M, int64_t N, int64_t K, con
     if (!sizes_ok(M, N, K)) return UVT_ERR_SIZE;
     const int64_t tm = uvt_cfg_tile_m(cfg), tn = uvt_cfg_tile_n(cfg);
     if (((M + tm - 1) / tm) * ((N + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    const bool vec = aligned16(A) && aligned16(B) && lda % 2 == 0 && ldb % 2 == 0;
-    if (cfg == UVT_CFG_64x64) launch_gemm<64, 64>(vec, M, N, K, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_128x32) launch_gemm<128, 32>(vec, M, N, K, A, lda, B, ldb, C, ldc, s);
-    else launch_gemm<128, 128>(vec, M, N, K, A, lda, B, ldb, C, ldc, s);
+    if (cfg == UVT_CFG_64x64) launch_gemm<64, 64>(M, N, K, A, lda, B, ldb, C, ldc, s);
+    else if (cfg == UVT_CFG_128x32) launch_gemm<128, 32>(M, N, K, A, lda, B, ldb, C, ldc, s);
+    else launch_gemm<128, 128>(M, N, K, A, lda, B, ldb, C, ldc, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }

@@ -8,23 +8,25 @@
 //   * the triangle  C[b+1:b+h] += tril(A_tri) * B_tri       (mask, accumulate)
 //   * the trapezoid C[r0:r0+TM] = A[r0:, 0:r0+TM] * B        (mask, store)
 //
-// Data path: A and B k-panels (BK = 16 deep) stream from HBM with 16-byte
-// loads into registers one panel ahead (two with AHEAD2), are written to a double-buffered LDS
-// tile, and each wave multiplies its (TM/WAVES_M) x (TN/WAVES_N) sub-tile with
-// v_mfma_f64_16x16x4_f64 (one double of A and B per lane, four doubles of
-// C per lane).  A keeps its row-major layout in LDS (rows of BK + 2 doubles)
-// and B its k-major one, so every LDS write is one 16-byte piece a thread
-// loaded; the writes for the next panel are issued during the current
-// panel's products (see compute()), and each lane reads its A values for a
-// panel as 16-byte pairs of one row.  (A transposed to k-major on the way in took
-// four conflicting 8-byte writes per thread and cost about 10 % of the MFMA
-// rate, measured register-only.)
+// Data path: A and B k-panels (16 deep) stream from HBM with 16-byte loads
+// into registers one panel ahead (two with AHEAD2), are written to a
+// double-buffered LDS tile, and each wave multiplies its (TM/WAVES_M) x
+// (TN/WAVES_N) sub-tile with v_mfma_f64_16x16x4_f64 (one double of A and B
+// per lane, four doubles of C per lane).  Each operand keeps its memory
+// layout in LDS (struct Panel), so every LDS write is one 16-byte piece a
+// thread loaded; the writes for the next panel are issued during the current
+// panel's products (see compute()), and each lane reads its values of a
+// k-contiguous operand as 16-byte pairs of one row.  (A transposed to k-major
+// on the way in took four conflicting 8-byte writes per thread and cost about
+// 10 % of the MFMA rate, measured register-only.)
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <type_traits>
+
+#include "uvt_panel.hpp"
 
 namespace uvt {
 
@@ -51,34 +53,157 @@ __device__ __forceinline__ UVT_GLOBAL T* gbl(T* p)
 constexpr int kTileLower = 1;  // UVT_TILE_LOWER
 constexpr int kTileAccum = 2;  // UVT_TILE_ACCUM
 
-template <int TM, int TN, int WAVES_M = 2, int WAVES_N = 2, int BK_ = 16>
-struct F64Cfg {
-    static constexpr int NT = 64 * WAVES_M * WAVES_N;
-    static constexpr int BK = BK_;  // k depth of one LDS panel (BK/4 MFMA steps)
-    static constexpr int WM = TM / WAVES_M, WN = TN / WAVES_N;
-    static constexpr int FM = WM / 16, FN = WN / 16;
-    // LDS row strides (doubles).  A: row-major rows of BK + 2 doubles (144 B,
-    // 16-byte aligned; the 16 rows a fragment read touches fall on distinct
-    // bank pairs).  B: k rows of TN + 16 doubles; a fragment read touches four
-    // k rows BK/4 apart (the k order of compute()), which share one half of
-    // the 64 LDS banks (a pitch of TN + 4, alternating halves, measured the same).
-    static constexpr int SA = BK + 2;
-    static constexpr int LDB_S = TN + 16;
-    static constexpr int A_ELEMS = TM * SA;
-    static constexpr int B_ELEMS = BK * LDB_S;
-    static constexpr int SMEM_DOUBLES = 2 * (A_ELEMS + B_ELEMS);
-    // 2-double pieces of a panel, and per thread (a panel smaller than the
-    // workgroup leaves the last threads idle for it: B_PART / A_PART)
-    static constexpr int A_PIECES = TM * BK / 2, B_PIECES = TN * BK / 2;
-    static constexpr int A_VEC = (A_PIECES + NT - 1) / NT;
-    static constexpr int B_VEC = (B_PIECES + NT - 1) / NT;
-    static constexpr bool A_PART = A_PIECES < NT, B_PART = B_PIECES < NT;
-    static_assert(A_PIECES % NT == 0 || A_PART, "uneven A panel split");
-    static_assert(B_PIECES % NT == 0 || B_PART, "uneven B panel split");
-    static_assert(FM >= 1 && FN >= 1, "wave tile below 16x16");
+// Two doubles at an 8-byte aligned address: one 16-byte global load (global
+// memory takes 16-byte accesses at any 4-byte alignment), so odd leading
+// dimensions load like even ones.
+typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// One operand's panel of a tile on its way from memory to LDS (uvt_panel.hpp:
+// which elements).  Its layout in LDS is the one it has in memory:
+//   KC:  rows of kTileK + 2 doubles (144 B, 16-byte aligned; the 16 rows a
+//        fragment read touches fall on distinct bank pairs);
+//   !KC: k rows of X + 16 doubles; a fragment read touches four k rows
+//        kTileK/4 apart (the k order of f64_tile), which share one half of
+//        the 64 LDS banks (a pitch of X + 4, alternating halves, measured
+//        the same).
+// Edge tiles run the steady state like any other.  With every element of
+// every panel of an edge tile checked instead, the edge tiles were the last
+// to finish: 8165 x 939 took 1193 us instead of 1081, a 1500 x 2000 x 3000
+// dgemm in 64x64 tiles 387 instead of 342 (same bits).
+template <int X, int NT, bool KC>
+struct Panel {
+    using Idx = PanelIdx<X, NT, KC>;
+    static constexpr int LD = KC ? kTileK + 2 : X + 16;
+    static constexpr int ELEMS = KC ? X * LD : kTileK * LD;
+    static constexpr int PIECES = Idx::PIECES, VEC = Idx::VEC;
+    static constexpr bool PART = Idx::PART;
+    // Steady-state addresses: a wave-uniform base (scalar registers, moved from
+    // panel to panel) plus a byte offset per thread that never changes; one
+    // offset serves all of a thread's pieces of an x-contiguous panel.
+    static constexpr int OFFS = KC ? VEC : 1;
+
+    const UVT_GLOBAL double* p;  // element (x0, k = 0)
+    int64_t ld;
+    int nx;  // rows (columns) inside the matrix, 1 .. X
+    int x0;  // the tile's first row (column): the triangle's coordinate
+    const UVT_GLOBAL char* at;
+    uint32_t off[OFFS];
+    dbl2 r[VEC];
+
+    __device__ __forceinline__ void init(int tid, const UVT_GLOBAL double* p_, int64_t ld_, int nx_, int x0_)
+    {
+        p = p_;
+        ld = ld_;
+        nx = nx_;
+        x0 = x0_;
+#pragma unroll
+        for (int q = 0; q < OFFS; ++q) {
+            const int v = tid + q * NT, x = Idx::full_x(v, nx), k = Idx::pk(v);
+            off[q] = 8u * (KC ? (uint32_t)x * (uint32_t)ld + (uint32_t)k : (uint32_t)k * (uint32_t)ld + (uint32_t)x);
+        }
+    }
+
+    static __device__ __forceinline__ int lds(int v)
+    {
+        return KC ? Idx::px(v) * LD + Idx::pk(v) : Idx::pk(v) * LD + Idx::px(v);
+    }
+    // load() reads the panel here next.
+    __device__ __forceinline__ void seek(int k0)
+    {
+        at = reinterpret_cast<const UVT_GLOBAL char*>(KC ? p + k0 : p + (int64_t)k0 * ld);
+    }
+    // The next panel in k, a full one.
+    __device__ __forceinline__ void load(int tid)
+    {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) {
+            if (PART && tid + q * NT >= PIECES) break;
+            // the 32-bit offset, opaque here: the access then takes it beside
+            // the scalar base instead of a 64-bit sum in vector registers
+            uint32_t o = off[KC ? q : 0];
+            asm volatile("" : "+v"(o));
+            r[q] = *reinterpret_cast<const UVT_GLOBAL dbl2u*>(at + q * (Idx::KSTEP * 8) * ld + o);
+        }
+        at += KC ? (int64_t)kTileK * 8 : ld * (kTileK * 8);
+    }
+
+    // Any panel: no load sits under a branch per element (such branches cost
+    // a small product most of its time: 257 x 257 17.2 us, now 14.9).  An
+    // operand without a triangle loads a panel inside the range as in the
+    // steady state, so beside the diagonal only the triangle's own panels go
+    // element by element.
+    template <bool TRI, bool GE>
+    __device__ __forceinline__ void load_masked(int tid, int k0, int k_lo, int k_hi, bool tri)
+    {
+        if (!(TRI && tri) && Idx::inside(k0, k_lo, k_hi, nx, ld)) {
+            seek(k0);
+            load(tid);
+            return;
+        }
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) {
+            const int v = tid + q * NT;
+            if (PART && v >= PIECES) break;
+            double e[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int xe = KC ? Idx::px(v) : Idx::px(v) + h, ke = k0 + (KC ? Idx::pk(v) + h : Idx::pk(v));
+                const int x = xe < nx ? xe : nx - 1, k = near_k<GE>(ke, x0 + x, k_hi, TRI && tri);
+                e[h] = KC ? p[(int64_t)x * ld + k] : p[(int64_t)k * ld + x];
+            }
+            r[q] = dbl2{e[0], e[1]};
+        }
+    }
+
+    __device__ __forceinline__ void store(int tid, double* s) const
+    {
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) {
+            const int v = tid + q * NT;
+            if (PART && v >= PIECES) break;
+            *reinterpret_cast<dbl2*>(&s[lds(v)]) = r[q];
+        }
+    }
+
+    // The panel at k0 with zeros outside [k_lo, k_hi) and outside the
+    // triangle, and (UNIT) ones on its diagonal.
+    template <bool TRI, bool GE, bool UNIT>
+    __device__ __forceinline__ void store_masked(int tid, double* s, int k0, int k_lo, int k_hi, bool tri,
+                                                 bool unit) const
+    {
+        if (!(TRI && tri) && k0 >= k_lo && k0 + kTileK <= k_hi) {
+            store(tid, s);
+            return;
+        }
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) {
+            const int v = tid + q * NT;
+            if (PART && v >= PIECES) break;
+            dbl2 w = r[q];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int x = x0 + (KC ? Idx::px(v) : Idx::px(v) + h), k = k0 + (KC ? Idx::pk(v) + h : Idx::pk(v));
+                bool in = k >= k_lo && k < k_hi;
+                if (TRI && tri) in = in && (GE ? k >= x : k <= x);
+                w[h] = in ? w[h] : 0.0;
+                if (UNIT && unit && k == x) w[h] = 1.0;
+            }
+            *reinterpret_cast<dbl2*>(&s[lds(v)]) = w;
+        }
+    }
 };
 
-// VEC: A, B 16-byte aligned and lda, ldb even, so 2-double loads are legal.
+// Which operand of a tile is triangular, and which part of it is kept.
+enum TriKind {
+    kTriALe,  // op(A)[i][k], k <= i (where the tile's flags hold kTileLower)
+    kTriAGe,  // op(A)[i][k], k >= i
+    kTriBLe,  // op(B)[k][j], k <= j
+    kTriBGe   // op(B)[k][j], k >= j
+};
+
+// A_KC / B_KC: k contiguous in memory (A as it is; B transposed).
+// UNIT_: the triangle's diagonal may be taken as ones (f64_tile's unit).
+// EPI_: C = alpha * product + beta * C, else C = product (or C += product).
 // EDGE_IDLE: waves of an edge tile that hold no row or column of C run no
 // products (off where a caller's own registers leave no room for the test:
 // the stream-K kernel then spills inside its masked k loop).
@@ -89,36 +214,79 @@ struct F64Cfg {
 // shapes (the persistent batch kernel: 12 bytes of spills per lane instead
 // of 52, 1.5-3 % faster); the single-shape kernels ran 0.2-1.7 % slower
 // with it.  The sums and their order are the same either way.
-template <int TM, int TN, bool VEC, int WAVES_M = 2, int WAVES_N = 2, int BK_ = 16, bool EDGE_IDLE = true,
-          bool AHEAD2 = false>
-__device__ __forceinline__ void f64_tile(int r0, int rows, int c0, int k_lo, int k_hi, int flags,
-                                         const UVT_GLOBAL double* __restrict__ A, int64_t lda,
+template <bool A_KC_ = true, bool B_KC_ = false, TriKind TRI_ = kTriALe, bool UNIT_ = false, bool EPI_ = false,
+          bool EDGE_IDLE_ = true, bool AHEAD2_ = false>
+struct TileOpt {
+    static constexpr bool A_KC = A_KC_, B_KC = B_KC_, UNIT = UNIT_, EPI = EPI_, EDGE_IDLE = EDGE_IDLE_,
+                          AHEAD2 = AHEAD2_;
+    static constexpr TriKind TRI = TRI_;
+    static constexpr bool TRI_A = TRI == kTriALe || TRI == kTriAGe, GE = TRI == kTriAGe || TRI == kTriBGe;
+};
+
+template <int TM, int TN, int WAVES_M = 2, int WAVES_N = 2, class OPT = TileOpt<>>
+struct F64Cfg {
+    static constexpr int NT = 64 * WAVES_M * WAVES_N;
+    static constexpr int WM = TM / WAVES_M, WN = TN / WAVES_N;
+    static constexpr int FM = WM / 16, FN = WN / 16;
+    using PA = Panel<TM, NT, OPT::A_KC>;
+    using PB = Panel<TN, NT, OPT::B_KC>;
+    static constexpr int SMEM_DOUBLES = 2 * (PA::ELEMS + PB::ELEMS);
+    static_assert(FM >= 1 && FN >= 1, "wave tile below 16x16");
+};
+
+// The part of C a tile covers, its reduction range and what to do with it.
+struct TileArgs {
+    int r0, rows, c0, k_lo, k_hi, flags;
+};
+// C = alpha * product + beta * C (C not read when beta == 0); unit: ones on
+// the triangle's diagonal.
+struct TileEpi {
+    double alpha = 1.0, beta = 0.0;
+    bool unit = false;
+};
+
+// thread: the caller's thread index when it must stay opaque to the compiler
+// (a persistent kernel running several tile shapes, whose per-thread offsets
+// would otherwise be hoisted out of its tile loop for every shape at once
+// and spilled); -1: threadIdx.x.
+// part: if set, the tile's product goes there instead of to C, as a TM x TN
+// row-major block (row r, column c of the tile at r * TN + c; only rows <
+// rows and columns inside C are written), to be added to C later in a fixed
+// order.
+// m: columns of C (and of op(B)).
+template <int TM, int TN, int WAVES_M, int WAVES_N, class OPT = TileOpt<>>
+__device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL double* __restrict__ A, int64_t lda,
                                          const UVT_GLOBAL double* __restrict__ B, int64_t ldb,
-                                         UVT_GLOBAL double* __restrict__ C, int64_t ldc, int64_t m,
-                                         double* smem, int thread = -1,
-                                         UVT_GLOBAL double* __restrict__ part = nullptr)
+                                         UVT_GLOBAL double* __restrict__ C, int64_t ldc, int64_t m, double* smem,
+                                         int thread = -1, UVT_GLOBAL double* __restrict__ part = nullptr,
+                                         const TileEpi& epi = TileEpi())
 {
-    using G = F64Cfg<TM, TN, WAVES_M, WAVES_N, BK_>;
-    constexpr int BK = G::BK, NT = G::NT;
-    // thread: the caller's thread index when it must stay opaque to the
-    // compiler (a persistent kernel running several tile shapes, whose
-    // per-thread offsets would otherwise be hoisted out of its tile loop for
-    // every shape at once and spilled); -1: threadIdx.x.
-    // part: if set, the tile's product goes there instead of to C, as a
-    // TM x TN row-major block (row r, column c of the tile at r * TN + c;
-    // only rows < rows and columns inside C are written), to be added to C
-    // later in a fixed order.
+    using G = F64Cfg<TM, TN, WAVES_M, WAVES_N, OPT>;
+    using PA = typename G::PA;
+    using PB = typename G::PB;
+    constexpr int BK = kTileK;
+    static_assert(!(OPT::AHEAD2 && OPT::GE), "AHEAD2: no diagonal at the tile's start");
+    constexpr bool AHEAD2 = OPT::AHEAD2, GE = OPT::GE, TRI_A = OPT::TRI_A, UNIT = OPT::UNIT;
     const int tid = thread >= 0 ? thread : (int)threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: branches on it stay scalar
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const bool lower = (flags & kTileLower) != 0;
-    double* As = smem;                    // [2][TM][SA]
-    double* Bs = smem + 2 * G::A_ELEMS;   // [2][BK][LDB_S]
+    // kTriALe is the plans' kernel, whose boxes have no triangle; the other
+    // kinds are launched for triangles only.
+    const bool tri = OPT::TRI != kTriALe || (t.flags & kTileLower) != 0;
+    const bool unit = UNIT && epi.unit;
+    double* As = smem;                  // [2][PA::ELEMS]
+    double* Bs = smem + 2 * PA::ELEMS;  // [2][PB::ELEMS]
 
-    const int k_start = k_lo & ~1;  // even, so 2-double loads stay aligned
+    const int k_lo = t.k_lo, k_hi = t.k_hi;
+    const int k_start = k_lo & ~1;
     const int nk = (k_hi > k_start) ? (k_hi - k_start + BK - 1) / BK : 0;
-    const bool cols_full = (int64_t)c0 + TN <= m;
+    const int cols = (int64_t)t.c0 + TN <= m ? TN : (int)(m - t.c0);
+
+    PA pa;
+    PB pb;
+    pa.init(tid, OPT::A_KC ? A + (int64_t)t.r0 * lda : A + t.r0, lda, t.rows, t.r0);
+    pb.init(tid, OPT::B_KC ? B + (int64_t)t.c0 * ldb : B + t.c0, ldb, cols, t.c0);
 
     dbl4 acc[G::FM][G::FN];
 #pragma unroll
@@ -126,180 +294,223 @@ __device__ __forceinline__ void f64_tile(int r0, int rows, int c0, int k_lo, int
 #pragma unroll
         for (int j = 0; j < G::FN; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
 
-    dbl2 ra[G::A_VEC], rb[G::B_VEC];
-
-    // full_tag: std::true_type when the whole k panel lies inside the tile's
-    // k range, below the diagonal and inside C (no masks at all); otherwise
-    // every element is checked.
+    // full_tag: std::true_type for a panel that needs no masks at all (see
+    // the panel ranges below); otherwise every element is checked.
+    int mtid = tid;  // thread index of the masked panels
     auto load = [&](int k0, auto full_tag) {
-        constexpr bool FULL = decltype(full_tag)::value;
-        const bool a_full = FULL;
-        const bool b_full = FULL;
-#pragma unroll
-        for (int q = 0; q < G::A_VEC; ++q) {
-            const int v = tid + q * NT;
-            if (G::A_PART && v >= G::A_PIECES) break;
-            const int row = v / (BK / 2), kp = (v % (BK / 2)) * 2;
-            const int gk = k0 + kp, gr = r0 + row;
-            const UVT_GLOBAL double* p = A + (int64_t)gr * lda + gk;
-            if (a_full) {
-                if (VEC) ra[q] = *reinterpret_cast<const UVT_GLOBAL dbl2*>(p);
-                else ra[q] = dbl2{p[0], p[1]};
-            } else {
-                const bool rv = row < rows;
-                const bool v0 = rv && gk >= k_lo && gk < k_hi && (!lower || gk <= gr);
-                const bool v1 = rv && gk + 1 >= k_lo && gk + 1 < k_hi && (!lower || gk + 1 <= gr);
-                ra[q] = dbl2{v0 ? p[0] : 0.0, v1 ? p[1] : 0.0};
-            }
+        if constexpr (decltype(full_tag)::value) {
+            pa.load(tid);  // panels of the steady state follow each other: see seek()
+            pb.load(tid);
+        } else {
+            pa.template load_masked<TRI_A, GE>(mtid, k0, k_lo, k_hi, tri);
+            pb.template load_masked<!TRI_A, GE>(mtid, k0, k_lo, k_hi, tri);
         }
-#pragma unroll
-        for (int q = 0; q < G::B_VEC; ++q) {
-            const int v = tid + q * NT;
-            if (G::B_PART && v >= G::B_PIECES) break;
-            const int kr = v / (TN / 2), col = (v % (TN / 2)) * 2;
-            const int gk = k0 + kr;
-            const UVT_GLOBAL double* p = B + (int64_t)gk * ldb + (c0 + col);
-            if (b_full) {
-                if (VEC) rb[q] = *reinterpret_cast<const UVT_GLOBAL dbl2*>(p);
-                else rb[q] = dbl2{p[0], p[1]};
-            } else {
-                const bool kv = gk >= k_lo && gk < k_hi;
-                const bool v0 = kv && (int64_t)c0 + col < m;
-                const bool v1 = kv && (int64_t)c0 + col + 1 < m;
-                rb[q] = dbl2{v0 ? p[0] : 0.0, v1 ? p[1] : 0.0};
-            }
+    };
+    auto store = [&](int buf, int k0, auto full_tag) {
+        double* as = As + buf * PA::ELEMS;
+        double* bs = Bs + buf * PB::ELEMS;
+        if constexpr (decltype(full_tag)::value) {
+            pa.store(tid, as);
+            pb.store(tid, bs);
+        } else {
+            pa.template store_masked<TRI_A, GE, UNIT && TRI_A>(mtid, as, k0, k_lo, k_hi, tri, unit);
+            pb.template store_masked<!TRI_A, GE, UNIT && !TRI_A>(mtid, bs, k0, k_lo, k_hi, tri, unit);
         }
     };
 
-    auto store = [&](int buf) {
-        double* as = As + buf * G::A_ELEMS;
-        double* bs = Bs + buf * G::B_ELEMS;
-#pragma unroll
-        for (int q = 0; q < G::A_VEC; ++q) {
-            const int v = tid + q * NT;
-            if (G::A_PART && v >= G::A_PIECES) break;
-            const int row = v / (BK / 2), kp = (v % (BK / 2)) * 2;
-            *reinterpret_cast<dbl2*>(&as[row * G::SA + kp]) = ra[q];
-        }
-#pragma unroll
-        for (int q = 0; q < G::B_VEC; ++q) {
-            const int v = tid + q * NT;
-            if (G::B_PART && v >= G::B_PIECES) break;
-            const int kr = v / (TN / 2), col = (v % (TN / 2)) * 2;
-            *reinterpret_cast<dbl2*>(&bs[kr * G::LDB_S + col]) = rb[q];
-        }
-    };
-
-    // The products of the panel in LDS buffer buf; with st, the registers
-    // loaded for the next panel go to buffer buf ^ 1.  The source places the
-    // writes after the second of the four MFMA steps (measured at N=32768,
-    // M=8192: 69.5-70.4 TFLOP/s against 67.4-69.2 with them after the
-    // first, third or fourth step); the compiler's scheduler then issues them
-    // after the first 4 products of the panel (256x128 tiles) or 8 (128x128),
-    // and moves the barrier that follows ahead of the last step's products.
-    // Pinning the writes with __builtin_amdgcn_sched_barrier after 0, 2, 4,
-    // 8, 16 or 24 products measured 3-12 % slower (4 included: the pins also
-    // stop the other interleaving), as did the max-ilp and iterative-ilp
-    // scheduler strategies (0.8-1.2 %); same bits in every case.
+    // The products of the panel in LDS buffer buf; st() puts the registers
+    // loaded for the next panel into buffer buf ^ 1.
+    //
+    // Software pipeline: the fragments of MFMA step s + 1 are read from LDS
+    // during the products of step s, and those of the next panel's first step
+    // during this panel's last one, behind the panel's one barrier.  (Read at
+    // the head of their own step instead, they left the matrix units idle for
+    // an LDS latency after each barrier, when every wave of a SIMD starts its
+    // panel at once: 16384^2 took 61.7-62.5 ms against 60.4, 4096^2 1016-1027
+    // us against 991, 2048^2 164 against 159, same bits.)  The source places the LDS
+    // writes after the second of the four steps; after the first, the third,
+    // or inside the second or third they measured 0-3 % slower (256x128
+    // tiles).  The order inside a step is the compiler's: pinned with
+    // __builtin_amdgcn_sched_barrier around each step's products, or with
+    // s_setprio around them, the same loop was 4-5 % slower, and
+    // sched_group_barrier (two products, one LDS read) changed nothing.
     //
     // k order inside a panel: at MFMA step s, lane group g = lane / 16 takes
     // k = g * BK/4 + s (A and B alike, so the four steps still cover the
-    // panel's BK values of k once each).  A lane's A values for the whole
-    // panel are then BK/4 consecutive doubles of one row, read as 16-byte
-    // pairs: half the LDS reads of one 8-byte read per step (1.4 % on a
-    // register-only probe of this loop, 73.2 -> 74.3 TFLOP/s).
-    static_assert(BK % 8 == 0, "panel depth: whole 16-byte A pairs per lane group");
-    auto compute = [&](int buf, bool st, auto&& next) {
-        const int kg = (lane >> 4) * (BK / 4);
-        const double* as = As + buf * G::A_ELEMS + (wm * G::WM + (lane & 15)) * G::SA + kg;
-        const double* bs = Bs + buf * G::B_ELEMS + kg * G::LDB_S + wn * G::WN + (lane & 15);
+    // panel's BK values of k once each).  A lane's values of a k-contiguous
+    // operand for the whole panel are then BK/4 consecutive doubles of one
+    // row, read as 16-byte pairs: half the LDS reads of one 8-byte read per
+    // step (1.4 % on a register-only probe of this loop, 73.2 -> 74.3 TFLOP/s).
+    // (Values of a k-contiguous operand come in pairs: steps s and s + 1 for
+    // even s.)
+    dbl2 a2[G::FM], b2[G::FN];
+    double a1[G::FM], b1[G::FN];
+    const int kg = (lane >> 4) * (BK / 4), xa = wm * G::WM + (lane & 15), xb = wn * G::WN + (lane & 15);
+    const int ao = OPT::A_KC ? xa * PA::LD + kg : kg * PA::LD + xa;
+    const int bo = OPT::B_KC ? xb * PB::LD + kg : kg * PB::LD + xb;
+    auto read = [&](int buf, int s, auto& ra2, auto& rb2, auto& ra1, auto& rb1) {
+        const double* as = As + buf * PA::ELEMS + ao;
+        const double* bs = Bs + buf * PB::ELEMS + bo;
 #pragma unroll
-        for (int sp = 0; sp < BK / 8; ++sp) {
-            dbl2 a2[G::FM];
+        for (int i = 0; i < G::FM; ++i) {
+            if constexpr (OPT::A_KC) {
+                if (s % 2 == 0) ra2[i] = *reinterpret_cast<const dbl2*>(&as[i * 16 * PA::LD + s]);
+            } else {
+                ra1[i] = as[s * PA::LD + i * 16];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < G::FN; ++j) {
+            if constexpr (OPT::B_KC) {
+                if (s % 2 == 0) rb2[j] = *reinterpret_cast<const dbl2*>(&bs[j * 16 * PB::LD + s]);
+            } else {
+                rb1[j] = bs[s * PB::LD + j * 16];
+            }
+        }
+    };
+    auto read0 = [&](int buf) { read(buf, 0, a2, b2, a1, b1); };
+    auto compute = [&](int buf, auto&& st) {
+#pragma unroll
+        for (int s = 0; s < BK / 4; ++s) {
+            dbl2 na2[G::FM], nb2[G::FN];
+            double na1[G::FM], nb1[G::FN];
+            if (s + 1 < BK / 4) {
+                read(buf, s + 1, na2, nb2, na1, nb1);
+            } else {
+                __syncthreads();
+                read(buf ^ 1, 0, na2, nb2, na1, nb1);
+            }
 #pragma unroll
             for (int i = 0; i < G::FM; ++i)
-                a2[i] = *reinterpret_cast<const dbl2*>(&as[i * 16 * G::SA + 2 * sp]);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int s = 2 * sp + h;
-                double b[G::FN];
+                for (int j = 0; j < G::FN; ++j) {
+                    const double a = OPT::A_KC ? a2[i][s % 2] : a1[i];
+                    const double b = OPT::B_KC ? b2[j][s % 2] : b1[j];
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[i][j], 0, 0, 0);
+                }
+            if (s == 1) st();
 #pragma unroll
-                for (int j = 0; j < G::FN; ++j) b[j] = bs[s * G::LDB_S + j * 16];
+            for (int i = 0; i < G::FM; ++i) {
+                if constexpr (OPT::A_KC) {
+                    if (s % 2 == 1) a2[i] = na2[i];
+                } else {
+                    a1[i] = na1[i];
+                }
+            }
 #pragma unroll
-                for (int i = 0; i < G::FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < G::FN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2[i][h], b[j], acc[i][j], 0, 0, 0);
-                if (s == 1 && st) {
-                    store(buf ^ 1);
-                    next();  // AHEAD2: the loads of the panel after next
+            for (int j = 0; j < G::FN; ++j) {
+                if constexpr (OPT::B_KC) {
+                    if (s % 2 == 1) b2[j] = nb2[j];
+                } else {
+                    b1[j] = nb1[j];
                 }
             }
         }
     };
 
-    // Panels kt in [kt0, nfull) need no masks: k0 >= k_lo (only panel 0 can
-    // start below an odd k_lo), k0 + BK <= k_hi, left of the diagonal for a
-    // lower tile, and the tile inside C.  They form the steady-state loop,
-    // free of per-panel branches; the rest (next to the diagonal, at the
-    // tile's k end) run masked.
+    // Panels [f0, f1) need no masks: the steady-state loop, free of per-panel
+    // branches.  The rest (next to the diagonal, at the tile's k ends) run
+    // masked.
     if (nk > 0) {
         const std::true_type full{};
         const std::false_type masked{};
-        const int lim = lower ? (k_hi < r0 + 1 ? k_hi : r0 + 1) : k_hi;
-        const int kt0 = k_start < k_lo ? 1 : 0;
-        const int nfull = (rows == TM && cols_full && lim >= k_start) ? (lim - k_start) / BK : 0;
-        if (kt0 == 0 && nfull > 0) load(k_start, full);
-        else load(k_start, masked);
-        store(0);
+        const bool odd = (!OPT::A_KC && (t.rows & 1)) || (!OPT::B_KC && (cols & 1));
+        // first and last coordinate of the triangular operand
+        const int tx0 = TRI_A ? t.r0 : t.c0, tx1 = tx0 + (TRI_A ? t.rows : cols) - 1;
+        const FullPanels fp = full_panels<GE>(k_start, k_lo, k_hi, tri, unit, tx0, tx1, odd);
+        const int f0 = fp.f0, f1 = PA::Idx::offsets_fit(lda) && PB::Idx::offsets_fit(ldb) ? fp.f1 : 0;
+        pa.seek(k_start + f0 * BK);
+        pb.seek(k_start + f0 * BK);
+
+        const bool first_full = f0 == 0 && f1 > 0;
+        if (first_full) {
+            load(k_start, full);
+            store(0, k_start, full);
+        } else {
+            load(k_start, masked);
+            store(0, k_start, masked);
+        }
         if (AHEAD2 && nk > 1) {
-            if (1 < nfull) load(k_start + BK, full);  // panel 1 is full from kt0 <= 1 on
+            if (f0 <= 1 && 1 < f1) load(k_start + BK, full);
             else load(k_start + BK, masked);
         }
         __syncthreads();
+        // A panel whose k lies on the zero side of the triangle for all of a
+        // wave's rows (columns) holds only zeros for it: the wave runs it
+        // without products (it only stores the next panel), which leaves the
+        // CU's matrix units to the other waves.  Panel counts are uniform over
+        // the wave.  Skipping adds of exact zeros changes no result (the sign
+        // of a zero aside).  Likewise a wave whose rows all lie past the
+        // tile's last row, or whose columns all lie past C's last column,
+        // writes nothing: outside the steady-state loop it runs no products.
+        const bool idle = OPT::EDGE_IDLE && (wm * G::WM >= t.rows || wn * G::WN >= cols);
         int kt = 0;
+        if constexpr (!GE) read0(0);
+        if constexpr (GE) {  // the diagonal comes first
+            const int wx0 = tx0 + (TRI_A ? wm * G::WM : wn * G::WN);  // this wave's first row (column)
+            const int kw = idle ? f0 : (wx0 - k_start) / BK;           // its first panel that is not all zeros
+            for (; kt + 1 < f0 && kt + 1 < nk; ++kt) {
+                load(k_start + (kt + 1) * BK, masked);
+                if (kt >= kw) {
+                    if (kt == max(kw, 0)) read0(kt & 1);
+                    compute(kt & 1, [&] { store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked); });
+                } else {
+                    store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
+                    __syncthreads();
+                }
+            }
+            if (kt <= max(kw, 0)) read0(kt & 1);
+        }
         // Registers hold the next panel's values from here on when AHEAD2.
         if constexpr (AHEAD2) {
-            for (; kt + 2 < nfull; ++kt) {  // the panel after next is full
-                compute(kt & 1, true, [&] { load(k_start + (kt + 2) * BK, full); });
+            if (idle) {  // this wave only feeds the others
+                for (; kt + 2 < f1; ++kt) {
+                    store((kt & 1) ^ 1, 0, full);
+                    load(k_start + (kt + 2) * BK, full);
+                    __syncthreads();
+                }
+            }
+            for (; kt + 2 < f1; ++kt) {  // the panel after next is full
+                compute(kt & 1, [&] {
+                    store((kt & 1) ^ 1, 0, full);
+                    load(k_start + (kt + 2) * BK, full);
+                });
+            }
+        } else if (idle) {  // this wave only feeds the others
+            for (; kt + 1 < f1; ++kt) {
+                load(k_start + (kt + 1) * BK, full);
+                store((kt & 1) ^ 1, 0, full);
                 __syncthreads();
             }
         } else {
-            for (; kt + 1 < nfull; ++kt) {  // the next panel is full
+            for (; kt + 1 < f1; ++kt) {  // the next panel is full
                 load(k_start + (kt + 1) * BK, full);
-                compute(kt & 1, true, [] {});
-                __syncthreads();
+                compute(kt & 1, [&] { store((kt & 1) ^ 1, 0, full); });
             }
         }
-        // In a lower tile, panels that start past the last of this wave's
-        // rows meet only masked (zero) A values: the wave runs them without
-        // products (the second loop: it only stores the next panel), which
-        // leaves the CU's matrix units to the other waves.  The panel count
-        // is uniform over the wave.  Skipping adds of exact zeros changes no
-        // result (the sign of a zero aside).
-        // Likewise a wave whose rows all lie past the tile's last row, or
-        // whose columns all lie past C's last column (a tile at the bottom or
-        // right edge, which never takes the steady-state loop), multiplies
-        // only zeros and writes nothing: it runs no products.
-        const bool idle = EDGE_IDLE && (wm * G::WM >= rows || (int64_t)c0 + wn * G::WN >= m);
+        // The masked panels' offsets are computed from here on, not held in
+        // registers (or spilled) since the tile's first panel.
+        asm volatile("" : "+v"(mtid));
         int nk_w = nk;
-        if (lower) {
-            const int last = idle ? -1 : r0 + wm * G::WM + G::WM - 1;  // last row of this wave
+        if (idle) nk_w = kt;
+        else if (tri && !GE) {
+            // last row (column) of this wave, inside C
+            const int last = tx0 + (TRI_A ? wm * G::WM + G::WM : wn * G::WN + G::WN) - 1;
             nk_w = last >= k_start ? (last - k_start) / BK + 1 : 0;
             nk_w = nk_w < kt ? kt : (nk_w > nk ? nk : nk_w);
         }
         for (; kt < nk_w; ++kt) {
             const bool more = kt + 1 < nk;
             if (!AHEAD2 && more) load(k_start + (kt + 1) * BK, masked);
-            compute(kt & 1, more, [&] {
+            compute(kt & 1, [&] {
+                if (more) store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
                 if (AHEAD2 && kt + 2 < nk) load(k_start + (kt + 2) * BK, masked);
             });
-            __syncthreads();
         }
         for (; kt < nk; ++kt) {
             if (kt + 1 < nk) {
                 if (!AHEAD2) load(k_start + (kt + 1) * BK, masked);
-                store((kt & 1) ^ 1);
+                store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
                 if (AHEAD2 && kt + 2 < nk) load(k_start + (kt + 2) * BK, masked);
             }
             __syncthreads();
@@ -308,23 +519,28 @@ __device__ __forceinline__ void f64_tile(int r0, int rows, int c0, int k_lo, int
 
     // D layout of v_mfma_f64_16x16x4_f64 (measured on gfx950): lane l,
     // element v holds row l/16 + 4*v, column l%16 of the 16x16 block.
-    const bool accum = (flags & kTileAccum) != 0;
+    const bool accum = (t.flags & kTileAccum) != 0;
 #pragma unroll
     for (int i = 0; i < G::FM; ++i) {
 #pragma unroll
         for (int j = 0; j < G::FN; ++j) {
             const int col = wn * G::WN + j * 16 + (lane & 15);
-            const bool cv = (int64_t)c0 + col < m;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int row = wm * G::WM + i * 16 + (lane >> 4) + 4 * v;
-                if (cv && row < rows) {
+                if (col < cols && row < t.rows) {
+                    const double x = acc[i][j][v];
                     if (part) {
-                        part[row * TN + col] = acc[i][j][v];
+                        part[row * TN + col] = x;
                     } else {
-                        UVT_GLOBAL double* p = C + (int64_t)(r0 + row) * ldc + (c0 + col);
-                        if (accum) *p += acc[i][j][v];
-                        else *p = acc[i][j][v];
+                        UVT_GLOBAL double* p = C + (int64_t)(t.r0 + row) * ldc + (t.c0 + col);
+                        if constexpr (OPT::EPI) {
+                            const double ax = epi.alpha * x;
+                            *p = epi.beta == 0.0 ? ax : ax + epi.beta * *p;
+                        } else {
+                            if (accum) *p += x;
+                            else *p = x;
+                        }
                     }
                 }
             }

@@ -1,0 +1,94 @@
+// uvt_panel.hpp -- which elements of an operand an FP64 tile reads (host and
+// device; the loads themselves are in uvt_f64_tile.hpp).
+//
+// A tile multiplies X rows of op(A) and X columns of op(B) over k in
+// [k_lo, k_hi), kTileK deep panels from k_start = k_lo rounded down to even.
+// An operand is k-contiguous in memory (KC: A, or B transposed; element
+// (x, k) at x * ld + k) or x-contiguous (B, or A transposed; k * ld + x).
+// Panels move as pairs along the contiguous direction.
+//
+//   full panels    pairs as they are, every row (column) past the tile's last
+//                  one replaced by the last: no masks.  An odd last x of an
+//                  x-contiguous operand reads its pair one element past the
+//                  row's end, so such a panel never holds the matrix's last k
+//                  row, and that element lies before the next row.
+//   other panels   element by element, each at the nearest place inside the
+//                  matrix, the k range and the triangle; what does not belong
+//                  is zeroed on the way to LDS.
+#pragma once
+
+#include <stdint.h>
+
+namespace uvt {
+
+constexpr int kTileK = 16;  // k depth of one LDS panel (4 MFMA steps)
+
+template <int X, int NT, bool KC>
+struct PanelIdx {
+    static constexpr int PIECES = X * kTileK / 2;         // pairs of a panel
+    static constexpr int VEC = (PIECES + NT - 1) / NT;    // per thread
+    static constexpr bool PART = PIECES < NT;             // the last threads hold none
+    static_assert(PIECES % NT == 0 || PART, "uneven panel split");
+    // Pieces of an x-contiguous panel that one thread holds sit KSTEP k rows
+    // apart at the same x.
+    static constexpr int KSTEP = KC ? 0 : NT / (X / 2);
+    static_assert(KC || NT % (X / 2) == 0, "k rows per piece");
+
+    // x and k of pair v (of its first element), relative to the panel.
+    static __host__ __device__ int px(int v) { return KC ? v / (kTileK / 2) : (v % (X / 2)) * 2; }
+    static __host__ __device__ int pk(int v) { return KC ? (v % (kTileK / 2)) * 2 : v / (X / 2); }
+    // The x a full panel reads pair v at, with nx of the X inside the matrix.
+    static __host__ __device__ int full_x(int v, int nx)
+    {
+        const int last = KC ? nx - 1 : (nx - 1) & ~1;
+        return px(v) < last ? px(v) : last;
+    }
+    // Byte offsets of full panels fit 32 bits for every matrix but one whose
+    // rows are 16 MB or longer; such a tile has no full panels.
+    static __host__ __device__ bool offsets_fit(int64_t ld)
+    {
+        return ld <= (int64_t)(0xFFFFFFFFu / (8u * (KC ? X : kTileK))) - 1;
+    }
+    // Whether the panel at k0 lies wholly inside [k_lo, k_hi) and may be read
+    // as a full one.
+    static __host__ __device__ bool inside(int k0, int k_lo, int k_hi, int nx, int64_t ld)
+    {
+        return k0 >= k_lo && k0 + kTileK <= k_hi - (!KC && (nx & 1) ? 1 : 0) && offsets_fit(ld);
+    }
+};
+
+// The k another panel reads element (x, k) at, x inside the matrix: the
+// nearest below k_hi and, with tri, in the triangle (GE: k >= x, else k <= x).
+template <bool GE>
+__host__ __device__ inline int near_k(int k, int x, int k_hi, bool tri)
+{
+    k = k < k_hi ? k : k_hi - 1;
+    if (tri) k = GE ? (k > x ? k : x) : (k < x ? k : x);
+    return k;
+}
+
+// Panels [f0, f1) of a tile need no masks: inside [k_lo, k_hi) (only panel 0
+// can start below an odd k_lo), off the diagonal of the triangle whose x run
+// from tx0 to tx1 (unit: the diagonal itself is replaced too), and away from
+// the last k row where odd asks for it.
+struct FullPanels {
+    int f0, f1;
+};
+template <bool GE>
+__host__ __device__ inline FullPanels full_panels(int k_start, int k_lo, int k_hi, bool tri, bool unit, int tx0,
+                                                  int tx1, bool odd)
+{
+    int lim = k_hi, f0 = k_start < k_lo ? 1 : 0;
+    if (tri && !GE) {
+        const int d = tx0 + (unit ? 0 : 1);
+        lim = lim < d ? lim : d;
+    }
+    if (tri && GE) {
+        const int d = tx1 + (unit ? 1 : 0) - k_start, f = d > 0 ? (d + kTileK - 1) / kTileK : 0;
+        f0 = f0 > f ? f0 : f;
+    }
+    lim -= odd ? 1 : 0;
+    return FullPanels{f0, lim > k_start ? (lim - k_start) / kTileK : 0};
+}
+
+}  // namespace uvt

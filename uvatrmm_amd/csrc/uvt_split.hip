@@ -735,12 +735,8 @@ __global__ __launch_bounds__(512, 4) void k_diag_f64(Desc one, const Desc* table
     const UVT_GLOBAL double* A = gbl(UVT_FIELD(A));
     const UVT_GLOBAL double* B = gbl(UVT_FIELD(B));
     UVT_GLOBAL double* C = gbl(UVT_FIELD(C));
-    if (UVT_FIELD(vec))
-        f64_tile<128, 128, true, 4, 2>(r0, rows, c0, k_lo, r0 + rows, kTileLower, A, UVT_FIELD(lda),
-                                       B, UVT_FIELD(ldb), C, UVT_FIELD(ldc), UVT_FIELD(m), smem);
-    else
-        f64_tile<128, 128, false, 4, 2>(r0, rows, c0, k_lo, r0 + rows, kTileLower, A, UVT_FIELD(lda),
-                                        B, UVT_FIELD(ldb), C, UVT_FIELD(ldc), UVT_FIELD(m), smem);
+    f64_tile<128, 128, 4, 2>(TileArgs{r0, rows, c0, k_lo, r0 + rows, kTileLower}, A, UVT_FIELD(lda), B,
+                             UVT_FIELD(ldb), C, UVT_FIELD(ldc), UVT_FIELD(m), smem);
 #undef UVT_FIELD
 }
 
