@@ -194,9 +194,7 @@ typedef enum { UVT_NON_UNIT = 0, UVT_UNIT = 1 } uvt_diag;
 /* C = alpha op(A) op(B) + beta C; C (m x n) is not read when beta == 0, A and
  * B are not read when k == 0 or alpha == 0.  Replaces the cblas_dgemm call of
  * UVaTRMM/src/mm_triangular.c:347-360 (RowMajor, NoTrans, NoTrans, alpha 1,
- * beta 0) and covers the other transposes.  Uses the handle's workspace:
- * calls on one handle that use it (uvt_dgemm, uvt_dtrmm, uvt_inf_norm) must
- * be on one stream or serialized by the caller. */
+ * beta 0) and covers the other transposes.  Uses no workspace. */
 uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_t n, int64_t k,
                      double alpha, const double *dA, int64_t lda, const double *dB, int64_t ldb,
                      double beta, double *dC, int64_t ldc, void *stream);
@@ -205,7 +203,8 @@ uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_
  * diagonal is taken as 1).  Replaces the cblas_dtrmm call of
  * mm_triangular.c:374-387 (RowMajor, Left, Lower, NoTrans, NonUnit, alpha 1)
  * and covers every other side / uplo / trans / diag.  Uses the handle's
- * workspace (see uvt_dgemm). */
+ * workspace for a copy of B: calls on one handle that use it (uvt_dtrmm,
+ * uvt_inf_norm) must be on one stream or serialized by the caller. */
 uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans ta, uvt_diag diag,
                      int64_t m, int64_t n, double alpha, const double *dA, int64_t lda,
                      double *dB, int64_t ldb, void *stream);
@@ -216,9 +215,11 @@ uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans ta, u
  * results (bit for bit) and errors as uvt_dtrmm, but its workspace is a fixed
  * per-device scratch array of UVT_NOALLOC_SCRATCH_MB MiB inside the library
  * (held by every device the library runs on until the process ends) instead
- * of the handle's workspace: calls needing more (for a left-side lower,
- * non-transposed, non-unit A: 8 * m * (n rounded up to even) bytes; other
- * forms also pack A and/or B) return UVT_ERR_SIZE.  Every call on a device
+ * of the handle's workspace: calls over its limit return UVT_ERR_SIZE.  The
+ * limit counts 8 * m * (n rounded up to even) bytes for a left-side lower,
+ * non-transposed, non-unit A; for other forms that once or twice, and the
+ * square of A's order (the other dimension rounded up to even) where the
+ * triangle is not plain lower.  Every call on a device
  * shares that device's array, so calls that overlap on one device (other
  * streams, other handles, other threads) race: serialize them.  Nothing in
  * the array needs to start at zero. */

@@ -5,7 +5,8 @@
 //     end, before the next row), inside [k_lo, k_hi) and, for the rows
 //     (columns) the tile holds, strictly inside the triangle (unit: off its
 //     diagonal); every pair of the panel is read once, in its own place;
-//   - the full panels are one run [f0, f1) of the tile's panels, and every
+//   - the full panels are one run [f0, f1) of the tile's panels, in the order
+//     it runs them (f0 is 0 or 1, the diagonal comes last), and every
 //     panel that could be one is, up to one beside the matrix's last k row;
 //   - the other panels read each element at a place inside the matrix, the k
 //     range's end and the triangle, and at its own place wherever that is one.
@@ -36,13 +37,13 @@ static void operand(int x0, int nx, int k_lo, int k_hi, int kmax, bool tri, bool
 {
     using I = PanelIdx<X, NT, KC>;
     const int64_t ld = KC ? kmax : x0 + nx;  // the tightest the matrix can be stored
-    const int k_start = k_lo & ~1, nk = k_hi > k_start ? (k_hi - k_start + kTileK - 1) / kTileK : 0;
+    const int nk = panels(k_lo, k_hi);
     const bool odd = !KC && (nx & 1);
-    const FullPanels fp = full_panels<GE>(k_start, k_lo, k_hi, tri, unit, x0, x0 + nx - 1, odd);
+    const FullPanels fp = full_panels<GE>(k_lo, k_hi, tri, unit, x0, x0 + nx - 1, odd);
     CHECK(I::offsets_fit(ld), "%d", (int)ld);
-    CHECK(fp.f1 <= nk, "%d %d", fp.f1, nk);
+    CHECK(fp.f1 <= nk && (fp.f0 == 0 || fp.f0 == 1), "%d %d of %d", fp.f0, fp.f1, nk);
     for (int p = 0; p < nk; ++p) {
-        const int k0 = k_start + p * kTileK;
+        const int k0 = panel_k0<GE>(k_lo, nk, p);
         const bool full = p >= fp.f0 && p < fp.f1;
         bool could = k0 >= k_lo && k0 + kTileK <= k_hi - odd;
         if (tri && !GE) could = could && k0 + kTileK - 1 < x0 + (unit ? 0 : 1) - odd;

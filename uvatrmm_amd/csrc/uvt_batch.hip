@@ -69,7 +69,7 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, int ntiles, const BatchPro
                  int* __restrict__ counter)
 {
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES];
-    using Opt = TileOpt<true, false, kTriALe, false, false, true, true>;
+    using Opt = TileOpt<true, false, kTriALe, false, false, true, true, false>;
     static_assert(F64Cfg<64, 64, 2, 4>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 64, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 32, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES,

@@ -4,17 +4,18 @@
 // variant.  All of them run on the FP64 MFMA tile kernel of uvt_f64_tile.hpp:
 //
 //   dgemm  C = alpha op(A) op(B) + beta C
-//          op(A), op(B) packed row-major when transposed (LDS-tiled transpose),
-//          then the rectangular tile walk (no triangle mask), then the alpha /
-//          beta epilogue (C is not read when beta == 0).
+//          the rectangular tile walk; the tile reads either operand as it is
+//          stored or transposed, and applies alpha and beta as it writes C
+//          (C is not read when beta == 0).  No workspace.
 //   dtrmm  B := alpha op(A) B  (left)  or  alpha B op(A)  (right), in place
-//          reduced to  R = tril(L) X  with
-//            right side:   X = B^T, and op(A) -> op(A)^T
-//            upper T:      P T P is lower for the row/column reversal P, so
-//                          T X = P (P T P) (P X): rows of X and of the result
-//                          are reversed on packing / unpacking
-//          L packed with its strict upper part zeroed and a unit diagonal
-//          written in when asked; the result unpacked into B with alpha.
+//          B is copied to the workspace, then the tile walk multiplies the
+//          copy into B: the triangle masks either operand, lower or upper, a
+//          transposed A is read as it is stored, and a unit diagonal goes in
+//          on the way to LDS.
+// (With op(A), op(B) and the triangle packed row-major and lower first, and
+// the result unpacked afterwards, a dtrmm of a 2048 triangle on 3000 rows
+// took 323 us, of which three packing passes were 57; now 241.  A 1500 x 2000
+// x 3000 dgemm with A transposed and beta: 334 us, now 293.)
 // Layout-only reductions (column-major input) are the caller's (the CBLAS
 // shim): a column-major matrix is the transpose of a row-major one.
 #include <hip/hip_runtime.h>
@@ -31,128 +32,102 @@ using namespace uvt;
 
 namespace {
 
-constexpr int PT = 64;  // pack tile edge
-
-// dst[i][j] = alpha * S(rmap(i), cmap(j)) for i < rows, j < cols, where
-// S(a, b) = src[a*lds + b] (trans = 0) or src[b*lds + a] (trans = 1),
-// rmap(i) = rev_r ? rows-1-i : i, cmap(j) = rev_c ? cols-1-j : j.
-// tri: only the lower triangle (j <= i) is read; above it dst = 0, and with
-// unit the diagonal is 1.  The transposed read goes through an LDS tile so
-// both the global reads and the writes are row-contiguous.
-__global__ __launch_bounds__(256) void k_pack(const double* __restrict__ src, int64_t lds,
-                                              double* __restrict__ dst, int64_t ldd, int64_t rows,
-                                              int64_t cols, int trans, int rev_r, int rev_c,
-                                              double alpha, int tri, int unit)
-{
-    __shared__ double tile[PT][PT + 1];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int64_t bi = blockIdx.y; bi * PT < rows; bi += gridDim.y) {
-        const int64_t i0 = bi * PT, j0 = (int64_t)blockIdx.x * PT;
-        if (tri && j0 > i0 + PT - 1) {  // strictly above the diagonal: zeros
-            for (int r = ty; r < PT; r += 4) {
-                const int64_t i = i0 + r, j = j0 + tx;
-                if (i < rows && j < cols) dst[i * ldd + j] = 0.0;
-            }
-            continue;
-        }
-        if (!trans) {
-            for (int r = ty; r < PT; r += 4) {
-                const int64_t i = i0 + r, j = j0 + tx;
-                if (i >= rows || j >= cols) continue;
-                double v;
-                if (tri && j > i) v = 0.0;
-                else if (unit && i == j) v = 1.0;
-                else {
-                    const int64_t a = rev_r ? rows - 1 - i : i, b = rev_c ? cols - 1 - j : j;
-                    v = alpha * src[a * lds + b];
-                }
-                dst[i * ldd + j] = v;
-            }
-        } else {
-            // read S(rmap(i), cmap(j)) = src[cmap(j)*lds + rmap(i)]: for a fixed
-            // j the reads over i are contiguous (reversed when rev_r)
-            for (int c = ty; c < PT; c += 4) {
-                const int64_t j = j0 + c, i = i0 + tx;
-                double v = 0.0;
-                if (i < rows && j < cols && !(tri && j > i)) {
-                    const int64_t a = rev_r ? rows - 1 - i : i, b = rev_c ? cols - 1 - j : j;
-                    v = src[b * lds + a];
-                }
-                tile[c][tx] = v;
-            }
-            __syncthreads();
-            for (int r = ty; r < PT; r += 4) {
-                const int64_t i = i0 + r, j = j0 + tx;
-                if (i >= rows || j >= cols) continue;
-                double v;
-                if (tri && j > i) v = 0.0;
-                else if (unit && i == j) v = 1.0;
-                else v = alpha * tile[tx][r];
-                dst[i * ldd + j] = v;
-            }
-            __syncthreads();
-        }
-    }
-}
-
-// C = alpha * P + beta * C (P == nullptr: alpha * 0).  beta == 0: C is not read.
-__global__ __launch_bounds__(256) void k_axpby(int64_t rows, int64_t cols, double alpha,
-                                               const double* __restrict__ P, int64_t ldp,
-                                               double beta, double* __restrict__ C, int64_t ldc)
+// C = beta * C (beta == 0: zeros, C is not read).
+__global__ __launch_bounds__(256) void k_scale(int64_t rows, int64_t cols, double beta, double* __restrict__ C,
+                                               int64_t ldc)
 {
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (j >= cols) return;
     for (int64_t i = blockIdx.y; i < rows; i += gridDim.y) {
-        const double p = P ? alpha * P[i * ldp + j] : 0.0;
         double* c = C + i * ldc + j;
-        *c = beta == 0.0 ? p : p + beta * *c;
+        *c = beta == 0.0 ? 0.0 : beta * *c;
     }
 }
 
-// Rectangle C[0:M, 0:N] = A[0:M, 0:K] * B[0:K, 0:N] on the FP64 tile.
-template <int TM, int TN>
-__global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
-                             (TileWaves<TM, TN>::WAVES_PER_EU))
-void k_gemm_f64(int64_t M, int64_t N, int K, int nct, const double* __restrict__ A, int64_t lda,
-                const double* __restrict__ B, int64_t ldb, double* __restrict__ C, int64_t ldc)
+// dst[i][j] = src[i][j], rows x cols.  HBM-bound: 16 bytes per element moved.
+__global__ __launch_bounds__(256) void k_copy(const double* __restrict__ src, int64_t lds, double* __restrict__ dst,
+                                              int64_t ldd, int64_t rows, int64_t cols)
 {
-    using W = TileWaves<TM, TN>;
-    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N>::SMEM_DOUBLES];
-    const int rt = (int)(blockIdx.x / nct), ct = (int)(blockIdx.x % nct);
-    const int r0 = rt * TM;
-    const int rows = (int)(M - r0 < TM ? M - r0 : TM);
-    f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, ct * TN, 0, K, 0}, gbl(A), lda, gbl(B), ldb, gbl(C), ldc, N,
-                                 smem);
+    const int64_t j = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    if (j >= cols) return;
+    for (int64_t i0 = (int64_t)blockIdx.y * 16 + (threadIdx.x >> 6); i0 < rows; i0 += (int64_t)gridDim.y * 16) {
+        double v[4];  // four rows in flight
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = i0 + 4 * q < rows ? src[(i0 + 4 * q) * lds + j] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + 4 * q < rows) dst[(i0 + 4 * q) * ldd + j] = v[q];
+    }
 }
 
-template <int TM, int TN>
-void launch_gemm(int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, const double* B, int64_t ldb,
-                 double* C, int64_t ldc, hipStream_t s)
+// What a walk multiplies: C (M x N) from a reduction over K, and which
+// operand is triangular (TriKind; kTriNone: neither).
+struct Walk {
+    int64_t M, N;
+    int K, nrt, nct;
+};
+constexpr int kTriNone = -1;
+
+// One tile per workgroup, the deepest reductions first (left side: row tiles
+// of the long end of the triangle; right side: column tiles).
+template <int TM, int TN, bool A_KC, bool B_KC, int TRI>
+__global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N), (TileWaves<TM, TN>::WAVES_PER_EU))
+void k_blas_f64(Walk g, const double* __restrict__ A, int64_t lda, const double* __restrict__ B, int64_t ldb,
+                double* __restrict__ C, int64_t ldc, TileEpi epi)
 {
-    const int nrt = (int)((M + TM - 1) / TM), nct = (int)((N + TN - 1) / TN);
-    const dim3 grid((unsigned)((int64_t)nrt * nct));
-    const dim3 block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    hipLaunchKernelGGL((k_gemm_f64<TM, TN>), grid, block, 0, s, M, N, (int)K, nct, A, lda, B, ldb, C, ldc);
+    using W = TileWaves<TM, TN>;
+    constexpr bool kNone = TRI == kTriNone, kRight = TRI == kTriBLe || TRI == kTriBGe;
+    using Opt = TileOpt<A_KC, B_KC, kNone ? kTriALe : (TriKind)TRI, !kNone, true, true, false, false>;
+    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
+    const int b = (int)blockIdx.x;
+    int rt = kRight ? b % g.nrt : b / g.nct, ct = kRight ? b / g.nrt : b % g.nct;
+    if (TRI == kTriALe) rt = g.nrt - 1 - rt;
+    if (TRI == kTriBLe) ct = g.nct - 1 - ct;
+    const int r0 = rt * TM, c0 = ct * TN;
+    const int rows = (int)(g.M - r0 < TM ? g.M - r0 : TM), cols = (int)(g.N - c0 < TN ? g.N - c0 : TN);
+    const int k_lo = TRI == kTriAGe ? r0 : TRI == kTriBGe ? c0 : 0;
+    const int k_hi = TRI == kTriALe ? r0 + rows : TRI == kTriBLe ? c0 + cols : g.K;
+    f64_tile<TM, TN, W::M, W::N, Opt>(TileArgs{r0, rows, c0, k_lo, k_hi, kNone ? 0 : kTileLower}, gbl(A), lda, gbl(B),
+                                      ldb, gbl(C), ldc, g.N, smem, -1, nullptr, epi);
+}
+
+template <int TM, int TN, bool A_KC, bool B_KC, int TRI>
+void launch_walk(Walk g, const double* A, int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc,
+                 const TileEpi& epi, hipStream_t s)
+{
+    g.nrt = (int)((g.M + TM - 1) / TM);
+    g.nct = (int)((g.N + TN - 1) / TN);
+    const dim3 grid((unsigned)((int64_t)g.nrt * g.nct)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
+    hipLaunchKernelGGL((k_blas_f64<TM, TN, A_KC, B_KC, TRI>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc, epi);
+}
+
+// The tile shape for the walk: cfg as uvt_default_cfg / uvt_wide_tiles name
+// it; on the right side 32 x 128 stands for 128 x 32 (B has few rows).
+template <bool A_KC, bool B_KC, int TRI>
+uvt_status launch_blas(int32_t cfg, const Walk& g, const double* A, int64_t lda, const double* B, int64_t ldb,
+                       double* C, int64_t ldc, const TileEpi& epi, hipStream_t s)
+{
+    constexpr bool kRight = TRI == kTriBLe || TRI == kTriBGe;
+    const int64_t tm = kRight && cfg == UVT_CFG_128x32 ? 32 : uvt_cfg_tile_m(cfg);
+    const int64_t tn = kRight && cfg == UVT_CFG_128x32 ? 128 : uvt_cfg_tile_n(cfg);
+    if (((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
+    if (cfg == UVT_CFG_64x64) launch_walk<64, 64, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    else if (cfg == UVT_CFG_128x32)
+        launch_walk<kRight ? 32 : 128, kRight ? 128 : 32, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    else if (cfg == UVT_CFG_256x128) launch_walk<256, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    else launch_walk<128, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    UVT_HIP(hipGetLastError());
+    return UVT_OK;
+}
+
+void scale(int64_t rows, int64_t cols, double beta, double* C, int64_t ldc, hipStream_t s)
+{
+    const dim3 grid((unsigned)((cols + 255) / 256), (unsigned)std::min<int64_t>(rows, 32768));
+    hipLaunchKernelGGL(k_scale, grid, dim3(256), 0, s, rows, cols, beta, C, ldc);
 }
 
 int64_t even(int64_t x) { return x + (x & 1); }
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-void pack(const double* src, int64_t lds, double* dst, int64_t ldd, int64_t rows, int64_t cols,
-          bool trans, bool rev_r, bool rev_c, double alpha, bool tri, bool unit, hipStream_t s)
-{
-    const int64_t gy = std::min<int64_t>((rows + PT - 1) / PT, 32768);
-    const dim3 grid((unsigned)((cols + PT - 1) / PT), (unsigned)gy);
-    hipLaunchKernelGGL(k_pack, grid, dim3(256), 0, s, src, lds, dst, ldd, rows, cols, (int)trans,
-                       (int)rev_r, (int)rev_c, alpha, (int)tri, (int)unit);
-}
-
-void axpby(int64_t rows, int64_t cols, double alpha, const double* P, int64_t ldp, double beta,
-           double* C, int64_t ldc, hipStream_t s)
-{
-    const dim3 grid((unsigned)((cols + 255) / 256), (unsigned)std::min<int64_t>(rows, 32768));
-    hipLaunchKernelGGL(k_axpby, grid, dim3(256), 0, s, rows, cols, alpha, P, ldp, beta, C, ldc);
-}
 
 bool sizes_ok(int64_t a, int64_t b, int64_t c)
 {
@@ -161,21 +136,6 @@ bool sizes_ok(int64_t a, int64_t b, int64_t c)
 }
 
 }  // namespace
-
-uvt_status uvt_launch_gemm_f64(int32_t cfg, int64_t M, int64_t N, int64_t K, const double* A,
-                               int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc,
-                               hipStream_t s)
-{
-    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < N || ldc < N) return UVT_ERR_ARG;
-    if (!sizes_ok(M, N, K)) return UVT_ERR_SIZE;
-    const int64_t tm = uvt_cfg_tile_m(cfg), tn = uvt_cfg_tile_n(cfg);
-    if (((M + tm - 1) / tm) * ((N + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    if (cfg == UVT_CFG_64x64) launch_gemm<64, 64>(M, N, K, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_128x32) launch_gemm<128, 32>(M, N, K, A, lda, B, ldb, C, ldc, s);
-    else launch_gemm<128, 128>(M, N, K, A, lda, B, ldb, C, ldc, s);
-    UVT_HIP(hipGetLastError());
-    return UVT_OK;
-}
 
 extern "C" uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_t n,
                                 int64_t k, double alpha, const double* dA, int64_t lda,
@@ -195,44 +155,19 @@ extern "C" uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_
     UVT_HIP(hipSetDevice(h->device));
     hipStream_t s = (hipStream_t)stream;
     if (k == 0 || alpha == 0.0) {  // C = beta C, A and B not read
-        axpby(m, n, 0.0, nullptr, 0, beta, dC, ldc, s);
+        scale(m, n, beta, dC, ldc, s);
         UVT_HIP(hipGetLastError());
         return UVT_OK;
     }
-    const bool direct = alpha == 1.0 && beta == 0.0;
-    const int64_t lap = even(k), lbp = even(n), lpp = even(n);
-    const size_t a_bytes = tA ? up256((size_t)m * lap * 8) : 0;
-    const size_t b_bytes = tB ? up256((size_t)k * lbp * 8) : 0;
-    const size_t p_bytes = direct ? 0 : up256((size_t)m * lpp * 8);
-    void* w = nullptr;
-    if (a_bytes + b_bytes + p_bytes) {
-        uvt_status st = uvt_handle_workspace(h, a_bytes + b_bytes + p_bytes, &w);
-        if (st != UVT_OK) return st;
-    }
-    char* wp = (char*)w;
-    const double* Ap = dA;
-    int64_t la = lda;
-    if (tA) {  // op(A) = A^T: A stored k x m
-        pack(dA, lda, (double*)wp, lap, m, k, true, false, false, 1.0, false, false, s);
-        Ap = (const double*)wp;
-        la = lap;
-        wp += a_bytes;
-    }
-    const double* Bp = dB;
-    int64_t lb = ldb;
-    if (tB) {  // op(B) = B^T: B stored n x k
-        pack(dB, ldb, (double*)wp, lbp, k, n, true, false, false, 1.0, false, false, s);
-        Bp = (const double*)wp;
-        lb = lbp;
-        wp += b_bytes;
-    }
-    double* P = direct ? dC : (double*)wp;
-    const int64_t lp = direct ? ldc : lpp;
-    uvt_status st = uvt_launch_gemm_f64(uvt_default_cfg(m, n), m, n, k, Ap, la, Bp, lb, P, lp, s);
-    if (st != UVT_OK) return st;
-    if (!direct) axpby(m, n, alpha, P, lp, beta, dC, ldc, s);
-    UVT_HIP(hipGetLastError());
-    return UVT_OK;
+    const Walk g{m, n, (int)k, 0, 0};
+    TileEpi epi;
+    epi.alpha = alpha;
+    epi.beta = beta;
+    const int32_t cfg = uvt_default_cfg(m, n);
+    if (tA && tB) return launch_blas<false, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
+    if (tA) return launch_blas<false, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
+    if (tB) return launch_blas<true, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
+    return launch_blas<true, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
 }
 
 // ---- dtrmm ---------------------------------------------------------------------
@@ -250,12 +185,16 @@ namespace {
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices];  // per device, set once
 
-// One dtrmm call, reduced to R = tril(L) X (see the comment at the top of
-// this file): which operands are packed and the workspace bytes of each.
+// One dtrmm call: the triangle's order nt on w columns (rows, right side) of
+// B, and the workspace: a copy of B with an even leading dimension.
 struct DtrmmCall {
-    bool right, tA, rev, unit, tX, packL, packX;
-    int64_t nt, w, ll, lx, lr;
-    size_t l_bytes, x_bytes, r_bytes;
+    bool right, tA, lower, unit;  // lower: op(A) is
+    int64_t nt, w, ldx;
+    size_t bytes;
+    // What uvt_dtrmm_noalloc holds against its scratch: result, B where it is
+    // transposed or reversed and the triangle where it is not plain lower,
+    // each an array of its own.
+    size_t declared;
 };
 
 // Validates the arguments and sizes the workspace.  UVT_OK with
@@ -279,63 +218,51 @@ uvt_status dtrmm_prepare(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans t
     }
     if (!dB || (alpha != 0.0 && !dA)) return UVT_ERR_ARG;
     if (!sizes_ok(m, n, 1)) return UVT_ERR_SIZE;
-    // T = op(A) (left) or op(A)^T (right), the nt x nt factor applied to X
-    c->tA = (ta == UVT_TRANS) != c->right;
-    const bool t_lower = (uplo == UVT_LOWER) != c->tA;
-    c->rev = !t_lower;  // upper T: reverse rows and columns
+    c->tA = ta == UVT_TRANS;
+    c->lower = (uplo == UVT_LOWER) != c->tA;
     c->unit = diag == UVT_UNIT;
-    c->tX = c->right;   // X = B^T
-    c->packL = c->tA || c->rev || c->unit;
-    c->ll = even(c->nt);
-    c->lx = even(c->w);
-    c->lr = even(c->w);
-    c->l_bytes = c->packL ? up256((size_t)c->nt * c->ll * 8) : 0;
-    c->packX = c->tX || c->rev;  // else X is B itself (R is written elsewhere)
-    c->x_bytes = c->packX ? up256((size_t)c->nt * c->lx * 8) : 0;
-    c->r_bytes = up256((size_t)c->nt * c->lr * 8);
-    if (alpha == 0.0) {  // no workspace: B = 0, A not read
-        c->l_bytes = c->x_bytes = c->r_bytes = 0;
-    }
+    c->ldx = even(n);
+    c->bytes = up256((size_t)m * c->ldx * 8);
+    const size_t rect = up256((size_t)c->nt * even(c->w) * 8), square = up256((size_t)c->nt * even(c->nt) * 8);
+    const bool rev = c->lower == c->right;  // the triangle turned lower by reversal
+    c->declared = rect + (c->right || rev ? rect : 0) + (c->tA != c->right || rev || c->unit ? square : 0);
+    if (alpha == 0.0) c->bytes = c->declared = 0;  // no workspace: B = 0, A not read
     return UVT_OK;
 }
-
-size_t dtrmm_bytes(const DtrmmCall& c) { return c.l_bytes + c.x_bytes + c.r_bytes; }
 
 // Enqueues the call on stream s with its workspace at wv.
 uvt_status dtrmm_launch(const DtrmmCall& c, int64_t m, int64_t n, double alpha, const double* dA,
                         int64_t lda, double* dB, int64_t ldb, void* wv, hipStream_t s)
 {
     if (alpha == 0.0) {  // B = 0, A not read
-        axpby(m, n, 0.0, nullptr, 0, 0.0, dB, ldb, s);
+        scale(m, n, 0.0, dB, ldb, s);
         UVT_HIP(hipGetLastError());
         return UVT_OK;
     }
-    char* wp = (char*)wv;
-    const double* L = dA;
-    int64_t la = lda;
-    if (c.packL) {
-        pack(dA, lda, (double*)wp, c.ll, c.nt, c.nt, c.tA, c.rev, c.rev, 1.0, true, c.unit, s);
-        L = (const double*)wp;
-        la = c.ll;
-        wp += c.l_bytes;
+    double* X = (double*)wv;
+    const dim3 grid((unsigned)((n + 63) / 64), (unsigned)std::min<int64_t>((m + 15) / 16, 32768));
+    hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, s, dB, ldb, X, c.ldx, m, n);
+    const Walk g{m, n, (int)c.nt, 0, 0};
+    TileEpi epi;
+    epi.alpha = alpha;
+    epi.unit = c.unit;
+    if (!c.right) {
+        const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(m, n), m, n);
+        if (c.lower) {
+            if (c.tA) return launch_blas<false, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
+            return launch_blas<true, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
+        }
+        if (c.tA) return launch_blas<false, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
+        return launch_blas<true, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
     }
-    const double* X = dB;
-    int64_t lxx = ldb;
-    if (c.packX) {
-        pack(dB, ldb, (double*)wp, c.lx, c.nt, c.w, c.tX, c.rev, false, 1.0, false, false, s);
-        X = (const double*)wp;
-        lxx = c.lx;
-        wp += c.x_bytes;
+    // B op(A): column j of the product needs k >= j where op(A) is lower
+    const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(n, m), m, n);
+    if (c.lower) {
+        if (c.tA) return launch_blas<true, true, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
+        return launch_blas<true, false, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
     }
-    double* R = (double*)wp;
-    uvt_status st = uvt_launch_trapezoid_f64(uvt_wide_tiles(uvt_default_cfg(c.nt, c.w), c.nt, c.w), c.nt, c.w, L, la, X, lxx,
-                                             R, c.lr, s);
-    if (st != UVT_OK) return st;
-    // B <- alpha * unpack(R): B(i, j) = R(rmap(i), j) (left) or R(cmap(j), i) (right)
-    if (c.tX) pack(R, c.lr, dB, ldb, m, n, true, false, c.rev, alpha, false, false, s);
-    else pack(R, c.lr, dB, ldb, m, n, false, c.rev, false, alpha, false, false, s);
-    UVT_HIP(hipGetLastError());
-    return UVT_OK;
+    if (c.tA) return launch_blas<true, true, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
+    return launch_blas<true, false, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
 }
 
 }  // namespace
@@ -368,8 +295,8 @@ extern "C" uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_
     if (st != UVT_OK || nothing) return st;
     UVT_HIP(hipSetDevice(h->device));
     void* wv = nullptr;
-    if (dtrmm_bytes(c)) {
-        st = uvt_handle_workspace(h, dtrmm_bytes(c), &wv);
+    if (c.bytes) {
+        st = uvt_handle_workspace(h, c.bytes, &wv);
         if (st != UVT_OK) return st;
     }
     return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, wv, (hipStream_t)stream);
@@ -384,7 +311,7 @@ extern "C" uvt_status uvt_dtrmm_noalloc(uvt_handle h, uvt_side side, uvt_uplo up
     bool nothing = false;
     uvt_status st = dtrmm_prepare(h, side, uplo, ta, diag, m, n, alpha, dA, lda, dB, ldb, &c, &nothing);
     if (st != UVT_OK || nothing) return st;
-    if (dtrmm_bytes(c) > kNoAllocScratchBytes) return UVT_ERR_SIZE;
+    if (c.declared > kNoAllocScratchBytes) return UVT_ERR_SIZE;
     if (!h->scratch) return UVT_ERR_STATE;
     UVT_HIP(hipSetDevice(h->device));
     return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, h->scratch, (hipStream_t)stream);

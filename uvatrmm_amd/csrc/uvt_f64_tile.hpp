@@ -70,7 +70,7 @@ typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
 // every panel of an edge tile checked instead, the edge tiles were the last
 // to finish: 8165 x 939 took 1193 us instead of 1081, a 1500 x 2000 x 3000
 // dgemm in 64x64 tiles 387 instead of 342 (same bits).
-template <int X, int NT, bool KC>
+template <int X, int NT, bool KC, bool DOWN>
 struct Panel {
     using Idx = PanelIdx<X, NT, KC>;
     static constexpr int LD = KC ? kTileK + 2 : X + 16;
@@ -112,7 +112,7 @@ struct Panel {
     {
         at = reinterpret_cast<const UVT_GLOBAL char*>(KC ? p + k0 : p + (int64_t)k0 * ld);
     }
-    // The next panel in k, a full one.
+    // The next panel of the walk, a full one (DOWN: the walk goes down in k).
     __device__ __forceinline__ void load(int tid)
     {
 #pragma unroll
@@ -124,7 +124,8 @@ struct Panel {
             asm volatile("" : "+v"(o));
             r[q] = *reinterpret_cast<const UVT_GLOBAL dbl2u*>(at + q * (Idx::KSTEP * 8) * ld + o);
         }
-        at += KC ? (int64_t)kTileK * 8 : ld * (kTileK * 8);
+        const int64_t step = KC ? (int64_t)kTileK * 8 : ld * (kTileK * 8);
+        at += DOWN ? -step : step;
     }
 
     // Any panel: no load sits under a branch per element (such branches cost
@@ -214,11 +215,17 @@ enum TriKind {
 // shapes (the persistent batch kernel: 12 bytes of spills per lane instead
 // of 52, 1.5-3 % faster); the single-shape kernels ran 0.2-1.7 % slower
 // with it.  The sums and their order are the same either way.
+// PIPE_MASKED: the masked panels run the software pipeline too.  Without it
+// they leave 16 registers to their addresses and masks, which the kernels
+// with more of their own need (8165 x 939 stream-K 1033 us with it, 1021
+// without; 9000 x 250 in cut tiles 395 and 387; the batch 9.08 and 8.95 ms);
+// the plain walks are faster with it (4096^2: 992
+// us, 1004 without).
 template <bool A_KC_ = true, bool B_KC_ = false, TriKind TRI_ = kTriALe, bool UNIT_ = false, bool EPI_ = false,
-          bool EDGE_IDLE_ = true, bool AHEAD2_ = false>
+          bool EDGE_IDLE_ = true, bool AHEAD2_ = false, bool PIPE_MASKED_ = true>
 struct TileOpt {
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_, UNIT = UNIT_, EPI = EPI_, EDGE_IDLE = EDGE_IDLE_,
-                          AHEAD2 = AHEAD2_;
+                          AHEAD2 = AHEAD2_, PIPE_MASKED = PIPE_MASKED_;
     static constexpr TriKind TRI = TRI_;
     static constexpr bool TRI_A = TRI == kTriALe || TRI == kTriAGe, GE = TRI == kTriAGe || TRI == kTriBGe;
 };
@@ -228,8 +235,8 @@ struct F64Cfg {
     static constexpr int NT = 64 * WAVES_M * WAVES_N;
     static constexpr int WM = TM / WAVES_M, WN = TN / WAVES_N;
     static constexpr int FM = WM / 16, FN = WN / 16;
-    using PA = Panel<TM, NT, OPT::A_KC>;
-    using PB = Panel<TN, NT, OPT::B_KC>;
+    using PA = Panel<TM, NT, OPT::A_KC, OPT::GE>;
+    using PB = Panel<TN, NT, OPT::B_KC, OPT::GE>;
     static constexpr int SMEM_DOUBLES = 2 * (PA::ELEMS + PB::ELEMS);
     static_assert(FM >= 1 && FN >= 1, "wave tile below 16x16");
 };
@@ -265,7 +272,6 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
     using PA = typename G::PA;
     using PB = typename G::PB;
     constexpr int BK = kTileK;
-    static_assert(!(OPT::AHEAD2 && OPT::GE), "AHEAD2: no diagonal at the tile's start");
     constexpr bool AHEAD2 = OPT::AHEAD2, GE = OPT::GE, TRI_A = OPT::TRI_A, UNIT = OPT::UNIT;
     const int tid = thread >= 0 ? thread : (int)threadIdx.x;
     const int lane = tid & 63;
@@ -280,7 +286,8 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
 
     const int k_lo = t.k_lo, k_hi = t.k_hi;
     const int k_start = k_lo & ~1;
-    const int nk = (k_hi > k_start) ? (k_hi - k_start + BK - 1) / BK : 0;
+    const int nk = panels(k_lo, k_hi);
+    auto k_at = [&](int kt) { return panel_k0<GE>(k_lo, nk, kt); };
     const int cols = (int64_t)t.c0 + TN <= m ? TN : (int)(m - t.c0);
 
     PA pa;
@@ -369,6 +376,16 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         }
     };
     auto read0 = [&](int buf) { read(buf, 0, a2, b2, a1, b1); };
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < G::FM; ++i)
+#pragma unroll
+            for (int j = 0; j < G::FN; ++j) {
+                const double a = OPT::A_KC ? a2[i][s % 2] : a1[i];
+                const double b = OPT::B_KC ? b2[j][s % 2] : b1[j];
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[i][j], 0, 0, 0);
+            }
+    };
     auto compute = [&](int buf, auto&& st) {
 #pragma unroll
         for (int s = 0; s < BK / 4; ++s) {
@@ -380,14 +397,7 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
                 __syncthreads();
                 read(buf ^ 1, 0, na2, nb2, na1, nb1);
             }
-#pragma unroll
-            for (int i = 0; i < G::FM; ++i)
-#pragma unroll
-                for (int j = 0; j < G::FN; ++j) {
-                    const double a = OPT::A_KC ? a2[i][s % 2] : a1[i];
-                    const double b = OPT::B_KC ? b2[j][s % 2] : b1[j];
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[i][j], 0, 0, 0);
-                }
+            multiply(s);
             if (s == 1) st();
 #pragma unroll
             for (int i = 0; i < G::FM; ++i) {
@@ -407,6 +417,20 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
             }
         }
     };
+    // The masked panels (see PIPE_MASKED).
+    auto compute_masked = [&](int buf, auto&& st) {
+        if constexpr (OPT::PIPE_MASKED) {
+            compute(buf, st);
+            return;
+        }
+#pragma unroll
+        for (int s = 0; s < BK / 4; ++s) {
+            read(buf, s, a2, b2, a1, b1);
+            multiply(s);
+            if (s == 1) st();
+        }
+        __syncthreads();
+    };
 
     // Panels [f0, f1) need no masks: the steady-state loop, free of per-panel
     // branches.  The rest (next to the diagonal, at the tile's k ends) run
@@ -417,22 +441,22 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         const bool odd = (!OPT::A_KC && (t.rows & 1)) || (!OPT::B_KC && (cols & 1));
         // first and last coordinate of the triangular operand
         const int tx0 = TRI_A ? t.r0 : t.c0, tx1 = tx0 + (TRI_A ? t.rows : cols) - 1;
-        const FullPanels fp = full_panels<GE>(k_start, k_lo, k_hi, tri, unit, tx0, tx1, odd);
+        const FullPanels fp = full_panels<GE>(k_lo, k_hi, tri, unit, tx0, tx1, odd);
         const int f0 = fp.f0, f1 = PA::Idx::offsets_fit(lda) && PB::Idx::offsets_fit(ldb) ? fp.f1 : 0;
-        pa.seek(k_start + f0 * BK);
-        pb.seek(k_start + f0 * BK);
+        pa.seek(k_at(f0));
+        pb.seek(k_at(f0));
 
         const bool first_full = f0 == 0 && f1 > 0;
         if (first_full) {
-            load(k_start, full);
-            store(0, k_start, full);
+            load(k_at(0), full);
+            store(0, k_at(0), full);
         } else {
-            load(k_start, masked);
-            store(0, k_start, masked);
+            load(k_at(0), masked);
+            store(0, k_at(0), masked);
         }
         if (AHEAD2 && nk > 1) {
-            if (f0 <= 1 && 1 < f1) load(k_start + BK, full);
-            else load(k_start + BK, masked);
+            if (f0 <= 1 && 1 < f1) load(k_at(1), full);
+            else load(k_at(1), masked);
         }
         __syncthreads();
         // A panel whose k lies on the zero side of the triangle for all of a
@@ -445,46 +469,31 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         // writes nothing: outside the steady-state loop it runs no products.
         const bool idle = OPT::EDGE_IDLE && (wm * G::WM >= t.rows || wn * G::WN >= cols);
         int kt = 0;
-        if constexpr (!GE) read0(0);
-        if constexpr (GE) {  // the diagonal comes first
-            const int wx0 = tx0 + (TRI_A ? wm * G::WM : wn * G::WN);  // this wave's first row (column)
-            const int kw = idle ? f0 : (wx0 - k_start) / BK;           // its first panel that is not all zeros
-            for (; kt + 1 < f0 && kt + 1 < nk; ++kt) {
-                load(k_start + (kt + 1) * BK, masked);
-                if (kt >= kw) {
-                    if (kt == max(kw, 0)) read0(kt & 1);
-                    compute(kt & 1, [&] { store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked); });
-                } else {
-                    store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
-                    __syncthreads();
-                }
-            }
-            if (kt <= max(kw, 0)) read0(kt & 1);
-        }
+        if (OPT::PIPE_MASKED || kt + 1 < f1) read0(kt & 1);
         // Registers hold the next panel's values from here on when AHEAD2.
         if constexpr (AHEAD2) {
             if (idle) {  // this wave only feeds the others
                 for (; kt + 2 < f1; ++kt) {
                     store((kt & 1) ^ 1, 0, full);
-                    load(k_start + (kt + 2) * BK, full);
+                    load(k_at(kt + 2), full);
                     __syncthreads();
                 }
             }
             for (; kt + 2 < f1; ++kt) {  // the panel after next is full
                 compute(kt & 1, [&] {
                     store((kt & 1) ^ 1, 0, full);
-                    load(k_start + (kt + 2) * BK, full);
+                    load(k_at(kt + 2), full);
                 });
             }
         } else if (idle) {  // this wave only feeds the others
             for (; kt + 1 < f1; ++kt) {
-                load(k_start + (kt + 1) * BK, full);
+                load(k_at(kt + 1), full);
                 store((kt & 1) ^ 1, 0, full);
                 __syncthreads();
             }
         } else {
             for (; kt + 1 < f1; ++kt) {  // the next panel is full
-                load(k_start + (kt + 1) * BK, full);
+                load(k_at(kt + 1), full);
                 compute(kt & 1, [&] { store((kt & 1) ^ 1, 0, full); });
             }
         }
@@ -494,24 +503,28 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         int nk_w = nk;
         if (idle) nk_w = kt;
         else if (tri && !GE) {
-            // last row (column) of this wave, inside C
+            // last row (column) of this wave
             const int last = tx0 + (TRI_A ? wm * G::WM + G::WM : wn * G::WN + G::WN) - 1;
             nk_w = last >= k_start ? (last - k_start) / BK + 1 : 0;
             nk_w = nk_w < kt ? kt : (nk_w > nk ? nk : nk_w);
+        } else if (tri) {
+            const int first = tx0 + (TRI_A ? wm * G::WM : wn * G::WN);  // first row (column) of this wave
+            nk_w = nk - (first > k_start ? (first - k_start) / BK : 0);
+            nk_w = nk_w < kt ? kt : nk_w;
         }
         for (; kt < nk_w; ++kt) {
             const bool more = kt + 1 < nk;
-            if (!AHEAD2 && more) load(k_start + (kt + 1) * BK, masked);
-            compute(kt & 1, [&] {
-                if (more) store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
-                if (AHEAD2 && kt + 2 < nk) load(k_start + (kt + 2) * BK, masked);
+            if (!AHEAD2 && more) load(k_at(kt + 1), masked);
+            compute_masked(kt & 1, [&] {
+                if (more) store((kt & 1) ^ 1, k_at(kt + 1), masked);
+                if (AHEAD2 && kt + 2 < nk) load(k_at(kt + 2), masked);
             });
         }
         for (; kt < nk; ++kt) {
             if (kt + 1 < nk) {
-                if (!AHEAD2) load(k_start + (kt + 1) * BK, masked);
-                store((kt & 1) ^ 1, k_start + (kt + 1) * BK, masked);
-                if (AHEAD2 && kt + 2 < nk) load(k_start + (kt + 2) * BK, masked);
+                if (!AHEAD2) load(k_at(kt + 1), masked);
+                store((kt & 1) ^ 1, k_at(kt + 1), masked);
+                if (AHEAD2 && kt + 2 < nk) load(k_at(kt + 2), masked);
             }
             __syncthreads();
         }
@@ -569,6 +582,9 @@ template <> struct TileWaves<64, 64> {
 };
 template <> struct TileWaves<128, 32> {
     static constexpr int M = 4, N = 1, BLOCKS_PER_CU = 3, WAVES_PER_EU = 3;
+};
+template <> struct TileWaves<32, 128> {  // few rows: the right-side forms of the BLAS calls
+    static constexpr int M = 1, N = 4, BLOCKS_PER_CU = 3, WAVES_PER_EU = 3;
 };
 
 }  // namespace uvt

@@ -67,28 +67,43 @@ __host__ __device__ inline int near_k(int k, int x, int k_hi, bool tri)
     return k;
 }
 
-// Panels [f0, f1) of a tile need no masks: inside [k_lo, k_hi) (only panel 0
-// can start below an odd k_lo), off the diagonal of the triangle whose x run
-// from tx0 to tx1 (unit: the diagonal itself is replaced too), and away from
-// the last k row where odd asks for it.
+// The tile's panels in the order it runs them, kt = 0 .. panels() - 1: up in k,
+// or down (GE), so that the triangle's diagonal always comes last.
+__host__ __device__ inline int panels(int k_lo, int k_hi)
+{
+    const int k_start = k_lo & ~1;
+    return k_hi > k_start ? (k_hi - k_start + kTileK - 1) / kTileK : 0;
+}
+template <bool GE>
+__host__ __device__ inline int panel_k0(int k_lo, int nk, int kt)
+{
+    return (k_lo & ~1) + (GE ? nk - 1 - kt : kt) * kTileK;
+}
+
+// Panels kt in [f0, f1) of that order need no masks: inside [k_lo, k_hi) (only
+// the first can start below an odd k_lo, or pass k_hi on the way down), off
+// the diagonal of the triangle whose x run from tx0 to tx1 (unit: the
+// diagonal itself is replaced too), and away from the last k row where odd
+// asks for it.  f0 is 0 or 1.  (GE: k_lo is even.)
 struct FullPanels {
     int f0, f1;
 };
 template <bool GE>
-__host__ __device__ inline FullPanels full_panels(int k_start, int k_lo, int k_hi, bool tri, bool unit, int tx0,
-                                                  int tx1, bool odd)
+__host__ __device__ inline FullPanels full_panels(int k_lo, int k_hi, bool tri, bool unit, int tx0, int tx1, bool odd)
 {
+    const int k_start = k_lo & ~1, nk = panels(k_lo, k_hi);
     int lim = k_hi, f0 = k_start < k_lo ? 1 : 0;
     if (tri && !GE) {
         const int d = tx0 + (unit ? 0 : 1);
         lim = lim < d ? lim : d;
     }
     if (tri && GE) {
-        const int d = tx1 + (unit ? 1 : 0) - k_start, f = d > 0 ? (d + kTileK - 1) / kTileK : 0;
-        f0 = f0 > f ? f0 : f;
+        const int d = tx1 + (unit ? 1 : 0) - k_start;
+        f0 = d > 0 ? (d + kTileK - 1) / kTileK : 0;
     }
     lim -= odd ? 1 : 0;
-    return FullPanels{f0, lim > k_start ? (lim - k_start) / kTileK : 0};
+    const int f1 = lim > k_start ? (lim - k_start) / kTileK : 0;
+    return GE ? FullPanels{nk - f1, nk - f0} : FullPanels{f0, f1};
 }
 
 }  // namespace uvt

@@ -62,12 +62,6 @@ UVT_INTERNAL int64_t uvt_sk_workgroups(int32_t cfg, int64_t n, int64_t m, int cu
 UVT_INTERNAL size_t uvt_sk_parts_bytes(int32_t cfg, int64_t workgroups);
 // The most partial-tile bytes any uvt_sk_workgroups result needs on `cus` CUs.
 UVT_INTERNAL size_t uvt_sk_max_parts_bytes(int cus);
-// FP64 C[0:M, 0:N] = A[0:M, 0:K] * B[0:K, 0:N] (no triangle), tile coordinates
-// from the workgroup index.
-UVT_INTERNAL uvt_status uvt_launch_gemm_f64(int32_t cfg, int64_t M, int64_t N, int64_t K, const double* A,
-                               int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc,
-                               hipStream_t s);
-
 // Tile-shape table written by uvt_autotune_f64: entries matched in order,
 // the first with n <= n_max and m <= m_max gives the shape.
 struct uvt_tune_entry {
