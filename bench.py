@@ -627,16 +627,15 @@ def main():
     cfg0 = int(plan.tiles(0)["cfg"][0]) if len(plan.tiles(0)) else 0
     tile, waves = {0: ("128,128", "8 waves of 32x64"), 1: ("64,64", "4 waves of 32x32"),
                    2: ("128,32", "4 waves of 32x32"), 4: ("256,128", "16 waves of 32x64")}[cfg0]
-    vec = "true" if n % 2 == 0 and m % 2 == 0 else "false"
-    launches = plan.phases
-    if parts and cfg0 == 0 and plan.phases == 1:
-        kernel = f"k_trmm_sk_f64<128,128,{vec}> (stream-K, {wg} workgroups) + k_sk_fixup"
+    launches = 1
+    if parts and cfg0 == 0:
+        kernel = f"k_trmm_sk_f64<128,128> (stream-K, {wg} workgroups) + k_sk_fixup"
         launches = 2
     elif parts:
-        kernel = f"k_trmm_tiles_f64<{tile},{vec}> ({waves}; reductions cut into pieces) + k_add_parts"
-        launches = plan.phases + 1
+        kernel = f"k_trmm_tiles_f64<{tile}> ({waves}; reductions cut into pieces) + k_add_parts"
+        launches = 2
     else:
-        kernel = f"k_trmm_tiles_f64<{tile},{vec}> ({waves})"
+        kernel = f"k_trmm_tiles_f64<{tile}> ({waves})"
     out = {
         "metric": "TRMM TFLOP/s + % MFMA peak at N=32768 (plain FP64 = value; split in 'split')",
         "value": round(value, 4),

@@ -68,8 +68,10 @@ typedef struct {
 
 typedef enum { UVT_MAP_REG = 0, UVT_MAP_BALANCED = 1 } uvt_map;
 /* boxes: per band a rectangular GEMM box over k in [0, b] followed by the
- * (h-1)-row diagonal triangle accumulated into C (two launches).
- * trapezoid: one triangle-aware tile walk over the lower trapezoid. */
+ * (h-1)-row diagonal triangle added to it.  trapezoid: one triangle-aware tile
+ * walk over the lower trapezoid.  The shape decides the plan's tile list; the
+ * device runs one walk over the lower trapezoid for either, so C is written
+ * once. */
 typedef enum { UVT_SHAPE_BOXES = 0, UVT_SHAPE_TRAPEZOID = 1 } uvt_shape;
 typedef enum { UVT_PREC_F64 = 0, UVT_PREC_SPLIT = 1 } uvt_prec;
 
@@ -111,7 +113,8 @@ typedef struct {
 uvt_status uvt_plan_create(int64_t n, int64_t m, uint32_t p, uvt_map map, uvt_shape shape,
                            uvt_plan *out, int *ref_exit);
 uvt_status uvt_plan_destroy(uvt_plan plan);
-/* Number of launches (phases): 2 for boxes, 1 for trapezoid. */
+/* Phases of the plan's tile list: 2 for boxes (boxes, triangles), 1 for
+ * trapezoid. */
 int32_t uvt_plan_phases(uvt_plan plan);
 int64_t uvt_plan_num_tiles(uvt_plan plan, int32_t phase);
 uvt_status uvt_plan_get_tiles(uvt_plan plan, int32_t phase, uvt_tile *out, int64_t cap);
@@ -138,12 +141,14 @@ int32_t uvt_device_cus(uvt_handle h);
  * 16-deep k panels of B, so a NaN or infinity in B[k][j] also reaches the
  * rows above k in k's 128-row tile through A's structural zeros (0 * Inf =
  * NaN), where a BLAS dtrmm would leave them finite; finite inputs are not
- * affected.  On its first use on a device the plan allocates its launch
- * records there.  A trapezoid plan of at least 2e9 flops whose whole tiles
- * would not finish together (narrow B: few, deep tiles) splits its long
- * reductions and adds the pieces after the first of a tile to C afterwards
- * in k order (results repeat bit for bit), with up to 64 MiB of partial
- * tiles on the device: with 128x128 tiles whose whole-tile span is 1.3x or
+ * affected.  Small products (at most 13000 16x16 tiles of C, under 6e9 to 8e9
+ * flops) run as one wave per tile and keep nothing on the device; for others
+ * the plan allocates its launch records there on its first use on a device.
+ * A plan of at least 2e9 flops whose whole tiles would not finish together
+ * (narrow B: few, deep tiles) splits its long reductions and adds the pieces
+ * after the first of a tile to C afterwards in k order (results repeat bit for
+ * bit), with up to 64 MiB of partial tiles on the device: with 128x128 tiles
+ * whose whole-tile span is 1.3x or
  * more an even share of the work, stream-K (up to one workgroup per slot,
  * each the same number of k panels, in groups that run a row tile's column
  * tiles side by side); with smaller tiles whose deepest tile is 1.5x or

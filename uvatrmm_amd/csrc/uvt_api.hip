@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "uvt_f64_tile.hpp"
+#include "uvt_f64_wave.hpp"
 #include "uvt_internal.h"
 #include "uvt_runtime.hpp"
 #include "uvt_sk.hpp"
@@ -94,6 +95,28 @@ void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, const double* 
     const int rows = (int)(n - r0 < TM ? n - r0 : TM);
     f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, ct * TN, 0, r0 + rows, kTileLower}, gbl(A), lda, gbl(B), ldb,
                                  gbl(C), ldc, m, smem);
+}
+
+// The trapezoid walk of a small product in wave tiles (uvt_f64_wave.hpp), four
+// to a workgroup, wn of them along the columns: deepest first, every second
+// run of `snake` workgroups turned round (see snake()).
+template <int FM, int FN, int D>
+__global__ __launch_bounds__(256) void k_trmm_waves_f64(int64_t n, int64_t m, int nrt, int nct, int wn, int snake,
+                                                        const double* __restrict__ A, int64_t lda,
+                                                        const double* __restrict__ B, int64_t ldb,
+                                                        double* __restrict__ C, int64_t ldc)
+{
+    int b = (int)blockIdx.x;
+    const int g = snake > 0 ? b / snake : 0;
+    if (g & 1) b = g * snake + min((g + 1) * snake, (int)gridDim.x) - 1 - b;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int rt = (nrt - 1 - b / nct) * (4 / wn) + wave / wn, ct = b % nct * wn + wave % wn;
+    const int64_t r0 = (int64_t)rt * (16 * FM), c0 = (int64_t)ct * (16 * FN);
+    __shared__ __attribute__((aligned(16))) double lds[4][wave_lds<FM, FN, TileOpt<>>()];
+    if (r0 >= n || c0 >= m) return;
+    const int rows = (int)(n - r0 < 16 * FM ? n - r0 : 16 * FM);
+    f64_wave<FM, FN, D>(TileArgs{(int)r0, rows, (int)c0, 0, (int)r0 + rows, kTileLower}, gbl(A), lda, gbl(B), ldb,
+                        gbl(C), ldc, m, lds[wave]);
 }
 
 // The trapezoid walk split stream-K (uvt_sk.hpp): workgroup w of group
@@ -342,7 +365,7 @@ uvt_status uvt_handle_workspace(uvt_handle h, size_t bytes, void** p)
 extern "C" void uvt_plan_release_device(uvt_plan plan)
 {
     if (!plan) return;
-    void** bufs[4] = {&plan->dev_launch[0], &plan->dev_launch[1], &plan->dev_sums, &plan->dev_parts};
+    void** bufs[3] = {&plan->dev_launch, &plan->dev_sums, &plan->dev_parts};
     for (void** b : bufs) {
         if (*b) {
             (void)hipSetDevice(plan->dev_id);
@@ -350,7 +373,7 @@ extern "C" void uvt_plan_release_device(uvt_plan plan)
             *b = nullptr;
         }
     }
-    plan->nlaunch[0] = plan->nlaunch[1] = plan->nsums = plan->nparts = plan->sk_grid = 0;
+    plan->nlaunch = plan->nsums = plan->nparts = plan->sk_grid = 0;
     plan->dev_id = -1;
 }
 
@@ -374,8 +397,20 @@ int blocks_per_cu(int32_t cfg)
     return TileWaves<128, 128>::BLOCKS_PER_CU;
 }
 
-// The launches of a plan on a GPU of `cus` compute units: its phases, one
-// launch each, with whole tiles, except for a trapezoid plan whose longest
+// Tiles that all fit the GPU at once are placed, not scheduled: workgroups i,
+// i + cus, i + 2 cus, ... of a launch run on one compute unit (checked on the
+// GPU: 1024 of 1024 workgroups, three launches).  So every second run of cus
+// tiles is turned round, and a compute unit's deep tiles meet shallow ones.
+void snake(std::vector<LaunchTile>& v, int cus)
+{
+    for (size_t g = cus; g < v.size(); g += 2 * (size_t)cus)
+        std::reverse(v.begin() + g, v.begin() + std::min(g + cus, v.size()));
+}
+
+// The launch of a plan on a GPU of `cus` compute units: the whole tiles of the
+// trapezoid walk, for either shape.  (A boxes plan's triangles were a second
+// launch, which read and wrote C once more and waited for the first: N=2048,
+// 4 bands, product and norm 193 us; now 170.)  Except for a plan whose longest
 // reduction is much longer than an even share of the work would give a
 // workgroup slot (narrow B, few tiles: the launch then lasts as long as its
 // deepest tile).  Such a plan cuts every reduction longer than about half
@@ -383,37 +418,37 @@ int blocks_per_cu(int32_t cfg)
 // the others write partial tiles, which k_add_parts adds to C afterwards in
 // k order.  Measured at 9000 x 250 (the deepest tile 2.7x the share): 0.73
 // -> 0.45 ms; at 4096 x 4096 (0.97x) cutting cost 7 %, between 0.9x and
-// 1.6x it changed -1 to +7 %, and cutting the boxes of the N=2048 boxes
-// plan (1.5x) cost 11 %, so boxes plans and plans below 1.5x keep whole
-// tiles (and the kernel without partial tiles).  (A trapezoid plan of
-// 128x128 tiles whose whole tiles would not finish together runs stream-K
-// instead, decided before this in plan_upload; so cuts serve the smaller
-// tile shapes, where they were faster than stream-K.)
-void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile> launch[2],
-                  std::vector<PartSum>& sums, int64_t& nparts)
+// 1.6x it changed -1 to +7 %, so plans below 1.5x keep whole tiles (and the
+// kernel without partial tiles); 64x64 tiles count three slots to a compute
+// unit here, as those figures did, though four fit.  (A plan of 128x128 tiles
+// whose whole tiles would not finish together runs stream-K instead, decided
+// before this in plan_upload; so cuts serve the smaller tile shapes, where
+// they were faster than stream-K.)
+void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile>& launch, std::vector<PartSum>& sums,
+                  int64_t& nparts)
 {
-    for (int ph = 0; ph < 2; ++ph) launch[ph].clear();
+    launch.clear();
     sums.clear();
     nparts = 0;
-    for (int ph = 0; ph < pl.phases; ++ph)
-        for (int64_t i = 0; i < pl.ntiles[ph]; ++i) launch[ph].push_back(LaunchTile{pl.tiles[ph][i], -1});
-    if (pl.phases != 1 || pl.flops < kSplitMinFlops || pl.ntiles[0] == 0) return;
-    const int64_t slots = (int64_t)cus * blocks_per_cu(pl.cfg);
+    std::vector<uvt_tile> walk(uvt_plan_trapezoid_tiles(pl.n, pl.m, pl.cfg, nullptr));
+    uvt_plan_trapezoid_tiles(pl.n, pl.m, pl.cfg, walk.data());  // deepest first
+    for (const uvt_tile& t : walk) launch.push_back(LaunchTile{t, -1});
+    if ((int64_t)launch.size() <= (int64_t)cus * blocks_per_cu(pl.cfg)) snake(launch, cus);
+    if (pl.flops < kSplitMinFlops) return;
     int64_t work = 0, deepest = 0;  // k steps, summed over the tiles and the longest
-    for (int64_t i = 0; i < pl.ntiles[0]; ++i) {
-        const int64_t len = (int64_t)pl.tiles[0][i].k_hi - pl.tiles[0][i].k_lo;
+    for (const uvt_tile& w : walk) {
+        const int64_t len = (int64_t)w.k_hi - w.k_lo;
         work += len;
         deepest = len > deepest ? len : deepest;
     }
-    const int64_t share = work / slots;
+    const int64_t share = work / ((int64_t)cus * std::min(blocks_per_cu(pl.cfg), 3));
     if (2 * deepest < 3 * share) return;
     int64_t kc = (share / 2 + 127) / 128 * 128;
     kc = kc < 512 ? 512 : kc;
     std::vector<LaunchTile> cut;
     std::vector<PartSum> cut_sums;
     int64_t cut_parts = 0;
-    for (int64_t i = 0; i < pl.ntiles[0]; ++i) {
-        const uvt_tile& t = pl.tiles[0][i];
+    for (const uvt_tile& t : walk) {
         const int64_t len = (int64_t)t.k_hi - t.k_lo;
         const int64_t np = len > kc ? (len + kc - 1) / kc : 1;
         if (np == 1) {
@@ -431,11 +466,11 @@ void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile> launch[
     }
     const size_t tile_bytes = (size_t)uvt_cfg_tile_m(pl.cfg) * uvt_cfg_tile_n(pl.cfg) * sizeof(double);
     if ((size_t)cut_parts * tile_bytes > kMaxPartBytes) return;
-    // deepest first (the planner's order among equals)
+    // deepest first (the walk's order among equals)
     std::stable_sort(cut.begin(), cut.end(), [](const LaunchTile& a, const LaunchTile& b) {
         return a.t.k_hi - a.t.k_lo > b.t.k_hi - b.t.k_lo;
     });
-    launch[0].swap(cut);
+    launch.swap(cut);
     sums.swap(cut_sums);
     nparts = cut_parts;
 }
@@ -446,9 +481,9 @@ static uvt_status plan_upload(uvt_handle h, uvt_plan plan)
 {
     if (plan->dev_id == h->device) return UVT_OK;
     uvt_plan_release_device(plan);
-    // A trapezoid plan whose whole tiles would not finish together runs
-    // stream-K: nothing to upload but its partial tiles.
-    const int64_t sk = plan->phases == 1 ? uvt_sk_workgroups(plan->cfg, plan->n, plan->m, h->cus) : 0;
+    // A plan whose whole tiles would not finish together runs stream-K:
+    // nothing to upload but its partial tiles.
+    const int64_t sk = uvt_sk_workgroups(plan->cfg, plan->n, plan->m, h->cus);
     if (sk > 0) {
         if (hipMalloc(&plan->dev_parts, uvt_sk_parts_bytes(plan->cfg, sk)) != hipSuccess) {
             (void)hipGetLastError();
@@ -463,7 +498,7 @@ static uvt_status plan_upload(uvt_handle h, uvt_plan plan)
             if (sk_piece(g, sk_start(g, b), sk_start(g, b + 1)).p0 > 0) plan->nparts += g.ncg;
         return UVT_OK;
     }
-    std::vector<LaunchTile> launch[2];
+    std::vector<LaunchTile> launch;
     std::vector<PartSum> sums;
     int64_t nparts = 0;
     build_launch(*plan, h->cus, launch, sums, nparts);
@@ -481,16 +516,14 @@ static uvt_status plan_upload(uvt_handle h, uvt_plan plan)
     };
     plan->dev_id = h->device;  // what is allocated below belongs to this device
     uvt_status st = UVT_OK;
-    for (int ph = 0; ph < 2 && st == UVT_OK; ++ph) {
-        if (nparts > 0) {
-            st = upload(&plan->dev_launch[ph], launch[ph].data(), launch[ph].size() * sizeof(LaunchTile));
-        } else {  // whole tiles: the plain records of the kernel without partial tiles
-            std::vector<uvt_tile> plain;
-            for (const LaunchTile& lt : launch[ph]) plain.push_back(lt.t);
-            st = upload(&plan->dev_launch[ph], plain.data(), plain.size() * sizeof(uvt_tile));
-        }
-        plan->nlaunch[ph] = (int64_t)launch[ph].size();
+    if (nparts > 0) {
+        st = upload(&plan->dev_launch, launch.data(), launch.size() * sizeof(LaunchTile));
+    } else {  // whole tiles: the plain records of the kernel without partial tiles
+        std::vector<uvt_tile> plain;
+        for (const LaunchTile& lt : launch) plain.push_back(lt.t);
+        st = upload(&plan->dev_launch, plain.data(), plain.size() * sizeof(uvt_tile));
     }
+    plan->nlaunch = (int64_t)launch.size();
     if (st == UVT_OK) st = upload(&plan->dev_sums, sums.data(), sums.size() * sizeof(PartSum));
     plan->nsums = (int64_t)sums.size();
     const int32_t tm = uvt_cfg_tile_m(plan->cfg), tn = uvt_cfg_tile_n(plan->cfg);
@@ -539,6 +572,76 @@ static void launch_trapezoid(int64_t n, int64_t m, const double* A, int64_t lda,
     const int nrt = (int)((n + TM - 1) / TM), nct = (int)((m + TN - 1) / TN);
     const dim3 grid((unsigned)((int64_t)nrt * nct)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
     hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN>), grid, block, 0, s, n, m, nrt, nct, A, lda, B, ldb, C, ldc);
+}
+
+// When a product runs in wave tiles, and in which (0: workgroup tiles): a rule
+// on the 16x16 tiles of C and the flops.  Measured on MI355X, 68 shapes from
+// 64 x 16 to 32000 x 32 (us; workgroup tiles / wave tiles of 16x16, 16x32,
+// 32x32):
+//     257 x 257      14.3 /   5.9    7.5   13.5     (289 tiles of 16x16)
+//    1000 x 200      43.3 /  15.7   20.2   39.5     (819)
+//     700 x 700      32.7 /  14.8   16.7   30.5     (1936)
+//     400 x 1600     20.5 /  11.6   12.2   19.1     (2500)
+//    1024 x 1024     44.9 /  28.7   22.9   42.0     (4096)
+//    1200 x 1200     52.4 /  48.3   39.5   49.3     (5625)
+//    1600 x 1600     98.4 / 108     91.7   80.0     (10000)
+//    1800 x 1800    127   / 182    159    123       (12769)
+//    2048 x 2048    136   / 202    154    155       (16384)
+// and, deep and narrow, where workgroup tiles cut their reductions:
+//    5000 x 128     106   /  89.0   89.3  184       (3.2e9 flops)
+//    5000 x 250     151   / 198    143    187       (6.2e9)
+//    5000 x 300     169   / 267    186    188       (7.5e9)
+//    4000 x 500     172   / 210    160    156       (8.0e9)
+//    9000 x 250     386   / 711    504    413       (2.0e10)
+// Small tiles share less per load, so each size's waves go from 16x16 to
+// 16x32 to 32x32 as there are enough of them for every SIMD; 32x32 ones need
+// reductions to spread (400 x 8192: 35.3 us in workgroup tiles, 34.4 in
+// 16x32, 40.5 in 32x32).
+int uvt_wave_shape(int64_t n, int64_t m, int64_t lda, int64_t ldb)
+{
+    const int64_t tiles = ((n + 15) / 16) * ((m + 15) / 16);
+    const double flops = (double)m * (double)n * (double)n;
+    if (n > 32768 || tiles > 13000 || flops >= (tiles > 7500 ? 8e9 : 6e9)) return 0;
+    if (!WaveOperand<2, true, false>::fits(lda) || !WaveOperand<2, false, false>::fits(ldb)) return 0;
+    return tiles <= 2500 ? 11 : tiles <= 7500 || n < 512 ? 12 : 22;
+}
+
+namespace {
+
+// Workgroups of four waves: wn of them along the columns, the rest along the
+// rows.
+struct WaveGrid {
+    int nrt, nct, wn;
+    int64_t launch() const { return (int64_t)nrt * nct; }
+};
+WaveGrid wave_grid(int shape, int64_t n, int64_t m)
+{
+    const int64_t tm = 16 * (shape / 10), tn = 16 * (shape % 10);
+    const int64_t rt = (n + tm - 1) / tm, ct = (m + tn - 1) / tn;
+    const int wn = ct > 1 ? 2 : 1, wm = 4 / wn;
+    return WaveGrid{(int)((rt + wm - 1) / wm), (int)((ct + wn - 1) / wn), wn};
+}
+
+template <int FM, int FN, int D>
+void launch_waves(int64_t n, int64_t m, const double* A, int64_t lda, const double* B, int64_t ldb, double* C,
+                  int64_t ldc, int cus, hipStream_t s)
+{
+    const WaveGrid g = wave_grid(10 * FM + FN, n, m);
+    hipLaunchKernelGGL((k_trmm_waves_f64<FM, FN, D>), dim3((unsigned)g.launch()), dim3(256), 0, s, n, m, g.nrt, g.nct,
+                       g.wn, cus, A, lda, B, ldb, C, ldc);
+}
+
+}  // namespace
+
+uvt_status uvt_launch_waves_f64(int shape, int64_t n, int64_t m, const double* A, int64_t lda, const double* B,
+                                int64_t ldb, double* C, int64_t ldc, int cus, hipStream_t s)
+{
+    if (n <= 0 || m <= 0 || lda < n || ldb < m || ldc < m) return UVT_ERR_ARG;
+    if (shape == 11) launch_waves<1, 1, 4>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    else if (shape == 12) launch_waves<1, 2, 4>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    else launch_waves<2, 2, 2>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    UVT_HIP(hipGetLastError());
+    return UVT_OK;
 }
 
 template <int TM, int TN>
@@ -651,25 +754,24 @@ extern "C" uvt_status uvt_trmm_f64(uvt_handle h, uvt_plan plan, const double* dA
     if (!h || !plan || !dA || !dB || !dC) return UVT_ERR_ARG;
     if (lda < plan->n || ldb < plan->m || ldc < plan->m) return UVT_ERR_ARG;
     UVT_HIP(hipSetDevice(h->device));
+    hipStream_t s = (hipStream_t)stream;
+    if (const int shape = uvt_wave_shape(plan->n, plan->m, lda, ldb))
+        return uvt_launch_waves_f64(shape, plan->n, plan->m, dA, lda, dB, ldb, dC, ldc, h->cus, s);
     uvt_status st = plan_upload(h, plan);
     if (st != UVT_OK) return st;
-    hipStream_t s = (hipStream_t)stream;
     double* parts = (double*)plan->dev_parts;
     if (plan->sk_grid > 0)
         return uvt_launch_trapezoid_sk_f64(plan->cfg, plan->n, plan->m, dA, lda, dB, ldb, dC, ldc,
                                            plan->sk_grid, parts, s);
     if (plan->nsums > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    for (int ph = 0; ph < 2; ++ph) {
-        st = launch_tiles_f64(plan->cfg, plan->dev_launch[ph], plan->nlaunch[ph], dA, lda, dB, ldb,
-                              dC, ldc, plan->m, plan->nparts > 0 ? parts : nullptr, s);
-        if (st != UVT_OK) return st;
-        if (ph == 0 && plan->nsums > 0) {  // the partial tiles belong to phase 0
-            const int32_t tm = uvt_cfg_tile_m(plan->cfg), tn = uvt_cfg_tile_n(plan->cfg);
-            hipLaunchKernelGGL(k_add_parts, dim3((unsigned)plan->nsums), dim3(256), 0, s,
-                               (const PartSum*)plan->dev_sums, (int)tn, (int)(tm * tn),
-                               (const double*)parts, dC, ldc, plan->m);
-            UVT_HIP(hipGetLastError());
-        }
+    st = launch_tiles_f64(plan->cfg, plan->dev_launch, plan->nlaunch, dA, lda, dB, ldb, dC, ldc, plan->m,
+                          plan->nparts > 0 ? parts : nullptr, s);
+    if (st != UVT_OK) return st;
+    if (plan->nsums > 0) {
+        const int32_t tm = uvt_cfg_tile_m(plan->cfg), tn = uvt_cfg_tile_n(plan->cfg);
+        hipLaunchKernelGGL(k_add_parts, dim3((unsigned)plan->nsums), dim3(256), 0, s, (const PartSum*)plan->dev_sums,
+                           (int)tn, (int)(tm * tn), (const double*)parts, dC, ldc, plan->m);
+        UVT_HIP(hipGetLastError());
     }
     return UVT_OK;
 }
@@ -678,6 +780,11 @@ extern "C" uvt_status uvt_plan_launch_info(uvt_handle h, uvt_plan plan, int64_t*
                                            int64_t* partial_tiles)
 {
     if (!h || !plan) return UVT_ERR_ARG;
+    if (const int shape = uvt_wave_shape(plan->n, plan->m, plan->n, plan->m)) {
+        if (workgroups) *workgroups = wave_grid(shape, plan->n, plan->m).launch();
+        if (partial_tiles) *partial_tiles = 0;
+        return UVT_OK;
+    }
     UVT_HIP(hipSetDevice(h->device));
     const uvt_status st = plan_upload(h, plan);
     if (st != UVT_OK) return st;
@@ -685,7 +792,7 @@ extern "C" uvt_status uvt_plan_launch_info(uvt_handle h, uvt_plan plan, int64_t*
         *workgroups = plan->sk_grid > 0 ? sk_launch(sk_geometry(plan->n, plan->m, uvt_cfg_tile_m(plan->cfg),
                                                                 uvt_cfg_tile_n(plan->cfg), plan->sk_grid,
                                                                 kSkGroupCols))
-                                        : plan->nlaunch[0] + plan->nlaunch[1];
+                                        : plan->nlaunch;
     if (partial_tiles) *partial_tiles = plan->nparts;
     return UVT_OK;
 }

@@ -38,12 +38,11 @@ struct uvt_plan_s {
     uvt_tile *tiles[2];
     double flops, issued;
     /* device state, owned by the plan, created by the HIP side on first use
-     * on a device: launch records of one or two launches, and, when tiles
-     * write partial products, the partial tiles and the records that add
-     * them to C */
+     * on a device: the launch's records, and, when tiles write partial
+     * products, the partial tiles and the records that add them to C */
     int dev_id;
-    void *dev_launch[2];
-    int64_t nlaunch[2];
+    void *dev_launch;
+    int64_t nlaunch;
     void *dev_sums;
     int64_t nsums;
     void *dev_parts;

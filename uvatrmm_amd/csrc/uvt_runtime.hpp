@@ -46,6 +46,14 @@ UVT_INTERNAL uvt_status uvt_handle_workspace(uvt_handle h, size_t bytes, void** 
 UVT_INTERNAL uvt_status uvt_launch_trapezoid_f64(int32_t cfg, int64_t n, int64_t m, const double* A, int64_t lda,
                                     const double* B, int64_t ldb, double* C, int64_t ldc,
                                     hipStream_t s);
+// Whether an n x n by n x m product with these leading dimensions runs in wave
+// tiles (uvt_f64_wave.hpp), and in which: 0 or the shape for
+// uvt_launch_waves_f64, 10 x its rows + its columns in units of 16.
+UVT_INTERNAL int uvt_wave_shape(int64_t n, int64_t m, int64_t lda, int64_t ldb);
+// The trapezoid walk in wave tiles, on a GPU of `cus` compute units.
+UVT_INTERNAL uvt_status uvt_launch_waves_f64(int shape, int64_t n, int64_t m, const double* A, int64_t lda,
+                                             const double* B, int64_t ldb, double* C, int64_t ldc, int cus,
+                                             hipStream_t s);
 // The same walk split stream-K (uvt_sk.hpp) over at most `workgroups`
 // workgroups (in column groups where there are at least 8 of them), then
 // its fixup launch; parts holds uvt_sk_parts_bytes(cfg, workgroups) bytes.

@@ -195,10 +195,16 @@ static uvt_status launch(uvt_server s, Slot& sl)
     if (int8) {
         e = uvt_trmm_split(s->h, n, m, s->cfg.slices, dA, n, dB, m, dC, m, work, wbytes, st);
     } else {
+        // Wave tiles for the smallest requests only (16x16 ones): beside other
+        // requests the larger ones lose more in shared loads than they gain
+        // in width (bursts of 40, orders to 1024 / 4096, 8 slots: 644 / 1726
+        // us without, 453 / 1730 with 16x16 ones, 460 / 1935 with 16x32).
+        const int shape = uvt_wave_shape(n, m, n, m), wave = shape == 11 ? shape : 0;
         const int tile = uvt_wide_tiles(s->tune.empty() ? uvt_default_cfg(n, m) : uvt_tune_pick(s->tune, n, m), n, m);
         const int64_t sk = uvt_sk_workgroups(tile, n, m, s->h->cus);
-        e = sk > 0 ? uvt_launch_trapezoid_sk_f64(tile, n, m, dA, n, dB, m, dC, m, sk, sl.parts, st)
-                   : uvt_launch_trapezoid_f64(tile, n, m, dA, n, dB, m, dC, m, st);
+        e = wave     ? uvt_launch_waves_f64(wave, n, m, dA, n, dB, m, dC, m, s->h->cus, st)
+            : sk > 0 ? uvt_launch_trapezoid_sk_f64(tile, n, m, dA, n, dB, m, dC, m, sk, sl.parts, st)
+                     : uvt_launch_trapezoid_f64(tile, n, m, dA, n, dB, m, dC, m, st);
     }
     if (e != UVT_OK) return e;
     UVT_HIP(hipEventRecord(sl.done, st));
