@@ -82,6 +82,7 @@ constexpr int kModuli[kMaxMods] = {256, 255, 253, 251, 247, 241, 239, 233,
 struct Mods {
     int n, l0, nl;
     int m[kMaxMods];
+    int c16[kMaxMods];  // 2^16 modulo m, symmetric
     double invd[kMaxMods];
     float invf[kMaxMods];
 };
@@ -130,12 +131,13 @@ struct Desc {
     double* err;              // [4]: bound, estimate (relative), ||C||_F, absolute bound
     int8_t* Ar;               // [mod][row tile t][16 blocks of a_tile_stride(t) bytes] (see k_resid_a)
     int8_t* Br;               // [mod in group][k block][column block] fragments (see k_resid_b)
-    uint8_t* R;               // [mod][n - 256][m]
+    uint32_t* R;              // [mod][row quad][m]: residues of rows 256 + 4q .. +3, a byte each
     double target;            // row / column 2-norm target before rounding
     double c_max;             // bound on |C'_ij| = |A'_i B'_j|
     int32_t nrt, nct;         // 256-row/column tiles
     int32_t nrt128, nct128;   // 128 tiles of the FP64 diagonal part
-    int32_t gxa, gxr;         // resid_a workgroups per 32-row block (128 k each), reconstruct per row
+    int32_t gxa;              // resid_a workgroups per 32-row block (128 k each)
+    int32_t gxr, rrows;       // reconstruct: 256-column blocks, rows per workgroup (a multiple of 4)
     int32_t vec;              // 16-byte FP64 loads allowed
     int32_t gr;               // row tiles per XCD group of the int8 products (x 32/gr columns)
     int32_t start[K_NUM];     // first workgroup of this problem in each stage
@@ -184,6 +186,8 @@ __host__ __device__ __forceinline__ int64_t a_tile_base(int64_t t)
 {
     return 16 * (2 * kFrag * t * (t - 1) + kFragSkew * t);
 }
+// Row quads of the product residues per modulus.
+__host__ __device__ __forceinline__ int64_t r_quads(int64_t n) { return (n - kTileI + 3) / 4; }
 // Bytes of A' residues per modulus.
 __host__ __device__ __forceinline__ int64_t a_mod_bytes(int64_t n) { return a_tile_base(pad_tile(n) / kTileI); }
 
@@ -680,7 +684,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_i8(Desc one, const Desc* table,
     const int lm = mods.l0 + l;  // the modulus
     const int8_t* Af = UVT_FIELD(Ar) + lm * a_mod_bytes(n) + a_tile_base(rt);
     const int8_t* B = UVT_FIELD(Br) + l * (pad_tile(m) * kmax) + (c0 / 16) * kFrag;
-    UVT_GLOBAL uint8_t* const Rout = gbl(UVT_FIELD(R));
+    UVT_GLOBAL uint32_t* const Rout = gbl(UVT_FIELD(R));
 #undef UVT_FIELD
 
     v4i acc[4][8];
@@ -690,30 +694,54 @@ __global__ __launch_bounds__(512, 1) void k_gemm_i8(Desc one, const Desc* table,
         for (int j = 0; j < 8; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     i8_tile_loop(Af, a_tile_stride(rt), B, pad_tile(m) / 16 * kFrag, (int)r0, smem, acc);
 
+    // The sums to residues in [0, 255] (x or x + m represent the same residue:
+    // the reconstruction takes either).  With x = 2^16 h + l, y = h c16 + l is
+    // congruent to x and below 2^22.1 in magnitude, exact in FP32; then r = y -
+    // m floor((y + 1/4) / m), the quotient in FP32 with an error below 0.0027:
+    // too small to pass an integer from 3/4 m below it (m <= 255), and when
+    // it falls short of one, r is m.  m = 256 keeps the low byte.
+    //
     // D layout of v_mfma_i32_16x16x64_i8: lane l, element v holds row
-    // 4*(l/16) + v, column l%16.
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // 4*(l/16) + v, column l%16: a lane's four values are one word of R, so a
+    // tile goes out in 32 word stores per thread.  (As bytes of rows, 128
+    // stores per thread, with a 12-instruction reduction each, the epilogue
+    // took 92 of 743 us at 5000 x 1500, 13 moduli, and 1.7 of 51.4 ms at
+    // 32768 x 8192, 12 moduli.)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int mod = mods.m[lm];
-    const float invf = mods.invf[lm];
-    UVT_GLOBAL uint8_t* out = Rout + lm * ((n - kTileI) * m);
+    const int mod = mods.m[lm], c16 = mods.c16[lm];
+    const float invf = mods.invf[lm], quarter = 0.25f * invf;
+    UVT_GLOBAL uint32_t* out = Rout + lm * (r_quads(n) * m);
+    // (every step in FP32 is exact but the quotient's product)
+    auto residue = [&](int x, uint32_t word, auto byte) {
+        const float y = (float)(__mul24(x >> 16, c16) + (x & 0xffff));
+        const float r = fmaf(-floorf(fmaf(y, invf, quarter)), (float)mod, y);
+        return __builtin_amdgcn_cvt_pk_u8_f32(r, byte(), word);
+    };
+    using std::integral_constant;
+    auto reduce = [&](v4i x) {
+        uint32_t w = residue(x.x, 0u, integral_constant<int, 0>{});
+        w = residue(x.y, w, integral_constant<int, 1>{});
+        w = residue(x.z, w, integral_constant<int, 2>{});
+        return residue(x.w, w, integral_constant<int, 3>{});
+    };
+    auto low_bytes = [](v4i x) {
+        return ((uint32_t)x.x & 255u) | ((uint32_t)x.y & 255u) << 8 | ((uint32_t)x.z & 255u) << 16 | (uint32_t)x.w << 24;
+    };
+    const int64_t left_r = n - r0 - wm * 64 - 4 * (lane >> 4), left_c = m - c0 - wn * 128 - (lane & 15);
+    UVT_GLOBAL uint32_t* o =
+        out + (((r0 - kTileI) >> 2) + wm * 16 + (lane >> 4)) * m + c0 + wn * 128 + (lane & 15);
+    auto put = [&](auto&& words) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int64_t col = c0 + wn * 128 + j * 16 + (lane & 15);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int64_t row = r0 + wm * 64 + i * 16 + 4 * (lane >> 4) + v;
-                if (row < n && col < m) {
-                    const int x = acc[i][j][v];
-                    int r = x - mod * (int)floorf((float)x * invf);
-                    if (r < 0) r += mod;
-                    if (r >= mod) r -= mod;
-                    out[(row - kTileI) * m + col] = (uint8_t)r;
-                }
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t w = words(acc[i][j]);
+                if (16 * i < left_r && 16 * j < left_c) o[i * (4 * m) + 16 * j] = w;
             }
-        }
+    };
+    if (mod == 256) put(low_bytes);
+    else put(reduce);
 }
 
 // ---- FP64 diagonal blocks ---------------------------------------------------
@@ -789,10 +817,11 @@ struct CrtTab {
 // 1e-6, and S / M is formed to about 2^-40); X_k = S_k - q M_k; a carry that
 // brings X_0 into [0, 2^40), so that X_2 2^40 + X_1 is the integer
 // floor(C' / 2^40); and C' = (X_2 2^40 + X_1) 2^40 + X_0 with two roundings
-// (fma), exact whenever C' is an FP64 number.  A workgroup takes 1024
-// columns of a row, four per thread, and adds the sum of squares of the
-// finished C values to the error statement's ||C||_F (workgroups of rows
-// 0 .. 255 only read C for it).
+// (fma), exact whenever C' is an FP64 number.  A workgroup takes 256 columns,
+// one per thread, of d.rrows rows, four rows (one word of residues per
+// modulus) at a time, and adds the sum of squares of the finished C values
+// to the error statement's ||C||_F (rows 0 .. 255 are only read for it).
+// HBM-bound: N + 16 bytes per element.
 template <int N>
 __global__ __launch_bounds__(256) void k_reconstruct(Desc one, const Desc* table, const int* lut)
 {
@@ -801,87 +830,49 @@ __global__ __launch_bounds__(256) void k_reconstruct(Desc one, const Desc* table
     __shared__ xd lds[4];
     const Desc d = fetch(one, table, lut);
     const int64_t wb = (int64_t)blockIdx.x - d.start[K_REC];
-    const int64_t i = wb / d.gxr;
-    const int64_t j4 = (wb % d.gxr) * 1024 + threadIdx.x * 4;
-    const int64_t m = d.m;
+    const int64_t i0 = wb / d.gxr * d.rrows, i1 = i0 + d.rrows < d.n ? i0 + d.rrows : d.n;
+    const int64_t j = wb % d.gxr * 256 + threadIdx.x, m = d.m;
     NormAcc acc;
-    if (i < d.n && j4 < m) {
-        const int ne = m - j4 < 4 ? (int)(m - j4) : 4;
-        UVT_GLOBAL double* crow = gbl(d.C) + i * d.ldc + j4;
-        double cv[4] = {0.0, 0.0, 0.0, 0.0};
-        if (i < kTileI) {  // no box part: C is final
+    if (j < m) {
+        const int be = gbl(d.beta)[j], bnf = gbl(d.bnf)[j];
+        for (int64_t i = i0; i < i1; i += 4) {
+            const int ne = i1 - i < 4 ? (int)(i1 - i) : 4;
+            UVT_GLOBAL double* c = gbl(d.C) + i * d.ldc + j;
+            double cv[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (e < ne) cv[e] = crow[e];
-        } else {
-            const bool vec4 = (m & 3) == 0 && ne == 4;
-            const int64_t mod_stride = (d.n - kTileI) * m;
-            uint32_t res[N][4];
+            for (int e = 0; e < 4; ++e) cv[e] = e < ne ? c[e * d.ldc] : 0.0;
+            if (i >= kTileI) {  // else no box part: C is final
+                uint32_t res[N];
+                const UVT_GLOBAL uint32_t* r = gbl(d.R) + ((i - kTileI) >> 2) * m + j;
+                const int64_t mod_stride = r_quads(d.n) * m;
 #pragma unroll
-            for (int l = 0; l < N; ++l) {
-                const UVT_GLOBAL uint8_t* r = gbl(d.R) + l * mod_stride + (i - kTileI) * m + j4;
-                if (vec4) {
-                    const uint32_t x = *reinterpret_cast<const UVT_GLOBAL uint32_t*>(r);
+                for (int l = 0; l < N; ++l) res[l] = r[l * mod_stride];
+                const int tile = (int)(i / kTileI);  // chunks c < tile feed this row's box
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) res[l][e] = (x >> (8 * e)) & 255u;
-                } else {
+                for (int e = 0; e < 4; ++e) {
+                    if (e >= ne) break;
+                    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) res[l][e] = e < ne ? r[e] : 0u;
-                }
-            }
-            const int ai = gbl(d.alpha)[i];
-            const int tile = (int)(i / kTileI);  // chunks c < tile feed this row's box
-            double xs[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-                for (int l = 0; l < N; ++l) {
-                    const double r = (double)res[l][e];
-                    s0 = fma(r, T.e[0][l], s0);
-                    s1 = fma(r, T.e[1][l], s1);
-                    s2 = fma(r, T.e[2][l], s2);
-                }
-                const double q = rint(fma(s1, inv40, fma(s0, inv80, s2)) * T.inv_mhi);
-                double x0 = fma(-q, T.mk[0], s0), x1 = fma(-q, T.mk[1], s1), x2 = fma(-q, T.mk[2], s2);
-                const double c0 = floor(x0 * inv40);
-                x0 = fma(-c0, two40, x0);
-                x1 += c0;
-                xs[e] = fma(fma(x2, two40, x1), two40, x0);
-            }
-            // C, beta and the non-finite markers in 16-byte pieces where
-            // aligned (the row start decides, the same for the whole
-            // workgroup), else element by element.
-            const UVT_GLOBAL int* brow = gbl(d.beta) + j4;
-            const UVT_GLOBAL int* frow = gbl(d.bnf) + j4;
-            if (ne == 4 && ((uintptr_t)crow & 15) == 0) {
-                const v4i b = *reinterpret_cast<const UVT_GLOBAL v4i*>(brow);
-                const v4i f = *reinterpret_cast<const UVT_GLOBAL v4i*>(frow);
-                d2 c01 = *reinterpret_cast<const UVT_GLOBAL d2*>(crow);
-                d2 c23 = *reinterpret_cast<const UVT_GLOBAL d2*>(crow + 2);
-                const bool bad = ai == kNonFinite;
-                c01.x += (bad || f.x < tile) ? nan_value() : ldexp(xs[0], -(ai + b.x));
-                c01.y += (bad || f.y < tile) ? nan_value() : ldexp(xs[1], -(ai + b.y));
-                c23.x += (bad || f.z < tile) ? nan_value() : ldexp(xs[2], -(ai + b.z));
-                c23.y += (bad || f.w < tile) ? nan_value() : ldexp(xs[3], -(ai + b.w));
-                *reinterpret_cast<UVT_GLOBAL d2*>(crow) = c01;
-                *reinterpret_cast<UVT_GLOBAL d2*>(crow + 2) = c23;
-                cv[0] = c01.x;
-                cv[1] = c01.y;
-                cv[2] = c23.x;
-                cv[3] = c23.y;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (e < ne) {
-                        const bool bad = ai == kNonFinite || frow[e] < tile;
-                        cv[e] = crow[e] + (bad ? nan_value() : ldexp(xs[e], -(ai + brow[e])));
-                        crow[e] = cv[e];
+                    for (int l = 0; l < N; ++l) {
+                        const double x = (double)((res[l] >> (8 * e)) & 255u);
+                        s0 = fma(x, T.e[0][l], s0);
+                        s1 = fma(x, T.e[1][l], s1);
+                        s2 = fma(x, T.e[2][l], s2);
                     }
+                    const double q = rint(fma(s1, inv40, fma(s0, inv80, s2)) * T.inv_mhi);
+                    double x0 = fma(-q, T.mk[0], s0), x1 = fma(-q, T.mk[1], s1), x2 = fma(-q, T.mk[2], s2);
+                    const double c0 = floor(x0 * inv40);
+                    x0 = fma(-c0, two40, x0);
+                    x1 += c0;
+                    const double x = fma(fma(x2, two40, x1), two40, x0);
+                    const int ai = gbl(d.alpha)[i + e];
+                    cv[e] += (ai == kNonFinite || bnf < tile) ? nan_value() : ldexp(x, -(ai + be));
+                    c[e * d.ldc] = cv[e];
+                }
             }
-        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc.add(cv[e]);  // zeros past the row end add nothing
+            for (int e = 0; e < 4; ++e) acc.add(cv[e]);  // zeros past the last row add nothing
+        }
     }
     const xd s = block_sum_sq(acc, lds);
     if (threadIdx.x == 0) d.cpart[wb] = s;
@@ -1010,6 +1001,8 @@ Mods make_mods(int nmod, int l0, int nl)
     md.nl = nl;
     for (int l = 0; l < nmod; ++l) {
         md.m[l] = kModuli[l];
+        const int c = 65536 % kModuli[l];
+        md.c16[l] = c > kModuli[l] / 2 ? c - kModuli[l] : c;
         md.invf[l] = 1.0f / (float)kModuli[l];
         md.invd[l] = 1.0 / (double)kModuli[l];
     }
@@ -1076,6 +1069,19 @@ int moduli_per_group(int64_t n, int64_t m, int nmod)
     return all > kBGroupBytes ? (nmod + 1) / 2 : nmod;
 }
 
+// Rows per reconstruction workgroup: four, more (up to 32) where enough
+// workgroups are left: each adds one partial sum of ||C||_F^2, which one
+// workgroup totals at the end (at one per 1024 columns of a row that took 25
+// us at 5000 x 1500 and 236 at 32768 x 8192).
+int64_t rec_cols(int64_t m) { return (m + 255) / 256; }
+int rec_rows(int64_t n, int64_t m)
+{
+    int rows = 4;
+    while (rows < 32 && (n + rows - 1) / rows * rec_cols(m) > 4096) rows *= 2;
+    return rows;
+}
+int64_t rec_blocks(int64_t n, int64_t m) { return (n + rec_rows(n, m) - 1) / rec_rows(n, m) * rec_cols(m); }
+
 // Workspace layout of one problem; every piece 256-byte aligned.
 struct Layout {
     size_t alpha, beta, bnf, rowq, part, pre, trow, tcol, cpart, err, Ar, Br, R, total;
@@ -1085,7 +1091,6 @@ Layout layout(int64_t n, int64_t m, int nmod, int per_group)
 {
     const int64_t kmax = kmax_of(n);
     const int64_t nrt = (n + kTileI - 1) / kTileI;
-    const int64_t gxr = (m + 1023) / 1024;
     Layout L;
     size_t o = 0;
     auto take = [&](size_t bytes) {
@@ -1101,11 +1106,11 @@ Layout layout(int64_t n, int64_t m, int nmod, int per_group)
     L.pre = take((size_t)nrt * m * sizeof(xd));
     L.trow = take((size_t)nrt * sizeof(TileRow));
     L.tcol = take((size_t)nrt * sizeof(TileCol));
-    L.cpart = take((size_t)n * gxr * sizeof(xd));
+    L.cpart = take((size_t)rec_blocks(n, m) * sizeof(xd));
     L.err = take(4 * sizeof(double));
     L.Ar = take(kmax > 0 ? (size_t)nmod * a_mod_bytes(n) : 0);
     L.Br = take(kmax > 0 ? (size_t)per_group * pad_tile(m) * kmax : 0);
-    L.R = take(kmax > 0 ? (size_t)nmod * (n - kTileI) * m : 0);
+    L.R = take(kmax > 0 ? (size_t)nmod * r_quads(n) * m * 4 : 0);
     L.total = o;
     return L;
 }
@@ -1147,7 +1152,8 @@ void describe(const uvt_split_problem* probs, int count, int nmod, int per_group
         d.nrt128 = (int32_t)((q.n + 127) / 128);
         d.nct128 = (int32_t)((q.m + 127) / 128);
         d.gxa = (int32_t)(d.kmax / 128);
-        d.gxr = (int32_t)((q.m + 1023) / 1024);
+        d.gxr = (int32_t)rec_cols(q.m);
+        d.rrows = rec_rows(q.n, q.m);
         d.vec = ((uintptr_t)q.A % 16 == 0) && ((uintptr_t)q.B % 16 == 0) && q.lda % 2 == 0 &&
                 q.ldb % 2 == 0;
         const Layout L = layout(q.n, q.m, nmod, per_group);
@@ -1164,7 +1170,7 @@ void describe(const uvt_split_problem* probs, int count, int nmod, int per_group
         d.err = (double*)(w + L.err);
         d.Ar = (int8_t*)(w + L.Ar);
         d.Br = (int8_t*)(w + L.Br);
-        d.R = (uint8_t*)(w + L.R);
+        d.R = (uint32_t*)(w + L.R);
         off += L.total;
         const int64_t ncb = (q.m + 255) / 256;
         d.count[K_DIAG] = d.nrt128 * d.nct128;
@@ -1173,7 +1179,7 @@ void describe(const uvt_split_problem* probs, int count, int nmod, int per_group
         d.count[K_BETA] = (int32_t)ncb;
         d.count[K_BROWS] = d.nrt;
         d.count[K_BCOLS] = d.nrt;
-        d.count[K_REC] = (int32_t)(q.n * d.gxr);
+        d.count[K_REC] = (int32_t)rec_blocks(q.n, q.m);
         d.count[K_BFIN] = 1;
         if (d.kmax > 0) {
             d.count[K_RA] = (int32_t)((pad_tile(q.n) - kTileI) / 32 * d.gxa);
