@@ -39,8 +39,9 @@ struct WaveOperand {
     const UVT_GLOBAL char* at;  // the full panel load() reads next
     uint32_t off[OFFS];         // byte offsets of this lane's loads in it
 
-    // Offsets fit 32 bits (the host takes workgroup tiles where they do not).
-    static bool fits(int64_t ld) { return ld < (int64_t)(0xFFFFFFFFu / (8u * 16 * F)) - 16; }
+    // Offsets fit 32 bits: else (rows of 128 MB or longer) there are no full
+    // panels, and the host takes workgroup tiles where it can.
+    static __host__ __device__ bool fits(int64_t ld) { return ld < (int64_t)(0xFFFFFFFFu / (8u * 16 * F)) - 16; }
 
     __device__ __forceinline__ void init(const UVT_GLOBAL double* p_, int64_t ld_, int nx_, int x0_, double* lds_)
     {
@@ -180,7 +181,7 @@ __device__ __forceinline__ void f64_wave(const TileArgs& t, const UVT_GLOBAL dou
     const int tx0 = TRI_A ? t.r0 : t.c0, tx1 = tx0 + (TRI_A ? t.rows : cols) - 1;
     const bool odd = (OA::PAIR && (t.rows & 1)) || (OB::PAIR && (cols & 1));
     const FullPanels fp = full_panels<GE>(k_lo, k_hi, tri, unit, tx0, tx1, odd);
-    const int f0 = fp.f0, f1 = fp.f1 > f0 ? fp.f1 : f0;
+    const int f0 = fp.f0, f1 = fp.f1 > f0 && OA::fits(lda) && OB::fits(ldb) ? fp.f1 : f0;
 
     OA pa;
     OB pb;
@@ -271,7 +272,7 @@ __device__ __forceinline__ void f64_wave(const TileArgs& t, const UVT_GLOBAL dou
 #pragma unroll
     for (int d = 0; d < TAIL; ++d)
         if (f1 + d < nk) multiply_masked(f1 + d, ta[d], tb[d]);
-    for (int kt = f1 + TAIL; kt < nk; ++kt) {  // a last k row kept out of the full panels
+    for (int kt = f1 + TAIL; kt < nk; ++kt) {  // a last k row kept out of the full panels, or no full panels
         load_masked(kt, ta[0], tb[0]);
         multiply_masked(kt, ta[0], tb[0]);
     }

@@ -66,6 +66,7 @@ constexpr int kI8BK = 64;    // k bytes per LDS stage (one v_mfma_i32_16x16x64_i
 constexpr int kI8Stage = kTileI * kI8BK;  // one B' stage in LDS: 16 fragments of 1 KiB
 constexpr int kFrag = 1024;       // one MFMA operand fragment: 16 rows x 64 k bytes
 constexpr int kFragSkew = 256;    // extra bytes per 16-row block of A' (see a_tile_stride)
+constexpr int kPrepLds = 32 * (128 + 4) * 8;  // LDS of the launch that builds residues
 constexpr int kNonFinite = 0x40000000;    // alpha of a row whose box part holds a NaN / infinity
 constexpr int kAllFinite = 0x7FFFFFFF;    // bnf of a column whose box rows are all finite
 // B' residues of more than this many bytes are built and multiplied in two
@@ -88,7 +89,7 @@ struct Mods {
 };
 
 // Stages, in launch order.
-enum { K_DIAG = 0, K_ALPHA, K_BPART, K_BETA, K_BROWS, K_BCOLS, K_RA, K_RB, K_GEMM, K_REC, K_BFIN, K_NUM };
+enum { K_ALPHA, K_BPART, K_BETA, K_BROWS, K_BCOLS, K_RA, K_RB, K_GEMM, K_REC, K_BFIN, K_NUM };
 static_assert(K_NUM == UVT_SPLIT_STAGES, "stage count");
 
 // Per row of A: 1-norm and sum of squares of the box part, sum of squares of
@@ -135,7 +136,6 @@ struct Desc {
     double target;            // row / column 2-norm target before rounding
     double c_max;             // bound on |C'_ij| = |A'_i B'_j|
     int32_t nrt, nct;         // 256-row/column tiles
-    int32_t nrt128, nct128;   // 128 tiles of the FP64 diagonal part
     int32_t gxa;              // resid_a workgroups per 32-row block (128 k each)
     int32_t gxr, rrows;       // reconstruct: 256-column blocks, rows per workgroup (a multiple of 4)
     int32_t vec;              // 16-byte FP64 loads allowed
@@ -157,13 +157,13 @@ __device__ __forceinline__ v4i ld_global16(const int8_t* base, uint32_t off)
 
 // The problem of this workgroup (a copy in scalar registers: every field is
 // uniform over the workgroup).
-__device__ __forceinline__ Desc fetch(const Desc& one, const Desc* table, const int* lut)
+__device__ __forceinline__ Desc fetch(const Desc& one, const Desc* table, const int* lut, int64_t block)
 {
     if (!table) return one;
     // word by word through a global pointer (global, not flat, loads)
     static_assert(sizeof(Desc) % 4 == 0, "Desc is copied in 4-byte words");
     Desc d;
-    const UVT_GLOBAL int* src = (const UVT_GLOBAL int*)gbl(&table[gbl(lut)[blockIdx.x]]);
+    const UVT_GLOBAL int* src = (const UVT_GLOBAL int*)gbl(&table[gbl(lut)[block]]);
     int* dst = reinterpret_cast<int*>(&d);
 #pragma unroll
     for (int w = 0; w < (int)(sizeof(Desc) / 4); ++w) dst[w] = src[w];
@@ -247,10 +247,10 @@ __device__ __forceinline__ int scale_exponent(double target, xd s2)
 
 // alpha_i from the 2-norm of A[i][0:kb(i)), and the row's bound terms; one
 // wave per row.
-__global__ __launch_bounds__(256) void k_alpha(Desc one, const Desc* table, const int* lut)
+__device__ __forceinline__ void do_alpha(const Desc& one, const Desc* table, const int* lut, int64_t block)
 {
-    const Desc d = fetch(one, table, lut);
-    const int64_t wb = (int64_t)blockIdx.x - d.start[K_ALPHA];
+    const Desc d = fetch(one, table, lut, block);
+    const int64_t wb = d.count[K_ALPHA] - 1 - (block - d.start[K_ALPHA]);  // the longest rows first
     const int64_t row = wb * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= d.n) return;
@@ -286,51 +286,84 @@ __global__ __launch_bounds__(256) void k_alpha(Desc one, const Desc* table, cons
 }
 
 // Per (256-row chunk, column) of B over all of B's rows: sum of squares and
-// of absolute values.
-__global__ __launch_bounds__(256) void k_beta_part(Desc one, const Desc* table, const int* lut)
+// of absolute values.  A workgroup takes 64 columns, each of its waves a
+// quarter of the chunk's rows, added up in row order (with a thread per
+// column over all 256 rows, 120 workgroups for 5000 x 1500 took 40 us).
+__device__ __forceinline__ void do_beta_part(const Desc& one, const Desc* table, const int* lut, int64_t block)
 {
-    const Desc d = fetch(one, table, lut);
-    const int64_t wb = (int64_t)blockIdx.x - d.start[K_BPART];
-    const int64_t ncb = (d.m + 255) / 256;
+    __shared__ Part quarter[4][64];
+    const Desc d = fetch(one, table, lut, block);
+    const int64_t wb = block - d.start[K_BPART];
+    const int64_t ncb = (d.m + 63) / 64;
     const int64_t chunk = wb / ncb;
-    const int64_t j = (wb % ncb) * 256 + threadIdx.x;
-    if (j >= d.m) return;
-    const int64_t k0 = chunk * 256;
-    const int64_t k1 = k0 + 256 < d.n ? k0 + 256 : d.n;
+    const int c = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t j = (wb % ncb) * 64 + c;
     NormAcc acc;
-    const UVT_GLOBAL double* b = gbl(d.B) + j;
-    int64_t k = k0;
-    for (; k + 3 < k1; k += 4) {  // four loads in flight, added in k order
-        const double v0 = b[k * d.ldb], v1 = b[(k + 1) * d.ldb], v2 = b[(k + 2) * d.ldb],
-                     v3 = b[(k + 3) * d.ldb];
-        acc.add(v0);
-        acc.add(v1);
-        acc.add(v2);
-        acc.add(v3);
+    if (j < d.m) {
+        const int64_t k0 = chunk * 256 + w * 64;
+        const int64_t k1 = k0 + 64 < d.n ? k0 + 64 : d.n;
+        const UVT_GLOBAL double* b = gbl(d.B) + j;
+        int64_t k = k0;
+        for (; k + 7 < k1; k += 8) {  // eight loads in flight, added in k order
+            double v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = b[(k + e) * d.ldb];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc.add(v[e]);
+        }
+        for (; k < k1; ++k) acc.add(b[k * d.ldb]);
     }
-    for (; k < k1; ++k) acc.add(b[k * d.ldb]);
-    const xd s2 = acc.sum_sq(), s1 = acc.sum_abs();
-    d.part[chunk * d.m + j] = Part{s2.f, acc.nonfinite ? nan_value() : s1.f, s2.e, s1.e};
+    xd s2 = acc.sum_sq(), s1 = acc.sum_abs();
+    quarter[w][c] = Part{s2.f, acc.nonfinite ? nan_value() : s1.f, s2.e, s1.e};
+    __syncthreads();
+    if (w != 0 || j >= d.m) return;
+    bool nf = acc.nonfinite;
+    for (int q = 1; q < 4; ++q) {
+        const Part p = quarter[q][c];
+        s2 = xd_add(s2, xd{p.sf, p.se});
+        if (p.af != p.af) nf = true;
+        else s1 = xd_add(s1, xd{p.af, p.ae});
+    }
+    d.part[chunk * d.m + j] = Part{s2.f, nf ? nan_value() : s1.f, s2.e, s1.e};
+}
+
+// The norms of A's rows and of B's chunks in one launch: na workgroups of
+// the first, the rest of the second.
+__global__ __launch_bounds__(256) void k_norms(Desc one, const Desc* table, const int* lut_a, const int* lut_b,
+                                               int64_t na)
+{
+    if ((int64_t)blockIdx.x < na) do_alpha(one, table, lut_a, blockIdx.x);
+    else do_beta_part(one, table, lut_b, blockIdx.x - na);
 }
 
 // beta_j from the 2-norm of B[0:kmax][j]; the column's first non-finite
 // chunk; and the prefix 1-norms pre[t][j] = sum_{c < t} |B[chunk c][j]|_1.
-__global__ __launch_bounds__(256) void k_beta(Desc one, const Desc* table, const int* lut)
+__global__ __launch_bounds__(64) void k_beta(Desc one, const Desc* table, const int* lut)
 {
-    const Desc d = fetch(one, table, lut);
+    const Desc d = fetch(one, table, lut, blockIdx.x);
     const int64_t wb = (int64_t)blockIdx.x - d.start[K_BETA];
-    const int64_t j = wb * 256 + threadIdx.x;
+    const int64_t j = wb * 64 + threadIdx.x;
     if (j >= d.m) return;
     const Part* part = d.part + j;  // small structs: generic (flat) accesses
     xd s2{0.0, 0};
     xd pre{0.0, 0};
     int nf = kAllFinite;
-    for (int t = 1; t < d.nrt; ++t) {  // chunk c = t - 1 < kmax / 256
-        const Part p = part[(int64_t)(t - 1) * d.m];
-        s2 = xd_add(s2, xd{p.sf, p.se});
-        if (p.af != p.af) nf = nf == kAllFinite ? t - 1 : nf;
-        else pre = xd_add(pre, xd{p.af, p.ae});
-        d.pre[(int64_t)t * d.m + j] = pre;
+    for (int t0 = 1; t0 < d.nrt; t0 += 8) {  // chunks c = t - 1 < kmax / 256, eight loads in flight
+        Part p[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int t = t0 + e < d.nrt ? t0 + e : d.nrt - 1;
+            p[e] = part[(int64_t)(t - 1) * d.m];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int t = t0 + e;
+            if (t >= d.nrt) break;
+            s2 = xd_add(s2, xd{p[e].sf, p[e].se});
+            if (p[e].af != p[e].af) nf = nf == kAllFinite ? t - 1 : nf;
+            else pre = xd_add(pre, xd{p[e].af, p[e].ae});
+            d.pre[(int64_t)t * d.m + j] = pre;
+        }
     }
     gbl(d.beta)[j] = s2.f > 0.0 ? scale_exponent(d.target, s2) : 0;
     gbl(d.bnf)[j] = nf;
@@ -340,12 +373,13 @@ __global__ __launch_bounds__(256) void k_beta(Desc one, const Desc* table, const
 // per row): with v_i = |A_box,i|_1 / 2 + kb_i 2^-alpha_i / 4,
 //   ru2 = sum v_i^2, ru1 = sum 2^-alpha_i v_i, rw = sum 4^-alpha_i,
 //   ra2 = sum |A_box,i|^2 (tiles t >= 1), rd2 = sum |A_diag,i|^2 (all tiles).
-__global__ __launch_bounds__(256) void k_bound_rows(Desc one, const Desc* table, const int* lut)
+__device__ __forceinline__ void do_bound_rows(const Desc& one, const Desc* table, const int* lut, int64_t block,
+                                             char* smem)
 {
-    __shared__ xd lds[4];
-    __shared__ int flag;
-    const Desc d = fetch(one, table, lut);
-    const int t = (int)((int64_t)blockIdx.x - d.start[K_BROWS]);
+    xd* lds = reinterpret_cast<xd*>(smem);
+    int& flag = *reinterpret_cast<int*>(smem + 4 * sizeof(xd));
+    const Desc d = fetch(one, table, lut, block);
+    const int t = (int)(block - d.start[K_BROWS]);
     const int64_t i = (int64_t)t * kTileI + threadIdx.x;
     xd ru2{0.0, 0}, ru1{0.0, 0}, rw{0.0, 0}, ra2{0.0, 0}, rd2{0.0, 0};
     int nf = 0;
@@ -380,12 +414,13 @@ __global__ __launch_bounds__(256) void k_bound_rows(Desc one, const Desc* table,
 // Column side, one workgroup per 256-row tile t (threads over columns):
 //   cq1 = sum_j 2^-beta_j pre[t][j], cq2 = sum_j pre[t][j]^2 (t >= 1),
 //   cb = |B[chunk t]|_F^2, and for t = 0 cv = sum_j 4^-beta_j.
-__global__ __launch_bounds__(256) void k_bound_cols(Desc one, const Desc* table, const int* lut)
+__device__ __forceinline__ void do_bound_cols(const Desc& one, const Desc* table, const int* lut, int64_t block,
+                                             char* smem)
 {
-    __shared__ xd lds[4];
-    __shared__ int flag;
-    const Desc d = fetch(one, table, lut);
-    const int t = (int)((int64_t)blockIdx.x - d.start[K_BCOLS]);
+    xd* lds = reinterpret_cast<xd*>(smem);
+    int& flag = *reinterpret_cast<int*>(smem + 4 * sizeof(xd));
+    const Desc d = fetch(one, table, lut, block);
+    const int t = (int)(block - d.start[K_BCOLS]);
     xd cq1{0.0, 0}, cq2{0.0, 0}, cb{0.0, 0}, cv{0.0, 0};
     int nf = 0;
     for (int64_t j = threadIdx.x; j < d.m; j += 256) {
@@ -434,11 +469,13 @@ __device__ __forceinline__ int sym_residue(double a, int m, double invm)
 // on 128 contiguous bytes (16 per lane), then taken back as 16 consecutive k
 // per thread (row t/8), so a wave writes 8 whole 128-byte lines per modulus.
 // Rows n .. pad_tile(n) are zeros, and so are rows with a non-finite entry.
-__global__ __launch_bounds__(256) void k_resid_a(Desc one, const Desc* table, const int* lut, Mods mods)
+__device__ __forceinline__ void do_resid_a(const Desc& one, const Desc* table, const int* lut, int64_t block,
+                                           const Mods& mods, char* smem)
 {
-    __shared__ __attribute__((aligned(16))) double tv[32][128 + 4];
-    const Desc d = fetch(one, table, lut);
-    const int64_t wb = (int64_t)blockIdx.x - d.start[K_RA];
+    double(*tv)[128 + 4] = reinterpret_cast<double(*)[128 + 4]>(smem);
+    static_assert(sizeof(double[32][128 + 4]) <= kPrepLds, "LDS of the residue launch");
+    const Desc d = fetch(one, table, lut, block);
+    const int64_t wb = block - d.start[K_RA];
     const int64_t rb = kTileI / 32 + wb / d.gxa, kq = wb % d.gxa;
     if (kq * 128 >= row_box_end(rb * 32)) return;  // boxes end on multiples of 256
     const int t = threadIdx.x, c = t & 7, r = t >> 3;
@@ -501,13 +538,15 @@ __global__ __launch_bounds__(256) void k_resid_a(Desc one, const Desc* table, co
 // w/2 + 2), one lane's 16 bytes each.  Two LDS buffers, so one barrier per
 // modulus.  Columns m .. pad_tile(m) are zeros, and so are non-finite
 // entries.
-__global__ __launch_bounds__(256) void k_resid_b(Desc one, const Desc* table, const int* lut, Mods mods)
+__device__ __forceinline__ void do_resid_b(const Desc& one, const Desc* table, const int* lut, int64_t block,
+                                           const Mods& mods, char* smem)
 {
     constexpr int kW = 32;          // 4-byte words per column of the tile (128 k)
     constexpr int kPitch = 64 + 4;  // 4 * kPitch = 16 (mod 32) banks: the readback's lanes hit distinct banks
-    __shared__ uint32_t t[2][kW][kPitch];  // [buffer][k word][column]
-    const Desc d = fetch(one, table, lut);
-    const int64_t wb = (int64_t)blockIdx.x - d.start[K_RB];
+    uint32_t(*t)[kW][kPitch] = reinterpret_cast<uint32_t(*)[kW][kPitch]>(smem);  // [buffer][k word][column]
+    static_assert(sizeof(uint32_t[2][kW][kPitch]) <= kPrepLds, "LDS of the residue launch");
+    const Desc d = fetch(one, table, lut, block);
+    const int64_t wb = block - d.start[K_RB];
     const int64_t nkx = d.kmax / 128;  // kmax is a multiple of 256
     const int64_t k0 = (wb % nkx) * 128, j0 = (wb / nkx) * 64;
     const int jj = threadIdx.x & 63, kq = threadIdx.x >> 6;
@@ -552,6 +591,29 @@ __global__ __launch_bounds__(256) void k_resid_b(Desc one, const Desc* table, co
             *reinterpret_cast<UVT_GLOBAL v4i*>(gbl(d.Br) + l * mod_stride + frag * kFrag + lane * 16) = x;
         }
     }
+}
+
+// What follows the scales, in one launch: the bound terms, whose few
+// workgroups would otherwise be the last to finish, then A' and B' residues
+// (workgroups up to and including each part; the residues of B have a launch
+// of their own where they are built in groups of moduli).
+struct PrepBlocks {
+    int64_t rows, cols, a;
+};
+__global__ __launch_bounds__(256) void k_residues(Desc one, const Desc* table, const int* lut_a, const int* lut_b,
+                                                  const int* lut_rows, const int* lut_cols, PrepBlocks nb, Mods mods)
+{
+    __shared__ __attribute__((aligned(16))) char smem[kPrepLds];
+    const int64_t b = blockIdx.x;
+    if (b < nb.rows) do_bound_rows(one, table, lut_rows, b, smem);
+    else if (b < nb.cols) do_bound_cols(one, table, lut_cols, b - nb.rows, smem);
+    else if (b < nb.a) do_resid_a(one, table, lut_a, b - nb.cols, mods, smem);
+    else do_resid_b(one, table, lut_b, b - nb.a, mods, smem);
+}
+__global__ __launch_bounds__(256) void k_resid_b(Desc one, const Desc* table, const int* lut, Mods mods)
+{
+    __shared__ __attribute__((aligned(16))) char smem[kPrepLds];
+    do_resid_b(one, table, lut, blockIdx.x, mods, smem);
 }
 
 // ---- int8 modular products ---------------------------------------------------
@@ -746,27 +808,25 @@ __global__ __launch_bounds__(512, 1) void k_gemm_i8(Desc one, const Desc* table,
 
 // ---- FP64 diagonal blocks ---------------------------------------------------
 
-// Rows [r0, r0+128) of C = A[rows, t0:row] * B[t0:row] where t0 is the start of
-// the 256-row tile holding r0 (lower mask), written (not accumulated).
-__global__ __launch_bounds__(512, 4) void k_diag_f64(Desc one, const Desc* table, const int* lut)
+// C = A[rows, t0:row] * B[t0:row] (lower mask), written (not accumulated),
+// where t0 is the start of the 256-row tile holding a row; one T x T tile of
+// at most 16 panels per workgroup (one problem, launched by itself).  64x64
+// tiles keep more of a short product in flight (us of a whole call, 128x128 /
+// 64x64: 3000 x 1000 221 / 216, 5000 x 1500 587 / 582, 8192 x 4096 2198 /
+// 2179), 128x128 ones read less (32768 x 8192 50.6 / 50.8 ms); in wave tiles
+// the same blocks took 83 us against 72 at 5000 x 1500.
+template <int T>
+__global__ __launch_bounds__((64 * TileWaves<T, T>::M * TileWaves<T, T>::N), 4) void k_diag_f64(Desc one)
 {
-    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES];
-    const Desc* dp = table ? &table[lut[blockIdx.x]] : nullptr;
-#define UVT_FIELD(f) (dp ? dp->f : one.f)
-    const int64_t wb = (int64_t)blockIdx.x - UVT_FIELD(start[K_DIAG]);
-    const int nct128 = UVT_FIELD(nct128);
-    const int64_t n = UVT_FIELD(n);
-    const int rt = (int)(wb / nct128), ct = (int)(wb % nct128);
-    const int r0 = rt * 128, c0 = ct * 128;
-    const int rows = (int)(n - r0 < 128 ? n - r0 : 128);
-    const int k_lo = (r0 / kTileI) * kTileI;
-    const UVT_GLOBAL double* A = gbl(UVT_FIELD(A));
-    const UVT_GLOBAL double* B = gbl(UVT_FIELD(B));
-    UVT_GLOBAL double* C = gbl(UVT_FIELD(C));
-    f64_tile<128, 128, 4, 2>(TileArgs{r0, rows, c0, k_lo, r0 + rows, kTileLower}, A, UVT_FIELD(lda), B,
-                             UVT_FIELD(ldb), C, UVT_FIELD(ldc), UVT_FIELD(m), smem);
-#undef UVT_FIELD
+    using W = TileWaves<T, T>;
+    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<T, T, W::M, W::N>::SMEM_DOUBLES];
+    const int64_t nct = (one.m + T - 1) / T;
+    const int r0 = (int)(blockIdx.x / nct) * T, c0 = (int)(blockIdx.x % nct) * T;
+    const int rows = (int)(one.n - r0 < T ? one.n - r0 : T);
+    f64_tile<T, T, W::M, W::N>(TileArgs{r0, rows, c0, (r0 / kTileI) * kTileI, r0 + rows, kTileLower}, gbl(one.A),
+                               one.lda, gbl(one.B), one.ldb, gbl(one.C), one.ldc, one.m, smem);
 }
+constexpr int64_t kDiagLarge = 8192;  // 128x128 tiles from this many of them on
 
 // ---- reconstruction -----------------------------------------------------------
 
@@ -828,7 +888,7 @@ __global__ __launch_bounds__(256) void k_reconstruct(Desc one, const Desc* table
     constexpr CrtTab<N> T{};
     constexpr double two40 = 1099511627776.0, inv40 = 1.0 / two40, inv80 = inv40 * inv40;
     __shared__ xd lds[4];
-    const Desc d = fetch(one, table, lut);
+    const Desc d = fetch(one, table, lut, blockIdx.x);
     const int64_t wb = (int64_t)blockIdx.x - d.start[K_REC];
     const int64_t i0 = wb / d.gxr * d.rrows, i1 = i0 + d.rrows < d.n ? i0 + d.rrows : d.n;
     const int64_t j = wb % d.gxr * 256 + threadIdx.x, m = d.m;
@@ -917,9 +977,9 @@ void launch_reconstruct(unsigned grid, hipStream_t s, const Desc& one, const Des
 // the worst-case signs).
 __global__ __launch_bounds__(1024) void k_bound_final(Desc one, const Desc* table, const int* lut)
 {
-    __shared__ xd lds[16];
-    __shared__ int flag;
-    const Desc d = fetch(one, table, lut);
+    __shared__ xd lds[6][16];
+    __shared__ int bad[16];
+    const Desc d = fetch(one, table, lut, blockIdx.x);
     int nf = 0;
     // ||C||^2 from the reconstruction's partial sums: eight independent
     // loads in flight per thread
@@ -950,13 +1010,28 @@ __global__ __launch_bounds__(1024) void k_bound_final(Desc one, const Desc* tabl
         if (t < d.nrt - 1) cn = xd_add(cn, c.cb);
         ds = xd_add(ds, xd_mul(r.rd2, c.cb));
     }
-    c2 = block_sum(c2, lds);
-    e2 = block_sum(e2, lds);
-    ra2 = block_sum(ra2, lds);
-    rw = block_sum(rw, lds);
-    cn = block_sum(cn, lds);
-    ds = block_sum(ds, lds);
-    nf = block_or(nf, &flag);
+    // the six totals together: wave sums side by side, then one barrier
+    xd* const sums[6] = {&c2, &e2, &ra2, &rw, &cn, &ds};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < 6; ++q) *sums[q] = xd_add(*sums[q], xd_shfl_xor(*sums[q], off));
+    nf = __any(nf);
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) lds[q][threadIdx.x >> 6] = *sums[q];
+        bad[threadIdx.x >> 6] = nf;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int w = threadIdx.x & 15;
+    nf = __any(bad[w]);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) *sums[q] = lds[q][w];
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < 6; ++q) *sums[q] = xd_add(*sums[q], xd_shfl_xor(*sums[q], off));
     if (threadIdx.x != 0) return;
     const double u = 0x1p-53;
     const double g257 = 257.0 * u / (1.0 - 257.0 * u);
@@ -1149,8 +1224,6 @@ void describe(const uvt_split_problem* probs, int count, int nmod, int per_group
         d.c_max = exp2(2.0 * lt) * (1.0 + 1e-6);
         d.nrt = (int32_t)((q.n + kTileI - 1) / kTileI);
         d.nct = (int32_t)((q.m + kTileI - 1) / kTileI);
-        d.nrt128 = (int32_t)((q.n + 127) / 128);
-        d.nct128 = (int32_t)((q.m + 127) / 128);
         d.gxa = (int32_t)(d.kmax / 128);
         d.gxr = (int32_t)rec_cols(q.m);
         d.rrows = rec_rows(q.n, q.m);
@@ -1172,8 +1245,7 @@ void describe(const uvt_split_problem* probs, int count, int nmod, int per_group
         d.Br = (int8_t*)(w + L.Br);
         d.R = (uint32_t*)(w + L.R);
         off += L.total;
-        const int64_t ncb = (q.m + 255) / 256;
-        d.count[K_DIAG] = d.nrt128 * d.nct128;
+        const int64_t ncb = (q.m + 63) / 64;
         d.count[K_ALPHA] = (int32_t)((q.n + 3) / 4);
         d.count[K_BPART] = (int32_t)(ncb * d.nrt);
         d.count[K_BETA] = (int32_t)ncb;
@@ -1229,6 +1301,9 @@ uvt_status uvt_split_batch_sizes(const uvt_split_problem* probs, int count, int 
         if (tot[k] > 0x7FFFFFFF) return UVT_ERR_SIZE;
         lut += tot[k];
     }
+    // the stages that share a launch
+    if (tot[K_ALPHA] + tot[K_BPART] > 0x7FFFFFFF || tot[K_RA] + tot[K_RB] + tot[K_BROWS] + tot[K_BCOLS] > 0x7FFFFFFF)
+        return UVT_ERR_SIZE;
     *work_bytes = w;
     *lut_entries = lut;
     return UVT_OK;
@@ -1281,16 +1356,32 @@ uvt_status uvt_split_batch_launch(const uvt_split_problem* single, int count, in
             hipLaunchKernelGGL(kernel, dim3((unsigned)totals[k]), dim3(256), 0, s, one, table, lut(k), args...);
     };
     // The FP64 diagonal part stores every row of C first; the box part adds to it.
-    if ((stages & UVT_SPLIT_DIAG) && totals[K_DIAG])
-        hipLaunchKernelGGL(k_diag_f64, dim3((unsigned)totals[K_DIAG]), dim3(512), 0, s, one, table, lut(K_DIAG));
+    if (stages & UVT_SPLIT_DIAG) {
+        if (table) return UVT_ERR_ARG;  // a batch's diagonal blocks run in its FP64 queue
+        const int64_t tiles = ((one.n + 127) / 128) * ((one.m + 127) / 128);
+        if (tiles >= kDiagLarge) {
+            if (tiles > 0x7FFFFFFF) return UVT_ERR_SIZE;
+            hipLaunchKernelGGL(k_diag_f64<128>, dim3((unsigned)tiles), dim3(512), 0, s, one);
+        } else {
+            const int64_t small = ((one.n + 63) / 64) * ((one.m + 63) / 64);
+            hipLaunchKernelGGL(k_diag_f64<64>, dim3((unsigned)small), dim3(256), 0, s, one);
+        }
+    }
     if (stages & UVT_SPLIT_PREP) {
-        launch(k_alpha, K_ALPHA);
-        launch(k_beta_part, K_BPART);
-        launch(k_beta, K_BETA);
-        launch(k_bound_rows, K_BROWS);
-        launch(k_bound_cols, K_BCOLS);
-        launch(k_resid_a, K_RA, mods);
-        if (per_group == nmod) launch(k_resid_b, K_RB, mods);
+        const dim3 norms((unsigned)(totals[K_ALPHA] + totals[K_BPART]));
+        if (norms.x)
+            hipLaunchKernelGGL(k_norms, norms, dim3(256), 0, s, one, table, lut(K_ALPHA), lut(K_BPART),
+                               totals[K_ALPHA]);
+        if (totals[K_BETA])
+            hipLaunchKernelGGL(k_beta, dim3((unsigned)totals[K_BETA]), dim3(64), 0, s, one, table, lut(K_BETA));
+        PrepBlocks nb;
+        nb.rows = totals[K_BROWS];
+        nb.cols = nb.rows + totals[K_BCOLS];
+        nb.a = nb.cols + totals[K_RA];
+        const dim3 prep((unsigned)(nb.a + (per_group == nmod ? totals[K_RB] : 0)));
+        if (prep.x)
+            hipLaunchKernelGGL(k_residues, prep, dim3(256), 0, s, one, table, lut(K_RA), lut(K_RB), lut(K_BROWS),
+                               lut(K_BCOLS), nb, mods);
     }
     if (stages & UVT_SPLIT_GEMM) {
         for (int l0 = 0; l0 < nmod; l0 += per_group) {

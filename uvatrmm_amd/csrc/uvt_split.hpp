@@ -22,7 +22,7 @@ struct uvt_split_problem {
 
 // Kernel stages of the split path (per-stage workgroup counts and lookup
 // tables are arrays of this length).
-constexpr int UVT_SPLIT_STAGES = 11;
+constexpr int UVT_SPLIT_STAGES = 10;
 
 // Whether an n x n triangle can run on the int8 path with nmod moduli: the
 // int32 accumulation bound (n <= 131072) and at least 6 bits left per scaled
@@ -46,7 +46,7 @@ UVT_INTERNAL uvt_status uvt_split_batch_build(const uvt_split_problem* probs, in
 // Stage groups.  The diagonal blocks store C; the reconstruction adds to C,
 // so it must run after them.
 enum {
-    UVT_SPLIT_DIAG = 1,  // FP64 diagonal blocks
+    UVT_SPLIT_DIAG = 1,  // FP64 diagonal blocks (of a single problem)
     UVT_SPLIT_PREP = 2,  // scales, residues, error-bound terms of A and B
     UVT_SPLIT_GEMM = 4,  // int8 residue products
     UVT_SPLIT_REC = 8,   // reconstruction and the error statement
