@@ -1,6 +1,6 @@
 """uvt_dgemm and uvt_dtrmm on the MI355X in every tile shape: each transpose,
-side, triangle and diagonal at sizes that pick 32x128, 128x32, 64x64, 128x128
-and 256x128 tiles with ragged edges, odd leading dimensions, and NaN in
+side, triangle and diagonal at sizes that pick wave tiles and 32x128, 128x32,
+64x64, 128x128 and 256x128 workgroup tiles with ragged edges, odd leading dimensions, and NaN in
 everything that is not an operand.  Small-integer inputs and power-of-two
 factors make every sum exact, so results equal NumPy's bit for bit."""
 import ctypes as c
@@ -32,7 +32,9 @@ def padded(x, pad, fill=np.nan):
 FORMS = list(itertools.product((0, 1), (0, 1), (0, 1), (0, 1)))  # side, uplo, trans, diag
 BIG = [(0, 0, 0, 0), (0, 1, 0, 1), (0, 0, 1, 1), (0, 1, 1, 0), (1, 0, 0, 1), (1, 1, 1, 1), (1, 0, 1, 0), (1, 1, 0, 0)]
 CASES = [(f, s) for f in FORMS for s in ((1, 1), (40, 301), (301, 40), (257, 131), (700, 633))] + \
-        [(f, (2900, 2951)) for f in BIG] + [(f, (4096, 4096)) for f in ((0, 1, 0, 0), (1, 1, 1, 1))]
+        [(f, (1901, 1802)) for f in BIG] + [(f, (2900, 2951)) for f in BIG] + \
+        [((0, 0, 1, 0), (12300, 41)), ((1, 1, 0, 1), (41, 12300))] + \
+        [(f, s) for f in BIG for s in ((1200, 1207), (1601, 1500))] + [(f, (4096, 4096)) for f in ((0, 1, 0, 0), (1, 1, 1, 1))]
 
 
 @pytest.mark.parametrize("form,size", CASES)
@@ -65,7 +67,7 @@ def test_dtrmm_exact(L, gpu, form, size):
 
 @pytest.mark.parametrize("ta,tb", list(itertools.product((0, 1), (0, 1))))
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (40, 301, 65), (301, 40, 33), (257, 131, 70), (700, 633, 1),
-                                   (2950, 2951, 129)])
+                                   (513, 1031, 259), (1500, 1601, 200), (40001, 43, 35), (2950, 2951, 129)])
 def test_dgemm_exact(L, gpu, m, n, k, ta, tb):
     rng = np.random.default_rng(m + 3 * n + 5 * k)
     A = rng.integers(-3, 4, (k, m) if ta else (m, k)).astype(np.float64)

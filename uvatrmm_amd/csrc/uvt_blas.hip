@@ -25,6 +25,7 @@
 #include <mutex>
 
 #include "uvt_f64_tile.hpp"
+#include "uvt_f64_wave.hpp"
 #include "uvt_internal.h"
 #include "uvt_runtime.hpp"
 
@@ -101,13 +102,78 @@ void launch_walk(Walk g, const double* A, int64_t lda, const double* B, int64_t 
     hipLaunchKernelGGL((k_blas_f64<TM, TN, A_KC, B_KC, TRI>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc, epi);
 }
 
+// The same walk in wave tiles, four to a workgroup, wn of them along the
+// columns; every second run of `snake` workgroups is turned round, as the
+// trapezoid walk's (uvt_api.hip).
+template <int FM, int FN, int D, bool A_KC, bool B_KC, int TRI>
+__global__ __launch_bounds__(256) void k_blas_waves_f64(Walk g, int wn, int snake, const double* __restrict__ A,
+                                                        int64_t lda, const double* __restrict__ B, int64_t ldb,
+                                                        double* __restrict__ C, int64_t ldc, TileEpi epi)
+{
+    constexpr bool kNone = TRI == kTriNone, kRight = TRI == kTriBLe || TRI == kTriBGe;
+    using Opt = TileOpt<A_KC, B_KC, kNone ? kTriALe : (TriKind)TRI, !kNone, true>;
+    __shared__ __attribute__((aligned(16))) double lds[4][wave_lds<FM, FN, Opt>() + 2];
+    int b = (int)blockIdx.x;
+    const int q = b / snake;
+    if (q & 1) b = q * snake + min((q + 1) * snake, (int)gridDim.x) - 1 - b;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int rt = kRight ? b % g.nrt : b / g.nct, ct = kRight ? b / g.nrt : b % g.nct;
+    if (TRI == kTriALe) rt = g.nrt - 1 - rt;
+    if (TRI == kTriBLe) ct = g.nct - 1 - ct;
+    const int64_t r0 = ((int64_t)rt * (4 / wn) + wave / wn) * (16 * FM), c0 = ((int64_t)ct * wn + wave % wn) * (16 * FN);
+    if (r0 >= g.M || c0 >= g.N) return;
+    const int rows = (int)(g.M - r0 < 16 * FM ? g.M - r0 : 16 * FM), cols = (int)(g.N - c0 < 16 * FN ? g.N - c0 : 16 * FN);
+    const int k_lo = (int)(TRI == kTriAGe ? r0 : TRI == kTriBGe ? c0 : 0);
+    const int k_hi = (int)(TRI == kTriALe ? r0 + rows : TRI == kTriBLe ? c0 + cols : g.K);
+    f64_wave<FM, FN, D, Opt>(TileArgs{(int)r0, rows, (int)c0, k_lo, k_hi, kNone ? 0 : kTileLower}, gbl(A), lda, gbl(B),
+                             ldb, gbl(C), ldc, g.N, lds[wave], epi);
+}
+
+template <int FM, int FN, int D, bool A_KC, bool B_KC, int TRI>
+void launch_walk_waves(Walk g, const double* A, int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc,
+                       const TileEpi& epi, int cus, hipStream_t s)
+{
+    const int64_t rt = (g.M + 16 * FM - 1) / (16 * FM), ct = (g.N + 16 * FN - 1) / (16 * FN);
+    const int wn = ct > 1 ? (rt > 1 ? 2 : 4) : 1, wm = 4 / wn;
+    g.nrt = (int)((rt + wm - 1) / wm);
+    g.nct = (int)((ct + wn - 1) / wn);
+    hipLaunchKernelGGL((k_blas_waves_f64<FM, FN, D, A_KC, B_KC, TRI>), dim3((unsigned)((int64_t)g.nrt * g.nct)),
+                       dim3(256), 0, s, g, wn, cus, A, lda, B, ldb, C, ldc, epi);
+}
+
+// Which dgemm walks run in wave tiles, and in which (as uvt_wave_shape): all
+// reductions are equally deep, so a second round of waves doubles the time,
+// and each shape stops where the GPU holds no more of them (a wave per SIMD
+// for 16x16 tiles, three for 16x32).  us, workgroup tiles / 16x16 / 16x32:
+//     257 x 257 x 257      13.9 /  6.4 /  8.5   (289 tiles of 16x16)
+//     512 x 512 x 512      22.9 /  9.5 / 12.2   (1024)
+//     600 x 600 x 6000    233   / 164  / 107    (1444)
+//    1024 x 1024 x 1024    43.6 / 50.6 / 39.1   (4096)
+//    3000 x 500 x 800      57.1 / 62.7 / 48.4   (6016)
+//    1300 x 1300 x 3000   205   / 345  / 289    (6724)
+int gemm_wave_shape(int64_t M, int64_t N)
+{
+    const int64_t tiles = ((M + 15) / 16) * ((N + 15) / 16);
+    return tiles <= 1024 ? 11 : tiles <= 6144 ? 12 : 0;
+}
+
 // The tile shape for the walk: cfg as uvt_default_cfg / uvt_wide_tiles name
 // it; on the right side 32 x 128 stands for 128 x 32 (B has few rows).
 template <bool A_KC, bool B_KC, int TRI>
 uvt_status launch_blas(int32_t cfg, const Walk& g, const double* A, int64_t lda, const double* B, int64_t ldb,
-                       double* C, int64_t ldc, const TileEpi& epi, hipStream_t s)
+                       double* C, int64_t ldc, const TileEpi& epi, int cus, hipStream_t s)
 {
     constexpr bool kRight = TRI == kTriBLe || TRI == kTriBGe;
+    const int wave = TRI == kTriNone ? gemm_wave_shape(g.M, g.N)
+                     : kRight        ? uvt_wave_shape(g.K, g.M, ldb, lda)
+                                     : uvt_wave_shape(g.K, g.N, lda, ldb);
+    if (wave) {
+        if (wave == 11) launch_walk_waves<1, 1, 4, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, cus, s);
+        else if (wave == 12) launch_walk_waves<1, 2, 4, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, cus, s);
+        else launch_walk_waves<2, 2, 2, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, cus, s);
+        UVT_HIP(hipGetLastError());
+        return UVT_OK;
+    }
     const int64_t tm = kRight && cfg == UVT_CFG_128x32 ? 32 : uvt_cfg_tile_m(cfg);
     const int64_t tn = kRight && cfg == UVT_CFG_128x32 ? 128 : uvt_cfg_tile_n(cfg);
     if (((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
@@ -164,10 +230,10 @@ extern "C" uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_
     epi.alpha = alpha;
     epi.beta = beta;
     const int32_t cfg = uvt_default_cfg(m, n);
-    if (tA && tB) return launch_blas<false, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
-    if (tA) return launch_blas<false, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
-    if (tB) return launch_blas<true, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
-    return launch_blas<true, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, s);
+    if (tA && tB) return launch_blas<false, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
+    if (tA) return launch_blas<false, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
+    if (tB) return launch_blas<true, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
+    return launch_blas<true, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
 }
 
 // ---- dtrmm ---------------------------------------------------------------------
@@ -232,7 +298,7 @@ uvt_status dtrmm_prepare(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans t
 
 // Enqueues the call on stream s with its workspace at wv.
 uvt_status dtrmm_launch(const DtrmmCall& c, int64_t m, int64_t n, double alpha, const double* dA,
-                        int64_t lda, double* dB, int64_t ldb, void* wv, hipStream_t s)
+                        int64_t lda, double* dB, int64_t ldb, void* wv, int cus, hipStream_t s)
 {
     if (alpha == 0.0) {  // B = 0, A not read
         scale(m, n, 0.0, dB, ldb, s);
@@ -249,20 +315,20 @@ uvt_status dtrmm_launch(const DtrmmCall& c, int64_t m, int64_t n, double alpha, 
     if (!c.right) {
         const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(m, n), m, n);
         if (c.lower) {
-            if (c.tA) return launch_blas<false, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
-            return launch_blas<true, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
+            if (c.tA) return launch_blas<false, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
+            return launch_blas<true, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
         }
-        if (c.tA) return launch_blas<false, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
-        return launch_blas<true, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, s);
+        if (c.tA) return launch_blas<false, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
+        return launch_blas<true, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
     }
     // B op(A): column j of the product needs k >= j where op(A) is lower
     const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(n, m), m, n);
     if (c.lower) {
-        if (c.tA) return launch_blas<true, true, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
-        return launch_blas<true, false, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
+        if (c.tA) return launch_blas<true, true, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
+        return launch_blas<true, false, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
     }
-    if (c.tA) return launch_blas<true, true, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
-    return launch_blas<true, false, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, s);
+    if (c.tA) return launch_blas<true, true, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
+    return launch_blas<true, false, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
 }
 
 }  // namespace
@@ -299,7 +365,7 @@ extern "C" uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_
         st = uvt_handle_workspace(h, c.bytes, &wv);
         if (st != UVT_OK) return st;
     }
-    return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, wv, (hipStream_t)stream);
+    return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, wv, h->cus, (hipStream_t)stream);
 }
 
 extern "C" uvt_status uvt_dtrmm_noalloc(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans ta,
@@ -314,5 +380,5 @@ extern "C" uvt_status uvt_dtrmm_noalloc(uvt_handle h, uvt_side side, uvt_uplo up
     if (c.declared > kNoAllocScratchBytes) return UVT_ERR_SIZE;
     if (!h->scratch) return UVT_ERR_STATE;
     UVT_HIP(hipSetDevice(h->device));
-    return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, h->scratch, (hipStream_t)stream);
+    return dtrmm_launch(c, m, n, alpha, dA, lda, dB, ldb, h->scratch, h->cus, (hipStream_t)stream);
 }
