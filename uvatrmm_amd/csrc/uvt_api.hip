@@ -60,21 +60,33 @@ void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__
     }
 }
 
-// Adds the partial tiles of each record to C in the record's order (one
-// workgroup per record; records cover disjoint parts of C), so the result
-// does not depend on which workgroup finished first.
+// Adds the partial tiles of each record to C in the record's order (gridDim.y
+// workgroups per record, each over its share of the rows; records cover
+// disjoint parts of C), so the result does not depend on which workgroup
+// finished first.  HBM-bound: 8 bytes per partial value, 16 per value of C
+// (one workgroup per record: 35 us of the 383 of 9000 x 250).
 __global__ __launch_bounds__(256) void k_add_parts(const PartSum* __restrict__ sums, int tn, int tile,
                                                    const double* __restrict__ parts, double* __restrict__ C,
                                                    int64_t ldc, int64_t m)
 {
     const PartSum ps = sums[blockIdx.x];
     const UVT_GLOBAL double* P = gbl(parts) + (int64_t)ps.first * tile;
-    for (int e = threadIdx.x; e < ps.rows * tn; e += 256) {
+    const int per = (ps.rows + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int e_hi = min(ps.rows, ((int)blockIdx.y + 1) * per) * tn;
+    for (int e = (int)blockIdx.y * per * tn + (int)threadIdx.x; e < e_hi; e += 256) {
         const int r = e / tn, c = e % tn;
         if ((int64_t)ps.c0 + c >= m) continue;
         UVT_GLOBAL double* p = gbl(C) + (int64_t)(ps.r0 + r) * ldc + (ps.c0 + c);
         double x = *p;
-        for (int q = 0; q < ps.count; ++q) x += P[(int64_t)q * tile + e];
+        int q = 0;
+        for (; q + 4 <= ps.count; q += 4) {  // four loads in flight, added in order
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = P[(int64_t)(q + u) * tile + e];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x += v[u];
+        }
+        for (; q < ps.count; ++q) x += P[(int64_t)q * tile + e];
         *p = x;
     }
 }
@@ -204,8 +216,29 @@ __global__ __launch_bounds__(256) void k_sk_fixup(SkGeo g, const double* __restr
     }
 }
 
-// One wave per row: sum_j |C[i][j]|, lanes strided over columns, then a
-// fixed butterfly, so the order (and the result) is the same on every run.
+// sum_j |c[j]| by one wave: lanes strided over columns, then a fixed
+// butterfly, so the order (and the result) is the same on every run.
+__device__ __forceinline__ double wave_abs_sum(const UVT_GLOBAL double* c, int64_t m, int lane)
+{
+    double s = 0.0;
+    for (int64_t j = lane; j < m; j += 16 * 64) {  // sixteen loads in flight, added in order
+        double v[16];
+        if (j + 15 * 64 < m) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = c[j + 64 * u];
+        } else {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = j + 64 * u < m ? c[j + 64 * u] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += fabs(v[u]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    return s;
+}
+
+// One wave per row.
 __global__ __launch_bounds__(256) void k_row_abs_sums(int64_t n, int64_t m,
                                                       const double* __restrict__ C, int64_t ldc,
                                                       double* __restrict__ out)
@@ -213,29 +246,48 @@ __global__ __launch_bounds__(256) void k_row_abs_sums(int64_t n, int64_t m,
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= n) return;
-    const double* c = C + row * ldc;
-    double s = 0.0;
-    for (int64_t j = lane; j < m; j += 64) s += fabs(c[j]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    const double s = wave_abs_sum(gbl(C) + row * ldc, m, lane);
     if (lane == 0) out[row] = s;
 }
 
-__global__ __launch_bounds__(1024) void k_max_reduce(int64_t n, const double* __restrict__ v,
-                                                     double* __restrict__ out)
+// max_i sum_j |C[i][j]| in one launch, HBM-bound: every wave keeps the largest
+// of its rows, every workgroup leaves one value in part, and the last one to
+// finish (done, left at zero again) writes the largest to host memory.  (Row
+// sums, a second launch for their maximum and a copy of 8 bytes took 21 us on
+// the GPU at 2048 x 2048, and the host waited for each in turn.)
+constexpr int kNormBlocks = 512, kNormWaves = 8;
+__global__ __launch_bounds__(64 * kNormWaves) void k_inf_norm(int64_t n, int64_t m, const double* __restrict__ C, int64_t ldc,
+                                                  double* __restrict__ part, unsigned* __restrict__ done,
+                                                  double* __restrict__ out)
 {
-    __shared__ double part[16];
+    __shared__ double best[kNormWaves];
+    __shared__ bool last;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto block_max = [&](double v) {  // over the waves' values, in thread 0
+        if (lane == 0) best[wave] = v;
+        __syncthreads();
+        for (int w = 1; w < kNormWaves; ++w) v = fmax(v, best[w]);
+        return v;
+    };
     double x = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += 1024) x = fmax(x, v[i]);
+    for (int64_t row = (int64_t)blockIdx.x * kNormWaves + wave; row < n; row += (int64_t)gridDim.x * kNormWaves)
+        x = fmax(x, wave_abs_sum(gbl(C) + row * ldc, m, lane));
+    x = block_max(x);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&part[blockIdx.x], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
+    }
+    __syncthreads();
+    if (!last) return;
+    x = 0.0;
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += 64 * kNormWaves)
+        x = fmax(x, __hip_atomic_load(&part[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        x = threadIdx.x < 16 ? part[threadIdx.x] : 0.0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
-        if (threadIdx.x == 0) out[0] = x;
+    x = block_max(x);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(out, x, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -328,6 +380,8 @@ extern "C" uvt_status uvt_destroy(uvt_handle h)
     if (!h) return UVT_ERR_ARG;
     (void)hipSetDevice(h->device);
     if (h->work) (void)hipFree(h->work);
+    if (h->norm_part) (void)hipFree(h->norm_part);
+    if (h->norm_host) (void)hipHostFree(h->norm_host);
     for (int i = 0; i < 2; ++i) {
         if (h->pin_done[i]) (void)hipEventSynchronize(h->pin_done[i]);
         if (h->pin[i]) (void)hipHostFree(h->pin[i]);
@@ -769,7 +823,7 @@ extern "C" uvt_status uvt_trmm_f64(uvt_handle h, uvt_plan plan, const double* dA
     if (st != UVT_OK) return st;
     if (plan->nsums > 0) {
         const int32_t tm = uvt_cfg_tile_m(plan->cfg), tn = uvt_cfg_tile_n(plan->cfg);
-        hipLaunchKernelGGL(k_add_parts, dim3((unsigned)plan->nsums), dim3(256), 0, s, (const PartSum*)plan->dev_sums,
+        hipLaunchKernelGGL(k_add_parts, dim3((unsigned)plan->nsums, 8), dim3(256), 0, s, (const PartSum*)plan->dev_sums,
                            (int)tn, (int)(tm * tn), (const double*)parts, dC, ldc, plan->m);
         UVT_HIP(hipGetLastError());
     }
@@ -819,18 +873,29 @@ extern "C" uvt_status uvt_inf_norm(uvt_handle h, int64_t n, int64_t m, const dou
 {
     if (!h || !dC || !norm || n <= 0 || m <= 0 || ldc < m) return UVT_ERR_ARG;
     UVT_HIP(hipSetDevice(h->device));
-    void* w = nullptr;
-    uvt_status st = uvt_handle_workspace(h, (size_t)(n + 1) * sizeof(double), &w);
-    if (st != UVT_OK) return st;
-    double* rows = (double*)w;
-    st = uvt_row_abs_sums(h, n, m, dC, ldc, rows, stream);
-    if (st != UVT_OK) return st;
-    hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(1024), 0, (hipStream_t)stream, n, rows,
-                       rows + n);
+    const int64_t want = (n + kNormWaves - 1) / kNormWaves;
+    if (!h->norm_part) {  // partial maxima and the counter, zeroed once
+        void* d = nullptr;
+        if (hipMalloc(&d, (kNormBlocks + 1) * sizeof(double)) != hipSuccess) {
+            (void)hipGetLastError();
+            return UVT_ERR_NOMEM;
+        }
+        if (hipMemset(d, 0, (kNormBlocks + 1) * sizeof(double)) != hipSuccess ||
+            hipStreamSynchronize(nullptr) != hipSuccess ||  // before any stream's launch
+            hipHostMalloc((void**)&h->norm_host, sizeof(double), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(d);
+            h->norm_host = nullptr;
+            return UVT_ERR_NOMEM;
+        }
+        h->norm_part = (double*)d;
+    }
+    hipLaunchKernelGGL(k_inf_norm, dim3((unsigned)std::min<int64_t>(want, kNormBlocks)),
+                       dim3(64 * kNormWaves), 0, (hipStream_t)stream, n, m, dC, ldc, h->norm_part, (unsigned*)(h->norm_part + kNormBlocks),
+                       h->norm_host);
     UVT_HIP(hipGetLastError());
-    UVT_HIP(hipMemcpyAsync(norm, rows + n, sizeof(double), hipMemcpyDeviceToHost,
-                           (hipStream_t)stream));
     UVT_HIP(hipStreamSynchronize((hipStream_t)stream));
+    *norm = *(volatile double*)h->norm_host;
     return UVT_OK;
 }
 

@@ -13,8 +13,10 @@ struct uvt_handle_s {
     int device;
     int cus;
     size_t vram;
-    void* work;        // grows on demand (norm row sums, BLAS-form packing)
+    void* work;        // grows on demand (dtrmm's copy of B)
     size_t work_bytes;
+    double* norm_part; // uvt_inf_norm: partial maxima and their counter (device),
+    double* norm_host; // and the result (pinned host memory), on first use
     void* scratch;     // this device's fixed scratch array (uvt_dtrmm_noalloc)
     // pinned bounce buffers of strided host copies (uvt_memcpy_2d), on first use
     void* pin[2];
