@@ -256,8 +256,8 @@ enum { UVT_ROUTE_AUTO = 0, UVT_ROUTE_INT8 = 1, UVT_ROUTE_FP64 = 2 };
 
 typedef struct uvt_batch_s *uvt_batch;
 
-/* Plans a batch: the FP64 problems become one longest-first tile queue
- * consumed by persistent kernels (tile shape per problem from the tuning
+/* Plans a batch: the tiles of the FP64 problems become one queue per XCD,
+ * drained by a persistent kernel (tile shape per problem from the tuning
  * table: a file written by uvt_autotune_f64, or NULL for the built-in one);
  * the split problems run through batched split stages with `slices` moduli.
  * Everything is captured once into a hipGraph on the handle's device.  Each

@@ -50,7 +50,7 @@ void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__
         const LaunchTile lt = static_cast<const LaunchTile*>(tiles)[blockIdx.x];
         const uvt_tile& t = lt.t;
         UVT_GLOBAL double* part = lt.part >= 0 ? gbl(parts) + (int64_t)lt.part * (TM * TN) : nullptr;
-        using Opt = TileOpt<true, false, kTriALe, false, false, true, false, false>;
+        using Opt = TileOpt<true, false, kTriALe, false, false, true, false>;
         f64_tile<TM, TN, W::M, W::N, Opt>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
                                           ldb, gbl(C), ldc, m, smem, -1, part);
     } else {
@@ -143,7 +143,7 @@ void k_trmm_sk_f64(SkGeo g, const double* __restrict__ A, int64_t lda, const dou
                    int64_t ldb, double* __restrict__ C, int64_t ldc, double* __restrict__ parts)
 {
     using W = TileWaves<TM, TN>;
-    using Opt = TileOpt<true, false, kTriALe, false, false, false, false, false>;
+    using Opt = TileOpt<true, false, kTriALe, false, false, false, false>;
     static_assert(kTileK == kSkPanel, "stream-K panels are the kernel's k panels");
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
     // The piece arithmetic (64-bit divisions) runs in vector registers; its

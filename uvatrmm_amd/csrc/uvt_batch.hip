@@ -5,13 +5,13 @@
 // A batch is captured once into a graph:
 //   zero the work counters (a fill kernel, not a memset node)
 //   -> scales and residues of the split problems
-//   -> fork: main branch: one persistent kernel draining one queue of the
-//                         FP64 tiles of every problem, each tile with its
-//                         problem's tile shape, most work first
+//   -> fork: main branch: one persistent kernel draining the FP64 tiles of
+//                         every problem, each tile with its problem's tile
+//                         shape, from one queue per XCD (deal_tiles)
 //            side branch: the int8 residue products of the split problems
 //   -> join -> the split reconstruction, which adds the integer box part to
-//              the diagonal blocks the FP64 queue stored.
-// The FP64 queue holds every tile of the FP64 problems and the diagonal-block
+//              the diagonal blocks the FP64 tiles stored.
+// The FP64 queues hold every tile of the FP64 problems and the diagonal-block
 // tiles of the split problems.  Split-class problems run wholly in FP64,
 // which meets their tolerance, unless their route asks for the int8 path or
 // (route auto) the int8 path is measured faster in a batch
@@ -45,6 +45,14 @@ struct BatchTile {
     int32_t prob, r0, rows, c0, k_lo, k_hi, cfg;  // cfg: UVT_CFG_* tile shape
 };
 
+// The queues of the persistent kernel, one per XCD: tiles first[q] to
+// first[q + 1] of the tile list, handed out by counter q * kCounterPad (each
+// counter has a cache line of its own).
+constexpr int kQueues = 8, kCounterPad = 16;
+struct TileQueues {
+    int32_t first[kQueues + 1];
+};
+
 struct BatchProb {
     const double* A;
     const double* B;
@@ -53,34 +61,70 @@ struct BatchProb {
     int32_t vec, pad;
 };
 
+// The next tile for a workgroup that draws from queue q, -1 once every queue
+// is empty; one thread's work.  A workgroup whose queue has run dry goes over
+// to the one with the most tiles left.  (Every failed draw after the first
+// means that a queue has been emptied since it was looked at, so the search
+// ends after at most kQueues of them.)
+__device__ __forceinline__ int draw_tile(int& q, const TileQueues& queues, int* counter)
+{
+    for (;;) {
+        const int i = atomicAdd(counter + kCounterPad * q, 1);
+        if (i < queues.first[q + 1] - queues.first[q]) return queues.first[q] + i;
+        int most = 0, now[kQueues];
+#pragma unroll
+        for (int j = 0; j < kQueues; ++j)
+            now[j] = __hip_atomic_load(counter + kCounterPad * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int j = 0; j < kQueues; ++j) {
+            const int left = queues.first[j + 1] - queues.first[j] - now[j];
+            if (left > most) {
+                most = left;
+                q = j;
+            }
+        }
+        if (most == 0) return -1;
+    }
+}
+
 // Persistent FP64 tile kernel for every tile shape: every workgroup (8
-// waves, LDS for the largest shape) takes the next tile of the queue (an
-// atomic counter) and runs it with that tile's shape, until the queue is
-// empty, so all waves exit once `ntiles` tiles have been handed out.  One
-// queue for all shapes means one drain at the end of the batch instead of
-// one per shape.  128x128 tiles run as 4 x 2 waves of 32x64, 64x64 tiles as
-// 2 x 4 waves of 32x16, 128x32 tiles as 4 x 2 waves of 32x16 (the B panel
-// has half as many pieces as threads).  The order of every sum does not
-// depend on the wave layout, so a tile gives the same bits as the
-// single-problem kernels' tiles of the same shape.
+// waves, LDS for the largest shape) takes the next tile of its XCD's queue
+// (workgroup b runs on XCD b % 8) and runs it with that tile's shape, until
+// every queue is empty.  All shapes share the queues, so there is one drain
+// at the end of the batch instead of one per shape.  128x128 tiles run as
+// 4 x 2 waves of 32x64, 64x64 tiles as 2 x 4 waves of 32x16, 128x32 tiles as
+// 4 x 2 waves of 32x16 (the B panel has half as many pieces as threads).  The
+// order of every sum does not depend on the wave layout, so a tile gives the
+// same bits as the single-problem kernels' tiles of the same shape.
+//
+// Bound: the matrix units, 86 % busy over a batch of 512 uneven problems (n
+// to 4096, m to 1024), at a clock that falls with the traffic behind the L2
+// caches: with one queue for the chip the L2s answered 36 % of the operand
+// reads and that batch took 8.9-9.4 ms, with neighbouring tiles on one XCD
+// (deal_tiles) 7.9-8.6 on the same boxes (same bits).
 constexpr int kBatchThreads = 512;
 __global__ __launch_bounds__(kBatchThreads, 4)
-void k_batch_f64(const BatchTile* __restrict__ tiles, int ntiles, const BatchProb* __restrict__ probs,
+void k_batch_f64(const BatchTile* __restrict__ tiles, TileQueues queues, const BatchProb* __restrict__ probs,
                  int* __restrict__ counter)
 {
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES];
-    using Opt = TileOpt<true, false, kTriALe, false, false, true, true, false>;
+    using Opt = TileOpt<true, false, kTriALe, false, false, true, false>;
     static_assert(F64Cfg<64, 64, 2, 4>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 64, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 32, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES,
                   "LDS sized for the largest shape");
-    __shared__ int next;
+    __shared__ int next, queue;
+    if (threadIdx.x == 0) queue = (int)blockIdx.x % kQueues;
     for (;;) {
-        if (threadIdx.x == 0) next = atomicAdd(counter, 1);
+        if (threadIdx.x == 0) {
+            int q = queue;
+            next = draw_tile(q, queues, counter);
+            queue = q;
+        }
         __syncthreads();
         const int t = __builtin_amdgcn_readfirstlane(next);  // uniform: its records load into scalar registers
         __syncthreads();  // every thread has read `next` before it is overwritten
-        if (t >= ntiles) break;
+        if (t < 0) break;
         const BatchTile bt = tiles[t];
         const BatchProb p = probs[bt.prob];
         // p.pad is always 0, but loaded per tile: the thread index built from
@@ -123,11 +167,11 @@ int persistent_grid(int cus)
     return cus * b;
 }
 
-void launch_persistent(int grid, const BatchTile* tiles, int ntiles, const BatchProb* probs,
+void launch_persistent(int grid, const BatchTile* tiles, const TileQueues& queues, const BatchProb* probs,
                        int* counter, hipStream_t s)
 {
-    const dim3 g((unsigned)std::max(1, std::min(grid, ntiles))), block(kBatchThreads);
-    hipLaunchKernelGGL(k_batch_f64, g, block, 0, s, tiles, ntiles, probs, counter);
+    const dim3 g((unsigned)std::max(1, std::min(grid, queues.first[kQueues]))), block(kBatchThreads);
+    hipLaunchKernelGGL(k_batch_f64, g, block, 0, s, tiles, queues, probs, counter);
 }
 
 // ---- tuning table ------------------------------------------------------------
@@ -223,14 +267,67 @@ void trapezoid_tiles(int prob, int64_t n, int64_t m, int cfg, std::vector<BatchT
         }
 }
 
-// Most work first (depth times tile area), so the queue drains with its
-// smallest tiles.
-void sort_longest_first(std::vector<BatchTile>& v)
+// Deals the tiles (in problem order) out to the queues and puts them in queue
+// order.  A queue takes groups of tiles that read the same operands, each
+// whole problem or as many of its row blocks, deepest first, as make up 1/64
+// of the batch's work; the deepest group goes first, to the queue with the
+// least work so far.  Tiles of a group then run side by side on one XCD and
+// find each other's panels in its L2.  Measured on 512 uneven problems, n to
+// 4096, m to 1024: groups of one row block 8.97-9.00 ms, of 256 rows 8.81-8.85,
+// 512 8.65-8.69, 1024 8.59, whole problems 8.34-8.35; 60 problems of 2048 x
+// 1024, where whole problems leave the queues uneven: 4.27-4.30 ms by 1/32 of
+// the work, 4.11-4.12 by 1/64, 4.14 by 1/128, 4.16 by 1/256.
+// The last 128 tiles of a queue (two for each of its XCD's 64 workgroups) go
+// most work first, so that it drains with its smallest: 200 problems of
+// 512 x 512 524 us, 550 without, 531 with 256.
+TileQueues deal_tiles(std::vector<BatchTile>& v)
 {
+    constexpr int kGroups = 64, kTail = 128;
     auto work = [](const BatchTile& t) {
         return (int64_t)(t.k_hi - t.k_lo) * uvt_cfg_tile_m(t.cfg) * uvt_cfg_tile_n(t.cfg);
     };
-    std::stable_sort(v.begin(), v.end(), [&](const BatchTile& a, const BatchTile& b) { return work(a) > work(b); });
+    struct Group {
+        size_t lo, hi;
+        int64_t top, sum;  // work of its largest tile and of all of them
+    };
+    int64_t total = 0;
+    for (const BatchTile& t : v) total += work(t);
+    std::vector<Group> groups;
+    for (size_t i = 0; i < v.size();) {
+        size_t e = i;
+        while (e < v.size() && v[e].prob == v[i].prob) ++e;
+        std::stable_sort(v.begin() + i, v.begin() + e,
+                         [](const BatchTile& a, const BatchTile& b) { return a.r0 > b.r0; });
+        while (i < e) {
+            Group g{i, i, 0, 0};
+            do {  // one row block
+                for (const int r0 = v[g.hi].r0; g.hi < e && v[g.hi].r0 == r0; ++g.hi) {
+                    g.top = std::max(g.top, work(v[g.hi]));
+                    g.sum += work(v[g.hi]);
+                }
+            } while (g.hi < e && g.sum < total / kGroups);
+            groups.push_back(g);
+            i = g.hi;
+        }
+    }
+    std::stable_sort(groups.begin(), groups.end(), [](const Group& a, const Group& b) { return a.top > b.top; });
+    std::vector<BatchTile> q[kQueues];
+    int64_t load[kQueues] = {0};
+    for (const Group& g : groups) {
+        const int to = (int)(std::min_element(load, load + kQueues) - load);
+        load[to] += g.sum;
+        q[to].insert(q[to].end(), v.begin() + g.lo, v.begin() + g.hi);
+    }
+    TileQueues r;
+    v.clear();
+    for (int j = 0; j < kQueues; ++j) {
+        std::stable_sort(q[j].end() - std::min<size_t>(q[j].size(), kTail), q[j].end(),
+                         [&](const BatchTile& a, const BatchTile& b) { return work(a) > work(b); });
+        r.first[j] = (int32_t)v.size();
+        v.insert(v.end(), q[j].begin(), q[j].end());
+    }
+    r.first[kQueues] = (int32_t)v.size();
+    return r;
 }
 
 // Split-class problems whose integer box part is too small to pay for its
@@ -245,7 +342,8 @@ struct uvt_batch_s {
     // FP64 part
     std::vector<int> f64_index;        // problem -> slot in the FP64 table
     std::vector<BatchProb> f64_probs;  // host image
-    std::vector<BatchTile> tiles;  // one queue of every tile shape
+    std::vector<BatchTile> tiles;  // every tile shape, queue after queue
+    TileQueues queues;
     BatchTile* d_tiles = nullptr;
     BatchProb* d_probs = nullptr;
     int* d_counters = nullptr;
@@ -374,8 +472,8 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         if (use_int8) b->int8_flops += (double)p.m * (double)p.n * (double)p.n;
         if (use_int8) b->sp.push_back(uvt_split_problem{p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.n, p.m});
     }
-    sort_longest_first(b->tiles);
     if (b->tiles.size() > 0x7FFFFFFF) st = UVT_ERR_SIZE;
+    else b->queues = deal_tiles(b->tiles);
     if (st != UVT_OK) {
         batch_free(b);
         return st;
@@ -398,7 +496,7 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         BATCH_HIP(hipMemcpy(b->d_probs, b->f64_probs.data(), b->f64_probs.size() * sizeof(BatchProb),
                             hipMemcpyHostToDevice));
     }
-    BATCH_HIP(hipMalloc(&b->d_counters, 128 * sizeof(int)));
+    BATCH_HIP(hipMalloc(&b->d_counters, kQueues * kCounterPad * sizeof(int)));
     // split buffers
     if (!b->sp.empty()) {
         int64_t lut_entries = 0;
@@ -428,7 +526,8 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
     BATCH_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
     BATCH_HIP(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     BATCH_HIP(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(128), 0, b->cap, b->d_counters, 128);
+    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kQueues * kCounterPad), 0, b->cap, b->d_counters,
+                       kQueues * kCounterPad);
     // scales and residues of the split problems first: short kernels that
     // would be starved behind the persistent FP64 workgroups
     if (!b->sp.empty())
@@ -437,16 +536,16 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
                                     b->cap, UVT_SPLIT_PREP);
     BATCH_HIP(hipEventRecord(b->fork, b->cap));
     BATCH_HIP(hipStreamWaitEvent(b->side, b->fork, 0));
-    // int8 residue products on the side branch, the FP64 queue on the main one
+    // int8 residue products on the side branch, the FP64 tiles on the main one
     if (st == UVT_OK && !b->sp.empty())
         st = uvt_split_batch_launch(b->sp.data(), (int)b->sp.size(), slices, b->d_split_work,
                                     b->d_split_desc, b->d_split_lut, b->split_totals, b->split_lut_off,
                                     b->side, UVT_SPLIT_GEMM);
     if (!b->tiles.empty())
-        launch_persistent(grid, b->d_tiles, (int)b->tiles.size(), b->d_probs, b->d_counters, b->cap);
+        launch_persistent(grid, b->d_tiles, b->queues, b->d_probs, b->d_counters, b->cap);
     BATCH_HIP(hipEventRecord(b->join, b->side));
     BATCH_HIP(hipStreamWaitEvent(b->cap, b->join, 0));
-    // the reconstruction adds to the diagonal blocks the FP64 queue stored
+    // the reconstruction adds to the diagonal blocks the FP64 tiles stored
     if (st == UVT_OK && !b->sp.empty())
         st = uvt_split_batch_launch(b->sp.data(), (int)b->sp.size(), slices, b->d_split_work,
                                     b->d_split_desc, b->d_split_lut, b->split_totals, b->split_lut_off,
@@ -576,7 +675,8 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
     if (hipMalloc(&A, (size_t)nmax * nmax * 8) != hipSuccess ||
         hipMalloc(&B, (size_t)nmax * mmax * 8) != hipSuccess ||
         hipMalloc(&C, c_bytes) != hipSuccess ||
-        hipMalloc(&counter, 64) != hipSuccess || hipMalloc(&dprobs, max_copies * sizeof(BatchProb)) != hipSuccess ||
+        hipMalloc(&counter, kQueues * kCounterPad * sizeof(int)) != hipSuccess ||
+        hipMalloc(&dprobs, max_copies * sizeof(BatchProb)) != hipSuccess ||
         hipStreamCreate(&s) != hipSuccess || hipEventCreate(&e0) != hipSuccess ||
         hipEventCreate(&e1) != hipSuccess) {
         (void)hipGetLastError();
@@ -605,7 +705,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
             for (int cfg = 0; cfg < UVT_NUM_CFGS; ++cfg) {
                 std::vector<BatchTile> tiles;
                 for (int c = 0; c < copies; ++c) trapezoid_tiles(c, n, m, cfg, tiles);
-                sort_longest_first(tiles);
+                const TileQueues queues = deal_tiles(tiles);
                 if (dtiles) (void)hipFree(dtiles);
                 dtiles = nullptr;
                 if (hipMalloc(&dtiles, tiles.size() * sizeof(BatchTile)) != hipSuccess ||
@@ -615,9 +715,10 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
                 }
                 float cfg_best = 1e30f;
                 for (int rep = 0; rep < 4; ++rep) {
-                    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, counter, 16);
+                    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kQueues * kCounterPad), 0, s, counter,
+                                       kQueues * kCounterPad);
                     (void)hipEventRecord(e0, s);
-                    launch_persistent(grid, dtiles, (int)tiles.size(), dprobs, counter, s);
+                    launch_persistent(grid, dtiles, queues, dprobs, counter, s);
                     (void)hipEventRecord(e1, s);
                     float ms_ = 0.f;
                     if (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms_, e0, e1) != hipSuccess) {

@@ -78,7 +78,7 @@ void k_blas_f64(Walk g, const double* __restrict__ A, int64_t lda, const double*
 {
     using W = TileWaves<TM, TN>;
     constexpr bool kNone = TRI == kTriNone, kRight = TRI == kTriBLe || TRI == kTriBGe;
-    using Opt = TileOpt<A_KC, B_KC, kNone ? kTriALe : (TriKind)TRI, !kNone, true, true, false, false>;
+    using Opt = TileOpt<A_KC, B_KC, kNone ? kTriALe : (TriKind)TRI, !kNone, true, true, false>;
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
     const int b = (int)blockIdx.x;
     int rt = kRight ? b % g.nrt : b / g.nct, ct = kRight ? b / g.nrt : b % g.nct;

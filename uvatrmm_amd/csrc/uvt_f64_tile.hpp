@@ -8,7 +8,7 @@
 // for k > i.
 //
 // Data path: A and B k-panels (16 deep) stream from HBM with 16-byte loads
-// into registers one panel ahead (two with AHEAD2), are written to a
+// into registers one panel ahead, are written to a
 // double-buffered LDS tile, and each wave multiplies its (TM/WAVES_M) x
 // (TN/WAVES_N) sub-tile with v_mfma_f64_16x16x4_f64 (one double of A and B
 // per lane, four doubles of C per lane).  Each operand keeps its memory
@@ -213,13 +213,6 @@ enum TriKind {
 // EDGE_IDLE: waves of an edge tile that hold no row or column of C run no
 // products (off where a caller's own registers leave no room for the test:
 // the stream-K kernel then spills inside its masked k loop).
-// AHEAD2: the global loads of panel kt + 2 are issued right after panel
-// kt + 1 goes to LDS (during the products of panel kt) instead of at the top
-// of panel kt + 1, so the load registers are never live across a panel's
-// start.  It lowers register pressure where one kernel holds several tile
-// shapes (the persistent batch kernel: 12 bytes of spills per lane instead
-// of 52, 1.5-3 % faster); the single-shape kernels ran 0.2-1.7 % slower
-// with it.  The sums and their order are the same either way.
 // PIPE_MASKED: the masked panels run the software pipeline too.  Without it
 // they leave 16 registers to their addresses and masks, which the kernels
 // with more of their own need (8165 x 939 stream-K 1033 us with it, 1021
@@ -227,10 +220,10 @@ enum TriKind {
 // the plain walks are faster with it (4096^2: 992
 // us, 1004 without).
 template <bool A_KC_ = true, bool B_KC_ = false, TriKind TRI_ = kTriALe, bool UNIT_ = false, bool EPI_ = false,
-          bool EDGE_IDLE_ = true, bool AHEAD2_ = false, bool PIPE_MASKED_ = true>
+          bool EDGE_IDLE_ = true, bool PIPE_MASKED_ = true>
 struct TileOpt {
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_, UNIT = UNIT_, EPI = EPI_, EDGE_IDLE = EDGE_IDLE_,
-                          AHEAD2 = AHEAD2_, PIPE_MASKED = PIPE_MASKED_;
+                          PIPE_MASKED = PIPE_MASKED_;
     static constexpr TriKind TRI = TRI_;
     static constexpr bool TRI_A = TRI == kTriALe || TRI == kTriAGe, GE = TRI == kTriAGe || TRI == kTriBGe;
 };
@@ -277,7 +270,7 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
     using PA = typename G::PA;
     using PB = typename G::PB;
     constexpr int BK = kTileK;
-    constexpr bool AHEAD2 = OPT::AHEAD2, GE = OPT::GE, TRI_A = OPT::TRI_A, UNIT = OPT::UNIT;
+    constexpr bool GE = OPT::GE, TRI_A = OPT::TRI_A, UNIT = OPT::UNIT;
     const int tid = thread >= 0 ? thread : (int)threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: branches on it stay scalar
@@ -459,10 +452,6 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
             load(k_at(0), masked);
             store(0, k_at(0), masked);
         }
-        if (AHEAD2 && nk > 1) {
-            if (f0 <= 1 && 1 < f1) load(k_at(1), full);
-            else load(k_at(1), masked);
-        }
         __syncthreads();
         // A panel whose k lies on the zero side of the triangle for all of a
         // wave's rows (columns) holds only zeros for it: the wave runs it
@@ -475,22 +464,7 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         const bool idle = OPT::EDGE_IDLE && (wm * G::WM >= t.rows || wn * G::WN >= cols);
         int kt = 0;
         if (OPT::PIPE_MASKED || kt + 1 < f1) read0(kt & 1);
-        // Registers hold the next panel's values from here on when AHEAD2.
-        if constexpr (AHEAD2) {
-            if (idle) {  // this wave only feeds the others
-                for (; kt + 2 < f1; ++kt) {
-                    store((kt & 1) ^ 1, 0, full);
-                    load(k_at(kt + 2), full);
-                    __syncthreads();
-                }
-            }
-            for (; kt + 2 < f1; ++kt) {  // the panel after next is full
-                compute(kt & 1, [&] {
-                    store((kt & 1) ^ 1, 0, full);
-                    load(k_at(kt + 2), full);
-                });
-            }
-        } else if (idle) {  // this wave only feeds the others
+        if (idle) {  // this wave only feeds the others
             for (; kt + 1 < f1; ++kt) {
                 load(k_at(kt + 1), full);
                 store((kt & 1) ^ 1, 0, full);
@@ -519,17 +493,15 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
         }
         for (; kt < nk_w; ++kt) {
             const bool more = kt + 1 < nk;
-            if (!AHEAD2 && more) load(k_at(kt + 1), masked);
+            if (more) load(k_at(kt + 1), masked);
             compute_masked(kt & 1, [&] {
                 if (more) store((kt & 1) ^ 1, k_at(kt + 1), masked);
-                if (AHEAD2 && kt + 2 < nk) load(k_at(kt + 2), masked);
             });
         }
         for (; kt < nk; ++kt) {
             if (kt + 1 < nk) {
-                if (!AHEAD2) load(k_at(kt + 1), masked);
+                load(k_at(kt + 1), masked);
                 store((kt & 1) ^ 1, k_at(kt + 1), masked);
-                if (AHEAD2 && kt + 2 < nk) load(k_at(kt + 2), masked);
             }
             __syncthreads();
         }
