@@ -11,6 +11,7 @@
 #include "uvt_f64_tile.hpp"
 #include "uvt_f64_wave.hpp"
 #include "uvt_internal.h"
+#include "uvt_place.hpp"
 #include "uvt_runtime.hpp"
 #include "uvt_sk.hpp"
 
@@ -91,27 +92,27 @@ __global__ __launch_bounds__(256) void k_add_parts(const PartSum* __restrict__ s
     }
 }
 
-// The trapezoid walk without a tile list: workgroup b takes row tile
-// nrt-1-b/nct (longest reduction first) and column tile b%nct.
+// The trapezoid walk without a tile list: longest reduction first, placed by
+// walk_tile (uvt_place.hpp).
 template <int TM, int TN>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
-void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, const double* __restrict__ A,
+void k_trmm_trapezoid_f64(int64_t n, int64_t m, int nrt, int nct, int cus, const double* __restrict__ A,
                           int64_t lda, const double* __restrict__ B, int64_t ldb,
                           double* __restrict__ C, int64_t ldc)
 {
     using W = TileWaves<TM, TN>;
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N>::SMEM_DOUBLES];
-    const int rt = nrt - 1 - (int)(blockIdx.x / nct), ct = (int)(blockIdx.x % nct);
-    const int r0 = rt * TM;
+    const WalkTile w = walk_tile((int)blockIdx.x, nrt * nct, nct, cus, W::BLOCKS_PER_CU);
+    const int r0 = (nrt - 1 - w.outer) * TM;
     const int rows = (int)(n - r0 < TM ? n - r0 : TM);
-    f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, ct * TN, 0, r0 + rows, kTileLower}, gbl(A), lda, gbl(B), ldb,
+    f64_tile<TM, TN, W::M, W::N>(TileArgs{r0, rows, w.inner * TN, 0, r0 + rows, kTileLower}, gbl(A), lda, gbl(B), ldb,
                                  gbl(C), ldc, m, smem);
 }
 
 // The trapezoid walk of a small product in wave tiles (uvt_f64_wave.hpp), four
 // to a workgroup, wn of them along the columns: deepest first, every second
-// run of `snake` workgroups turned round (see snake()).
+// run of `snake` workgroups turned round (as uvt_place.hpp's).
 template <int FM, int FN, int D>
 __global__ __launch_bounds__(256) void k_trmm_waves_f64(int64_t n, int64_t m, int nrt, int nct, int wn, int snake,
                                                         const double* __restrict__ A, int64_t lda,
@@ -451,16 +452,6 @@ int blocks_per_cu(int32_t cfg)
     return TileWaves<128, 128>::BLOCKS_PER_CU;
 }
 
-// Tiles that all fit the GPU at once are placed, not scheduled: workgroups i,
-// i + cus, i + 2 cus, ... of a launch run on one compute unit (checked on the
-// GPU: 1024 of 1024 workgroups, three launches).  So every second run of cus
-// tiles is turned round, and a compute unit's deep tiles meet shallow ones.
-void snake(std::vector<LaunchTile>& v, int cus)
-{
-    for (size_t g = cus; g < v.size(); g += 2 * (size_t)cus)
-        std::reverse(v.begin() + g, v.begin() + std::min(g + cus, v.size()));
-}
-
 // The launch of a plan on a GPU of `cus` compute units: the whole tiles of the
 // trapezoid walk, for either shape.  (A boxes plan's triangles were a second
 // launch, which read and wrote C once more and waited for the first: N=2048,
@@ -486,8 +477,13 @@ void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile>& launch
     nparts = 0;
     std::vector<uvt_tile> walk(uvt_plan_trapezoid_tiles(pl.n, pl.m, pl.cfg, nullptr));
     uvt_plan_trapezoid_tiles(pl.n, pl.m, pl.cfg, walk.data());  // deepest first
-    for (const uvt_tile& t : walk) launch.push_back(LaunchTile{t, -1});
-    if ((int64_t)launch.size() <= (int64_t)cus * blocks_per_cu(pl.cfg)) snake(launch, cus);
+    const int64_t total = (int64_t)walk.size();
+    const int nct = (int)((pl.m + uvt_cfg_tile_n(pl.cfg) - 1) / uvt_cfg_tile_n(pl.cfg));
+    for (int64_t b = 0; b < total; ++b) {
+        WalkTile w{(int)(b / nct), (int)(b % nct)};
+        if (total <= 0x7FFFFFFF) w = walk_tile((int)b, (int)total, nct, cus, blocks_per_cu(pl.cfg));  // else not launched
+        launch.push_back(LaunchTile{walk[(int64_t)w.outer * nct + w.inner], -1});
+    }
     if (pl.flops < kSplitMinFlops) return;
     int64_t work = 0, deepest = 0;  // k steps, summed over the tiles and the longest
     for (const uvt_tile& w : walk) {
@@ -520,10 +516,22 @@ void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile>& launch
     }
     const size_t tile_bytes = (size_t)uvt_cfg_tile_m(pl.cfg) * uvt_cfg_tile_n(pl.cfg) * sizeof(double);
     if ((size_t)cut_parts * tile_bytes > kMaxPartBytes) return;
-    // deepest first (the walk's order among equals)
+    // Deepest first, and of the pieces of one depth those that read the same
+    // part of A (one for each column tile) one after another; then every 8 such
+    // groups are dealt out to the XCDs, a group to each.  (A piece's column
+    // neighbours on other XCDs each read A from memory: 9000 x 250 381 us, now
+    // 367; 5000 x 300 158 and 151; 12000 x 128 350 and 342.)
     std::stable_sort(cut.begin(), cut.end(), [](const LaunchTile& a, const LaunchTile& b) {
-        return a.t.k_hi - a.t.k_lo > b.t.k_hi - b.t.k_lo;
+        const int32_t la = a.t.k_hi - a.t.k_lo, lb = b.t.k_hi - b.t.k_lo;
+        if (la != lb) return la > lb;
+        return a.t.r0 != b.t.r0 ? a.t.r0 > b.t.r0 : a.t.k_lo < b.t.k_lo;
     });
+    std::vector<LaunchTile> dealt;
+    const int64_t run = (int64_t)kXcds * nct, full = (int64_t)cut.size() / run * run;
+    for (int64_t i = 0; i < full; ++i) dealt.push_back(cut[i / run * run + i % kXcds * nct + i % run / kXcds]);
+    cut.erase(cut.begin(), cut.begin() + full);
+    dealt.insert(dealt.end(), cut.begin(), cut.end());
+    cut.swap(dealt);
     launch.swap(cut);
     sums.swap(cut_sums);
     nparts = cut_parts;
@@ -621,11 +629,12 @@ static uvt_status launch_tiles_f64(int32_t cfg, const void* dtiles, int64_t ntil
 
 template <int TM, int TN>
 static void launch_trapezoid(int64_t n, int64_t m, const double* A, int64_t lda, const double* B, int64_t ldb,
-                             double* C, int64_t ldc, hipStream_t s)
+                             double* C, int64_t ldc, int cus, hipStream_t s)
 {
     const int nrt = (int)((n + TM - 1) / TM), nct = (int)((m + TN - 1) / TN);
     const dim3 grid((unsigned)((int64_t)nrt * nct)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN>), grid, block, 0, s, n, m, nrt, nct, A, lda, B, ldb, C, ldc);
+    hipLaunchKernelGGL((k_trmm_trapezoid_f64<TM, TN>), grid, block, 0, s, n, m, nrt, nct, cus, A, lda, B,
+                       ldb, C, ldc);
 }
 
 // When a product runs in wave tiles, and in which (0: workgroup tiles): a rule
@@ -786,17 +795,17 @@ uvt_status uvt_launch_trapezoid_sk_f64(int32_t cfg, int64_t n, int64_t m, const 
 }
 
 uvt_status uvt_launch_trapezoid_f64(int32_t cfg, int64_t n, int64_t m, const double* A, int64_t lda,
-                                    const double* B, int64_t ldb, double* C, int64_t ldc,
+                                    const double* B, int64_t ldb, double* C, int64_t ldc, int cus,
                                     hipStream_t s)
 {
     if (n <= 0 || m <= 0 || lda < n || ldb < m || ldc < m) return UVT_ERR_ARG;
     if (n > 0x3FFFFFFF || m > 0x3FFFFFFF) return UVT_ERR_SIZE;
     const int64_t tm = uvt_cfg_tile_m(cfg), tn = uvt_cfg_tile_n(cfg);
     if (((n + tm - 1) / tm) * ((m + tn - 1) / tn) > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    if (cfg == UVT_CFG_256x128) launch_trapezoid<256, 128>(n, m, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_64x64) launch_trapezoid<64, 64>(n, m, A, lda, B, ldb, C, ldc, s);
-    else if (cfg == UVT_CFG_128x32) launch_trapezoid<128, 32>(n, m, A, lda, B, ldb, C, ldc, s);
-    else launch_trapezoid<128, 128>(n, m, A, lda, B, ldb, C, ldc, s);
+    if (cfg == UVT_CFG_256x128) launch_trapezoid<256, 128>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    else if (cfg == UVT_CFG_64x64) launch_trapezoid<64, 64>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    else if (cfg == UVT_CFG_128x32) launch_trapezoid<128, 32>(n, m, A, lda, B, ldb, C, ldc, cus, s);
+    else launch_trapezoid<128, 128>(n, m, A, lda, B, ldb, C, ldc, cus, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }

@@ -27,6 +27,7 @@
 #include "uvt_f64_tile.hpp"
 #include "uvt_f64_wave.hpp"
 #include "uvt_internal.h"
+#include "uvt_place.hpp"
 #include "uvt_runtime.hpp"
 
 using namespace uvt;
@@ -62,15 +63,17 @@ __global__ __launch_bounds__(256) void k_copy(const double* __restrict__ src, in
 }
 
 // What a walk multiplies: C (M x N) from a reduction over K, and which
-// operand is triangular (TriKind; kTriNone: neither).
+// operand is triangular (TriKind; kTriNone: neither); cus: the GPU's compute
+// units.
 struct Walk {
     int64_t M, N;
-    int K, nrt, nct;
+    int K, nrt, nct, cus;
 };
 constexpr int kTriNone = -1;
 
 // One tile per workgroup, the deepest reductions first (left side: row tiles
-// of the long end of the triangle; right side: column tiles).
+// of the long end of the triangle; right side: column tiles), placed by
+// walk_tile (uvt_place.hpp).
 template <int TM, int TN, bool A_KC, bool B_KC, int TRI>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N), (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_blas_f64(Walk g, const double* __restrict__ A, int64_t lda, const double* __restrict__ B, int64_t ldb,
@@ -80,8 +83,8 @@ void k_blas_f64(Walk g, const double* __restrict__ A, int64_t lda, const double*
     constexpr bool kNone = TRI == kTriNone, kRight = TRI == kTriBLe || TRI == kTriBGe;
     using Opt = TileOpt<A_KC, B_KC, kNone ? kTriALe : (TriKind)TRI, !kNone, true, true, false>;
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
-    const int b = (int)blockIdx.x;
-    int rt = kRight ? b % g.nrt : b / g.nct, ct = kRight ? b / g.nrt : b % g.nct;
+    const WalkTile wt = walk_tile((int)blockIdx.x, g.nrt * g.nct, kRight ? g.nrt : g.nct, g.cus, W::BLOCKS_PER_CU);
+    int rt = kRight ? wt.inner : wt.outer, ct = kRight ? wt.outer : wt.inner;
     if (TRI == kTriALe) rt = g.nrt - 1 - rt;
     if (TRI == kTriBLe) ct = g.nct - 1 - ct;
     const int r0 = rt * TM, c0 = ct * TN;
@@ -225,7 +228,7 @@ extern "C" uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_
         UVT_HIP(hipGetLastError());
         return UVT_OK;
     }
-    const Walk g{m, n, (int)k, 0, 0};
+    const Walk g{m, n, (int)k, 0, 0, h->cus};
     TileEpi epi;
     epi.alpha = alpha;
     epi.beta = beta;
@@ -308,7 +311,7 @@ uvt_status dtrmm_launch(const DtrmmCall& c, int64_t m, int64_t n, double alpha, 
     double* X = (double*)wv;
     const dim3 grid((unsigned)((n + 63) / 64), (unsigned)std::min<int64_t>((m + 15) / 16, 32768));
     hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, s, dB, ldb, X, c.ldx, m, n);
-    const Walk g{m, n, (int)c.nt, 0, 0};
+    const Walk g{m, n, (int)c.nt, 0, 0, cus};
     TileEpi epi;
     epi.alpha = alpha;
     epi.unit = c.unit;

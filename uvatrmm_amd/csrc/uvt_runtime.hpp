@@ -46,7 +46,7 @@ UVT_INTERNAL uvt_status uvt_handle_workspace(uvt_handle h, size_t bytes, void** 
 // FP64 C = tril(A) * B as one trapezoid walk with the given tile shape,
 // tile coordinates from the workgroup index (no plan, nothing to upload).
 UVT_INTERNAL uvt_status uvt_launch_trapezoid_f64(int32_t cfg, int64_t n, int64_t m, const double* A, int64_t lda,
-                                    const double* B, int64_t ldb, double* C, int64_t ldc,
+                                    const double* B, int64_t ldb, double* C, int64_t ldc, int cus,
                                     hipStream_t s);
 // Whether an n x n by n x m product with these leading dimensions runs in wave
 // tiles (uvt_f64_wave.hpp), and in which: 0 or the shape for

@@ -204,7 +204,7 @@ static uvt_status launch(uvt_server s, Slot& sl)
         const int64_t sk = uvt_sk_workgroups(tile, n, m, s->h->cus);
         e = wave     ? uvt_launch_waves_f64(wave, n, m, dA, n, dB, m, dC, m, s->h->cus, st)
             : sk > 0 ? uvt_launch_trapezoid_sk_f64(tile, n, m, dA, n, dB, m, dC, m, sk, sl.parts, st)
-                     : uvt_launch_trapezoid_f64(tile, n, m, dA, n, dB, m, dC, m, st);
+                     : uvt_launch_trapezoid_f64(tile, n, m, dA, n, dB, m, dC, m, s->h->cus, st);
     }
     if (e != UVT_OK) return e;
     UVT_HIP(hipEventRecord(sl.done, st));

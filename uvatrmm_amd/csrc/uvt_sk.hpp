@@ -29,10 +29,11 @@
 
 #include <stdint.h>
 
+#include "uvt_place.hpp"
+
 namespace uvt {
 
 constexpr int kSkPanel = 16;  // k panel of the FP64 tile kernels
-constexpr int kXcds = 8;      // MI355X: workgroup i of a launch runs on XCD i % 8
 
 struct SkGeo {
     int64_t n, m;  // C = tril(A) * B: A n x n, B and C n x m
