@@ -1,7 +1,8 @@
 // Host-only check of the placement of a walk's tiles (uvt_place.hpp; built
 // and run by tests/test_place_host.py, no GPU): every tile is run by one
 // workgroup, an outer row's inner tiles go to the XCDs in runs, and turning
-// runs of workgroups round keeps each on its XCD.
+// runs of workgroups round keeps each on its XCD; a sequence dealt out in runs
+// gives every XCD as many tiles.
 #include <stdio.h>
 
 #include <vector>
@@ -40,8 +41,8 @@ static void walk(int outer, int inner, int cus, int blocks)
     std::vector<char> seen(total, 0);
     for (int b = 0; b < total; ++b) {
         const int s = snake(b, total, cus, blocks);
-        CHECK(s >= 0 && s < total && s % kXcds == b % kXcds && snake(s, total, cus, blocks) == b && s / cus == b / cus &&
-                  (b < resident || s == b),
+        CHECK(s >= 0 && s < total && s % kXcds == b % kXcds && snake(s, total, cus, blocks) == b &&
+                  s / cus == b / cus && (b < resident || s == b),
               "total %d cus %d blocks %d: %d -> %d", total, cus, blocks, b, s);
         const WalkTile w = walk_tile(b, total, inner, cus, blocks);
         const bool in = w.outer >= 0 && w.outer < outer && w.inner >= 0 && w.inner < inner;
@@ -54,8 +55,31 @@ static void walk(int outer, int inner, int cus, int blocks)
     }
 }
 
+static void runs(int count)
+{
+    std::vector<int> xcd(count, -1);
+    int none = 0, blocks = (count + 255) / 256 * 256, load[kXcds] = {0};
+    for (int b = 0; b < blocks; ++b) {
+        const int p = run_place(b, count);
+        if (p < 0) {
+            ++none;
+            continue;
+        }
+        CHECK(p < count && xcd[p] < 0 && p / 256 == b / 256, "%d tiles, b %d: %d", count, b, p);
+        if (p < count) xcd[p] = b % kXcds;
+        ++load[b % kXcds];
+    }
+    CHECK(none == blocks - count, "%d tiles, %d workgroups without", count, none);
+    for (int x = 0; x < kXcds; ++x)
+        CHECK(load[x] == count / kXcds || load[x] == (count + kXcds - 1) / kXcds, "%d tiles, XCD %d: %d", count, x,
+              load[x]);
+    for (int p = 1; p < count; ++p)
+        CHECK(p % 32 == 0 || p >= count / 256 * 256 || xcd[p] == xcd[p - 1], "%d tiles, place %d", count, p);
+}
+
 int main()
 {
+    for (int count = 1; count <= 1100; ++count) runs(count);
     for (int count = 1; count <= 70; ++count)
         for (int base = 0; base < 8; ++base) band(base, count);
     band(0x7FFFFFFF - 65535, 65535);

@@ -66,4 +66,17 @@ __host__ __device__ inline WalkTile walk_tile(int b, int total, int inner, int c
     return WalkTile{outer, xcd_band(t - outer * inner, outer * inner, inner)};
 }
 
+// The place in a sequence of `count` tiles that workgroup b of a launch with
+// 32 resident workgroups on each XCD runs, -1 for none (the launch is padded
+// to a multiple of 256): an XCD takes runs of 32 tiles; every second round of
+// runs goes the other way, as the sequence falls in depth (5000 x 1500 split
+// products 507 us, 519 without), and the last, short round is shared evenly.
+__host__ __device__ inline int run_place(int b, int count)
+{
+    const int x = b % kXcds, round = b / 256, i = b % 256 / kXcds, full = count / 256;
+    if (round < full) return (round * kXcds + (round % 2 ? kXcds - 1 - x : x)) * 32 + i;
+    const int rest = count % 256, lo = (x * rest + 7) / kXcds, hi = ((x + 1) * rest + 7) / kXcds;
+    return lo + i < hi ? full * 256 + lo + i : -1;
+}
+
 }  // namespace uvt

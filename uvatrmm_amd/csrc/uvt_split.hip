@@ -51,6 +51,7 @@
 #include <string.h>
 
 #include "uvt_f64_tile.hpp"
+#include "uvt_place.hpp"
 #include "uvt_runtime.hpp"
 #include "uvt_split.hpp"
 #include "uvt_xd.hpp"
@@ -712,6 +713,15 @@ __device__ __forceinline__ void i8_tile_loop(const int8_t* __restrict__ Af, int6
 
 // One workgroup: a 256 x 256 tile of (A' B') mod m_l over k in [0, r0), for
 // the launch's moduli l0 .. l0+nl-1.
+//
+// A problem's tiles form one sequence, deepest rows first: runs of gr row
+// tiles; in each, modulus by modulus, groups of gr x 32/gr tiles (fewer at the
+// edges, none of them padding), whose panels an XCD's 32 resident workgroups
+// share through its L2.  run_place (uvt_place.hpp) deals the sequence out to
+// the XCDs.  Whole groups dealt out one by one, padded to 32, left XCDs with
+// up to a third more to do than others: 5000 x 1500 with 13 moduli 574 -> 507
+// us for the call, 10000 x 700 1040 -> 943, 9000 x 3300 2.50 -> 2.36 ms; where
+// the groups fit evenly (8192 x 4096, 32768 x 8192) within 0.3 %.
 __global__ __launch_bounds__(512, 1) void k_gemm_i8(Desc one, const Desc* table, const int* lut, Mods mods)
 {
     __shared__ __attribute__((aligned(16))) int8_t smem[2 * kI8Stage];  // B' only
@@ -720,27 +730,18 @@ __global__ __launch_bounds__(512, 1) void k_gemm_i8(Desc one, const Desc* table,
     const Desc* dp = table ? &table[lut[blockIdx.x]] : nullptr;
 #define UVT_FIELD(f) (dp ? dp->f : one.f)
     const int64_t wb = (int64_t)blockIdx.x - UVT_FIELD(start[K_GEMM]);
-    // XCD-aware mapping.  Workgroups go to the 8 XCDs round-robin (every
-    // problem starts at a multiple of 256 workgroups), so XCD x runs local
-    // blocks x, x+8, ...; its s-th block takes tile s%32 of tile group
-    // (s/32)*8 + x.  A group is gr row tiles x 32/gr column tiles of one
-    // modulus (8 x 4 for large problems), i.e. the 32 workgroups one XCD holds
-    // at once, so they share their A and B panels through that XCD's L2.
-    // Groups run longest-k first.
-    const int xcd = (int)(wb & 7), slot = (int)(wb >> 3);
-    const int g = (slot >> 5) * 8 + xcd, t = slot & 31;
-    const int nct = UVT_FIELD(nct), nrt = UVT_FIELD(nrt);
-    const int gr = UVT_FIELD(gr), gc = 32 / gr;
-    const int ngc = (nct + gc - 1) / gc, per_rg = ngc * mods.nl;
-    const int rg = g / per_rg, grem = g % per_rg;
+    const int nct = UVT_FIELD(nct), nrt = UVT_FIELD(nrt), gr = UVT_FIELD(gr), gc = 32 / gr;
+    const int p = run_place((int)wb, (nrt - 1) * nct * mods.nl);
+    if (p < 0) return;  // padding of the last round (uniform per block)
     // Uniform over the workgroup by construction; readfirstlane tells the
     // compiler, so the depth and the panel bases stay in scalar registers
-    // (the divisions above otherwise leave them in vector registers, and
-    // every k step's clamp and addresses become per-lane arithmetic).
-    const int l = __builtin_amdgcn_readfirstlane(grem / ngc);
-    const int ct = __builtin_amdgcn_readfirstlane((grem % ngc) * gc + t % gc);
-    const int rt = __builtin_amdgcn_readfirstlane(nrt - 1 - (rg * gr + t / gc));
-    if (rt < 1 || ct >= nct) return;  // padding of the last groups (uniform per block)
+    // (the divisions otherwise leave them in vector registers, and every k
+    // step's clamp and addresses become per-lane arithmetic).
+    const int rg = p / (gr * nct * mods.nl), rows = min(gr, nrt - 1 - rg * gr);
+    const int q = p - rg * gr * nct * mods.nl, l = __builtin_amdgcn_readfirstlane(q / (rows * nct));
+    const int u = q - l * rows * nct, cg = u / (rows * gc), v = u - cg * rows * gc, w = min(gc, nct - cg * gc);
+    const int ct = __builtin_amdgcn_readfirstlane(cg * gc + v % w);
+    const int rt = __builtin_amdgcn_readfirstlane(nrt - 1 - (rg * gr + v / w));
     const int64_t r0 = (int64_t)rt * kTileI, c0 = (int64_t)ct * kTileI;
     const int64_t n = UVT_FIELD(n), m = UVT_FIELD(m), kmax = UVT_FIELD(kmax);
     const int lm = mods.l0 + l;  // the modulus
@@ -1109,8 +1110,11 @@ bool too_few_moduli(int64_t n, int nmod)
 }
 
 // Row tiles per XCD group of the int8 products.  8 x 4 groups share panels
-// best through an XCD's L2 (measured); another shape is taken only when it
-// leaves at least 15 % fewer group slots over rtiles x ctiles tiles.
+// best through an XCD's L2 (32768 x 8192 49.0 ms, 49.9 with 4 x 8); up to 256
+// tiles per modulus 4 x 8 ones, whose rows differ less in depth (2000 x 2000
+// 198 us, 207 with 8 x 4; 4000 x 4000 747 and 754).  Another shape is taken
+// only when it leaves at least 15 % fewer group slots over rtiles x ctiles
+// tiles (5000 x 1500 507 us, 519 with 8 x 4 regardless).
 int group_rows(int64_t rtiles, int64_t ctiles)
 {
     static const int pref[] = {8, 4, 16, 2, 32, 1};
@@ -1120,6 +1124,7 @@ int group_rows(int64_t rtiles, int64_t ctiles)
     };
     int64_t best = INT64_MAX;
     for (int gr : pref) best = std::min(best, slots(gr));
+    if (rtiles * ctiles <= 256 && slots(4) * 100 <= best * 115) return 4;
     for (int gr : pref)
         if (slots(gr) * 100 <= best * 115) return gr;
     return 8;
@@ -1127,13 +1132,11 @@ int group_rows(int64_t rtiles, int64_t ctiles)
 
 int64_t kmax_of(int64_t n) { return ((n - 1) / kTileI) * kTileI; }
 
-// Workgroups of one product launch over nl moduli: XCD groups of gr x 32/gr
-// tiles per modulus, 32 workgroups each, padded to a multiple of 256 (8
-// groups) so that every problem starts on XCD 0.
+// Workgroups of one product launch over nl moduli: a tile each, padded to a
+// multiple of 256 so that every problem starts on XCD 0.
 int64_t gemm_blocks(const Desc& d, int nl)
 {
-    const int64_t groups = (int64_t)((d.nrt - 1 + d.gr - 1) / d.gr) * ((d.nct + 32 / d.gr - 1) / (32 / d.gr)) * nl;
-    return (groups + 7) / 8 * 8 * 32;
+    return ((int64_t)(d.nrt - 1) * d.nct * nl + 255) / 256 * 256;
 }
 
 // Moduli per residue-B buffer of a single-problem call: all of them, or half
