@@ -216,9 +216,9 @@ enum TriKind {
 // PIPE_MASKED: the masked panels run the software pipeline too.  Without it
 // they leave 16 registers to their addresses and masks, which the kernels
 // with more of their own need (8165 x 939 stream-K 1033 us with it, 1021
-// without; 9000 x 250 in cut tiles 395 and 387; the batch 9.08 and 8.95 ms);
-// the plain walks are faster with it (4096^2: 992
-// us, 1004 without).
+// without; 9000 x 250 in cut tiles 395 and 387; 512 problems in a batch, from
+// one queue, 9.08 and 8.95 ms); the plain walks are faster with it (4096^2:
+// 992 us, 1004 without).
 template <bool A_KC_ = true, bool B_KC_ = false, TriKind TRI_ = kTriALe, bool UNIT_ = false, bool EPI_ = false,
           bool EDGE_IDLE_ = true, bool PIPE_MASKED_ = true>
 struct TileOpt {
