@@ -61,29 +61,31 @@ struct BatchProb {
     int32_t vec, pad;
 };
 
-// The next tile for a workgroup that draws from queue q, -1 once every queue
-// is empty; one thread's work.  A workgroup whose queue has run dry goes over
-// to the one with the most tiles left.  (Every failed draw after the first
-// means that a queue has been emptied since it was looked at, so the search
-// ends after at most kQueues of them.)
-__device__ __forceinline__ int draw_tile(int& q, const TileQueues& queues, int* counter)
+// The next tile from another queue than q, which has run dry: from the one with
+// the most tiles left, which becomes q; -1 once every queue is empty.  One
+// thread's work.  (Every failed draw means that a queue has been emptied since
+// it was looked at, so the search ends after at most kQueues of them.)
+__device__ __forceinline__ int draw_elsewhere(int& q, const TileQueues& queues, int* counter)
 {
     for (;;) {
-        const int i = atomicAdd(counter + kCounterPad * q, 1);
-        if (i < queues.first[q + 1] - queues.first[q]) return queues.first[q] + i;
-        int most = 0, now[kQueues];
+        int most = 0, lo = 0, now[kQueues];
 #pragma unroll
         for (int j = 0; j < kQueues; ++j)
             now[j] = __hip_atomic_load(counter + kCounterPad * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int size = 0;
 #pragma unroll
         for (int j = 0; j < kQueues; ++j) {
             const int left = queues.first[j + 1] - queues.first[j] - now[j];
             if (left > most) {
                 most = left;
                 q = j;
+                lo = queues.first[j];
+                size = queues.first[j + 1] - lo;
             }
         }
         if (most == 0) return -1;
+        const int i = atomicAdd(counter + kCounterPad * q, 1);
+        if (i < size) return lo + i;
     }
 }
 
@@ -114,17 +116,24 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, TileQueues queues, const B
                       F64Cfg<128, 32, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES,
                   "LDS sized for the largest shape");
     __shared__ int next, queue;
-    if (threadIdx.x == 0) queue = (int)blockIdx.x % kQueues;
+    int q = (int)blockIdx.x % kQueues, first = queues.first[q], size = queues.first[q + 1] - first;  // scalar
     for (;;) {
         if (threadIdx.x == 0) {
-            int q = queue;
-            next = draw_tile(q, queues, counter);
-            queue = q;
+            int from = q;
+            const int i = atomicAdd(counter + kCounterPad * q, 1);
+            next = i < size ? first + i : draw_elsewhere(from, queues, counter);
+            queue = from;
         }
         __syncthreads();
         const int t = __builtin_amdgcn_readfirstlane(next);  // uniform: its records load into scalar registers
-        __syncthreads();  // every thread has read `next` before it is overwritten
+        const int from = __builtin_amdgcn_readfirstlane(queue);
+        __syncthreads();  // every thread has read them before they are overwritten
         if (t < 0) break;
+        if (from != q) {
+            q = from;
+            first = queues.first[q];
+            size = queues.first[q + 1] - first;
+        }
         const BatchTile bt = tiles[t];
         const BatchProb p = probs[bt.prob];
         // p.pad is always 0, but loaded per tile: the thread index built from
