@@ -199,7 +199,8 @@ typedef enum { UVT_NON_UNIT = 0, UVT_UNIT = 1 } uvt_diag;
 /* C = alpha op(A) op(B) + beta C; C (m x n) is not read when beta == 0, A and
  * B are not read when k == 0 or alpha == 0.  Replaces the cblas_dgemm call of
  * UVaTRMM/src/mm_triangular.c:347-360 (RowMajor, NoTrans, NoTrans, alpha 1,
- * beta 0) and covers the other transposes.  Uses no workspace. */
+ * beta 0) and covers the other transposes.  C may share elements with A or B;
+ * only then the call uses the handle's workspace, for C (see uvt_dtrmm). */
 uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_t n, int64_t k,
                      double alpha, const double *dA, int64_t lda, const double *dB, int64_t ldb,
                      double beta, double *dC, int64_t ldc, void *stream);
@@ -207,9 +208,10 @@ uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_
  * in place, A triangular (uplo; only that triangle is read; unit: its
  * diagonal is taken as 1).  Replaces the cblas_dtrmm call of
  * mm_triangular.c:374-387 (RowMajor, Left, Lower, NoTrans, NonUnit, alpha 1)
- * and covers every other side / uplo / trans / diag.  Uses the handle's
- * workspace for a copy of B: calls on one handle that use it (uvt_dtrmm,
- * uvt_inf_norm) must be on one stream or serialized by the caller. */
+ * and covers every other side / uplo / trans / diag.  A may share elements
+ * with B.  Uses the handle's workspace, the size of B: calls on one handle
+ * that use it (uvt_dtrmm, uvt_dgemm with overlapping operands, uvt_inf_norm)
+ * must be on one stream or serialized by the caller. */
 uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans ta, uvt_diag diag,
                      int64_t m, int64_t n, double alpha, const double *dA, int64_t lda,
                      double *dB, int64_t ldb, void *stream);

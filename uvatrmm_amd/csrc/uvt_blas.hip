@@ -6,12 +6,14 @@
 //   dgemm  C = alpha op(A) op(B) + beta C
 //          the rectangular tile walk; the tile reads either operand as it is
 //          stored or transposed, and applies alpha and beta as it writes C
-//          (C is not read when beta == 0).  No workspace.
+//          (C is not read when beta == 0).  No workspace, unless C shares
+//          elements with A or B: then C is computed there and copied back.
 //   dtrmm  B := alpha op(A) B  (left)  or  alpha B op(A)  (right), in place
 //          B is copied to the workspace, then the tile walk multiplies the
-//          copy into B: the triangle masks either operand, lower or upper, a
-//          transposed A is read as it is stored, and a unit diagonal goes in
-//          on the way to LDS.
+//          copy into B (where A shares elements with B: B into the workspace,
+//          which is then copied to B): the triangle masks either operand,
+//          lower or upper, a transposed A is read as it is stored, and a unit
+//          diagonal goes in on the way to LDS.
 // (With op(A), op(B) and the triangle packed row-major and lower first, and
 // the result unpacked afterwards, a dtrmm of a 2048 triangle on 3000 rows
 // took 323 us, of which three packing passes were 57; now 241.  A 1500 x 2000
@@ -27,6 +29,7 @@
 #include "uvt_f64_tile.hpp"
 #include "uvt_f64_wave.hpp"
 #include "uvt_internal.h"
+#include "uvt_overlap.hpp"
 #include "uvt_place.hpp"
 #include "uvt_runtime.hpp"
 
@@ -195,6 +198,12 @@ void scale(int64_t rows, int64_t cols, double beta, double* C, int64_t ldc, hipS
     hipLaunchKernelGGL(k_scale, grid, dim3(256), 0, s, rows, cols, beta, C, ldc);
 }
 
+void copy(const double* src, int64_t lds, double* dst, int64_t ldd, int64_t rows, int64_t cols, hipStream_t s)
+{
+    const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)std::min<int64_t>((rows + 15) / 16, 32768));
+    hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, s, src, lds, dst, ldd, rows, cols);
+}
+
 int64_t even(int64_t x) { return x + (x & 1); }
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -233,10 +242,27 @@ extern "C" uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_
     epi.alpha = alpha;
     epi.beta = beta;
     const int32_t cfg = uvt_default_cfg(m, n);
-    if (tA && tB) return launch_blas<false, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
-    if (tA) return launch_blas<false, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
-    if (tB) return launch_blas<true, true, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
-    return launch_blas<true, false, kTriNone>(cfg, g, dA, lda, dB, ldb, dC, ldc, epi, h->cus, s);
+    const auto walk = [&](double* R, int64_t ldr) {
+        if (tA && tB) return launch_blas<false, true, kTriNone>(cfg, g, dA, lda, dB, ldb, R, ldr, epi, h->cus, s);
+        if (tA) return launch_blas<false, false, kTriNone>(cfg, g, dA, lda, dB, ldb, R, ldr, epi, h->cus, s);
+        if (tB) return launch_blas<true, true, kTriNone>(cfg, g, dA, lda, dB, ldb, R, ldr, epi, h->cus, s);
+        return launch_blas<true, false, kTriNone>(cfg, g, dA, lda, dB, ldb, R, ldr, epi, h->cus, s);
+    };
+    if (!overlap(dC, m, n, ldc, dA, tA ? k : m, tA ? m : k, lda) &&
+        !overlap(dC, m, n, ldc, dB, tB ? n : k, tB ? k : n, ldb))
+        return walk(dC, ldc);
+    // A tile would write C while others still read A or B there.
+    const int64_t ldr = even(n);
+    void* w = nullptr;
+    uvt_status st = uvt_handle_workspace(h, (size_t)m * ldr * 8, &w);
+    if (st != UVT_OK) return st;
+    double* R = (double*)w;
+    if (beta != 0.0) copy(dC, ldc, R, ldr, m, n, s);
+    st = walk(R, ldr);
+    if (st != UVT_OK) return st;
+    copy(R, ldr, dC, ldc, m, n, s);
+    UVT_HIP(hipGetLastError());
+    return UVT_OK;
 }
 
 // ---- dtrmm ---------------------------------------------------------------------
@@ -255,10 +281,10 @@ std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices];  // per device, set once
 
 // One dtrmm call: the triangle's order nt on w columns (rows, right side) of
-// B, and the workspace: a copy of B with an even leading dimension.
+// B, and the workspace: B or the result with an even leading dimension.
 struct DtrmmCall {
     bool right, tA, lower, unit;  // lower: op(A) is
-    int64_t nt, w, ldx;
+    int64_t nt, w, ldw;
     size_t bytes;
     // What uvt_dtrmm_noalloc holds against its scratch: result, B where it is
     // transposed or reversed and the triangle where it is not plain lower,
@@ -290,8 +316,8 @@ uvt_status dtrmm_prepare(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans t
     c->tA = ta == UVT_TRANS;
     c->lower = (uplo == UVT_LOWER) != c->tA;
     c->unit = diag == UVT_UNIT;
-    c->ldx = even(n);
-    c->bytes = up256((size_t)m * c->ldx * 8);
+    c->ldw = even(n);
+    c->bytes = up256((size_t)m * c->ldw * 8);
     const size_t rect = up256((size_t)c->nt * even(c->w) * 8), square = up256((size_t)c->nt * even(c->nt) * 8);
     const bool rev = c->lower == c->right;  // the triangle turned lower by reversal
     c->declared = rect + (c->right || rev ? rect : 0) + (c->tA != c->right || rev || c->unit ? square : 0);
@@ -308,30 +334,41 @@ uvt_status dtrmm_launch(const DtrmmCall& c, int64_t m, int64_t n, double alpha, 
         UVT_HIP(hipGetLastError());
         return UVT_OK;
     }
-    double* X = (double*)wv;
-    const dim3 grid((unsigned)((n + 63) / 64), (unsigned)std::min<int64_t>((m + 15) / 16, 32768));
-    hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, s, dB, ldb, X, c.ldx, m, n);
+    // Where A shares elements with B, B is written only once A has been read.
+    double* const W = (double*)wv;
+    const bool late = overlap(dB, m, n, ldb, dA, c.nt, c.nt, lda);
+    const double* X = late ? dB : W;
+    double* R = late ? W : dB;
+    const int64_t ldx = late ? ldb : c.ldw, ldr = late ? c.ldw : ldb;
+    if (!late) copy(dB, ldb, W, c.ldw, m, n, s);
     const Walk g{m, n, (int)c.nt, 0, 0, cus};
     TileEpi epi;
     epi.alpha = alpha;
     epi.unit = c.unit;
-    if (!c.right) {
-        const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(m, n), m, n);
-        if (c.lower) {
-            if (c.tA) return launch_blas<false, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
-            return launch_blas<true, false, kTriALe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
+    const auto walk = [&] {
+        if (!c.right) {
+            const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(m, n), m, n);
+            if (c.lower) {
+                if (c.tA) return launch_blas<false, false, kTriALe>(cfg, g, dA, lda, X, ldx, R, ldr, epi, cus, s);
+                return launch_blas<true, false, kTriALe>(cfg, g, dA, lda, X, ldx, R, ldr, epi, cus, s);
+            }
+            if (c.tA) return launch_blas<false, false, kTriAGe>(cfg, g, dA, lda, X, ldx, R, ldr, epi, cus, s);
+            return launch_blas<true, false, kTriAGe>(cfg, g, dA, lda, X, ldx, R, ldr, epi, cus, s);
         }
-        if (c.tA) return launch_blas<false, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
-        return launch_blas<true, false, kTriAGe>(cfg, g, dA, lda, X, c.ldx, dB, ldb, epi, cus, s);
-    }
-    // B op(A): column j of the product needs k >= j where op(A) is lower
-    const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(n, m), m, n);
-    if (c.lower) {
-        if (c.tA) return launch_blas<true, true, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
-        return launch_blas<true, false, kTriBGe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
-    }
-    if (c.tA) return launch_blas<true, true, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
-    return launch_blas<true, false, kTriBLe>(cfg, g, X, c.ldx, dA, lda, dB, ldb, epi, cus, s);
+        // B op(A): column j of the product needs k >= j where op(A) is lower
+        const int32_t cfg = uvt_wide_tiles(uvt_default_cfg(n, m), m, n);
+        if (c.lower) {
+            if (c.tA) return launch_blas<true, true, kTriBGe>(cfg, g, X, ldx, dA, lda, R, ldr, epi, cus, s);
+            return launch_blas<true, false, kTriBGe>(cfg, g, X, ldx, dA, lda, R, ldr, epi, cus, s);
+        }
+        if (c.tA) return launch_blas<true, true, kTriBLe>(cfg, g, X, ldx, dA, lda, R, ldr, epi, cus, s);
+        return launch_blas<true, false, kTriBLe>(cfg, g, X, ldx, dA, lda, R, ldr, epi, cus, s);
+    };
+    const uvt_status st = walk();
+    if (st != UVT_OK) return st;
+    if (late) copy(W, c.ldw, dB, ldb, m, n, s);
+    UVT_HIP(hipGetLastError());
+    return UVT_OK;
 }
 
 }  // namespace
