@@ -210,8 +210,8 @@ uvt_status uvt_dgemm(uvt_handle h, uvt_trans ta, uvt_trans tb, int64_t m, int64_
  * mm_triangular.c:374-387 (RowMajor, Left, Lower, NoTrans, NonUnit, alpha 1)
  * and covers every other side / uplo / trans / diag.  A may share elements
  * with B.  Uses the handle's workspace, the size of B: calls on one handle
- * that use it (uvt_dtrmm, uvt_dgemm with overlapping operands, uvt_inf_norm)
- * must be on one stream or serialized by the caller. */
+ * that use it (uvt_dtrmm, uvt_dgemm with overlapping operands) must be on one
+ * stream or serialized by the caller. */
 uvt_status uvt_dtrmm(uvt_handle h, uvt_side side, uvt_uplo uplo, uvt_trans ta, uvt_diag diag,
                      int64_t m, int64_t n, double alpha, const double *dA, int64_t lda,
                      double *dB, int64_t ldb, void *stream);
@@ -384,7 +384,8 @@ uvt_status uvt_serve_destroy(uvt_server s);
 /* Row sums of |C| into d_rowsum[n] (device). */
 uvt_status uvt_row_abs_sums(uvt_handle h, int64_t n, int64_t m, const double *dC, int64_t ldc,
                             double *d_rowsum, void *stream);
-/* max_i sum_j |C[i][j]|; synchronous, result in *norm (host). */
+/* max_i sum_j |C[i][j]|; synchronous, result in *norm (host).  Calls on one
+ * handle from several threads, on any streams, take turns. */
 uvt_status uvt_inf_norm(uvt_handle h, int64_t n, int64_t m, const double *dC, int64_t ldc,
                         double *norm, void *stream);
 

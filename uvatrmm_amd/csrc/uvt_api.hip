@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "uvt_f64_tile.hpp"
@@ -362,18 +363,25 @@ extern "C" uvt_status uvt_create(int device, uvt_handle* out)
     UVT_HIP(hipSetDevice(device));
     hipDeviceProp_t prop;
     UVT_HIP(hipGetDeviceProperties(&prop, device));
-    uvt_handle h = (uvt_handle)calloc(1, sizeof(struct uvt_handle_s));
+    uvt_handle h = new (std::nothrow) uvt_handle_s();  // zeros
     if (!h) return UVT_ERR_NOMEM;
     h->device = device;
     h->cus = prop.multiProcessorCount;
     h->vram = prop.totalGlobalMem;
     const uvt_status st = uvt_noalloc_setup(h);
     if (st != UVT_OK) {
-        free(h);
+        delete h;
         return st;
     }
     *out = h;
     return UVT_OK;
+}
+
+static void norm_free(uvt_handle h)
+{
+    if (h->norm_part) (void)hipFree(h->norm_part);
+    if (h->norm_host) (void)hipHostFree(h->norm_host);
+    h->norm_part = h->norm_host = nullptr;
 }
 
 extern "C" uvt_status uvt_destroy(uvt_handle h)
@@ -381,14 +389,13 @@ extern "C" uvt_status uvt_destroy(uvt_handle h)
     if (!h) return UVT_ERR_ARG;
     (void)hipSetDevice(h->device);
     if (h->work) (void)hipFree(h->work);
-    if (h->norm_part) (void)hipFree(h->norm_part);
-    if (h->norm_host) (void)hipHostFree(h->norm_host);
+    norm_free(h);
     for (int i = 0; i < 2; ++i) {
         if (h->pin_done[i]) (void)hipEventSynchronize(h->pin_done[i]);
         if (h->pin[i]) (void)hipHostFree(h->pin[i]);
         if (h->pin_done[i]) (void)hipEventDestroy(h->pin_done[i]);
     }
-    free(h);
+    delete h;
     return UVT_OK;
 }
 
@@ -883,14 +890,16 @@ extern "C" uvt_status uvt_inf_norm(uvt_handle h, int64_t n, int64_t m, const dou
     if (!h || !dC || !norm || n <= 0 || m <= 0 || ldc < m) return UVT_ERR_ARG;
     UVT_HIP(hipSetDevice(h->device));
     const int64_t want = (n + kNormWaves - 1) / kNormWaves;
+    // Held until the result is read: the handle has one set of partial maxima
+    // and one result, which the next call would write over.
+    std::lock_guard<std::mutex> lk(h->norm_mu);
     if (!h->norm_part) {  // partial maxima and the counter, zeroed once
         void* d = nullptr;
         if (hipMalloc(&d, (kNormBlocks + 1) * sizeof(double)) != hipSuccess) {
             (void)hipGetLastError();
             return UVT_ERR_NOMEM;
         }
-        if (hipMemset(d, 0, (kNormBlocks + 1) * sizeof(double)) != hipSuccess ||
-            hipStreamSynchronize(nullptr) != hipSuccess ||  // before any stream's launch
+        if (hipMemsetAsync(d, 0, (kNormBlocks + 1) * sizeof(double), (hipStream_t)stream) != hipSuccess ||
             hipHostMalloc((void**)&h->norm_host, sizeof(double), hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             (void)hipFree(d);
@@ -899,11 +908,14 @@ extern "C" uvt_status uvt_inf_norm(uvt_handle h, int64_t n, int64_t m, const dou
         }
         h->norm_part = (double*)d;
     }
-    hipLaunchKernelGGL(k_inf_norm, dim3((unsigned)std::min<int64_t>(want, kNormBlocks)),
-                       dim3(64 * kNormWaves), 0, (hipStream_t)stream, n, m, dC, ldc, h->norm_part, (unsigned*)(h->norm_part + kNormBlocks),
+    hipLaunchKernelGGL(k_inf_norm, dim3((unsigned)std::min<int64_t>(want, kNormBlocks)), dim3(64 * kNormWaves), 0,
+                       (hipStream_t)stream, n, m, dC, ldc, h->norm_part, (unsigned*)(h->norm_part + kNormBlocks),
                        h->norm_host);
-    UVT_HIP(hipGetLastError());
-    UVT_HIP(hipStreamSynchronize((hipStream_t)stream));
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {
+        (void)hipGetLastError();
+        norm_free(h);  // the counter may not be zero: the next call makes new ones
+        return UVT_ERR_HIP;
+    }
     *norm = *(volatile double*)h->norm_host;
     return UVT_OK;
 }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <mutex>
 #include <vector>
 
 #include "uvt_internal.h"
@@ -15,8 +16,9 @@ struct uvt_handle_s {
     size_t vram;
     void* work;        // grows on demand (dtrmm's copy of B)
     size_t work_bytes;
-    double* norm_part; // uvt_inf_norm: partial maxima and their counter (device),
-    double* norm_host; // and the result (pinned host memory), on first use
+    std::mutex norm_mu; // uvt_inf_norm, one call at a time: its partial maxima
+    double* norm_part;  // and their counter (device) and its result (pinned
+    double* norm_host;  // host memory), on first use
     void* scratch;     // this device's fixed scratch array (uvt_dtrmm_noalloc)
     // pinned bounce buffers of strided host copies (uvt_memcpy_2d), on first use
     void* pin[2];
