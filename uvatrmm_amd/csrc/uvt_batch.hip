@@ -7,7 +7,8 @@
 //   -> scales and residues of the split problems
 //   -> fork: main branch: one persistent kernel draining the FP64 tiles of
 //                         every problem, each tile with its problem's tile
-//                         shape, from one queue per XCD (deal_tiles)
+//                         shape, from one queue per XCD and one that all
+//                         share (uvt_queues.hpp)
 //            side branch: the int8 residue products of the split problems
 //   -> join -> the split reconstruction, which adds the integer box part to
 //              the diagonal blocks the FP64 tiles stored.
@@ -34,24 +35,13 @@
 
 #include "uvt_f64_tile.hpp"
 #include "uvt_internal.h"
+#include "uvt_queues.hpp"
 #include "uvt_runtime.hpp"
 #include "uvt_split.hpp"
 
 using namespace uvt;
 
 namespace {
-
-struct BatchTile {
-    int32_t prob, r0, rows, c0, k_lo, k_hi, cfg;  // cfg: UVT_CFG_* tile shape
-};
-
-// The queues of the persistent kernel, one per XCD: tiles first[q] to
-// first[q + 1] of the tile list, handed out by counter q * kCounterPad (each
-// counter has a cache line of its own).
-constexpr int kQueues = 8, kCounterPad = 16;
-struct TileQueues {
-    int32_t first[kQueues + 1];
-};
 
 struct BatchProb {
     const double* A;
@@ -61,39 +51,11 @@ struct BatchProb {
     int32_t vec, pad;
 };
 
-// The next tile from another queue than q, which has run dry: from the one with
-// the most tiles left, which becomes q; -1 once every queue is empty.  One
-// thread's work.  (Every failed draw means that a queue has been emptied since
-// it was looked at, so the search ends after at most kQueues of them.)
-__device__ __forceinline__ int draw_elsewhere(int& q, const TileQueues& queues, int* counter)
-{
-    for (;;) {
-        int most = 0, lo = 0, now[kQueues];
-#pragma unroll
-        for (int j = 0; j < kQueues; ++j)
-            now[j] = __hip_atomic_load(counter + kCounterPad * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int size = 0;
-#pragma unroll
-        for (int j = 0; j < kQueues; ++j) {
-            const int left = queues.first[j + 1] - queues.first[j] - now[j];
-            if (left > most) {
-                most = left;
-                q = j;
-                lo = queues.first[j];
-                size = queues.first[j + 1] - lo;
-            }
-        }
-        if (most == 0) return -1;
-        const int i = atomicAdd(counter + kCounterPad * q, 1);
-        if (i < size) return lo + i;
-    }
-}
-
 // Persistent FP64 tile kernel for every tile shape: every workgroup (8
-// waves, LDS for the largest shape) takes the next tile of its XCD's queue
-// (workgroup b runs on XCD b % 8) and runs it with that tile's shape, until
-// every queue is empty.  All shapes share the queues, so there is one drain
-// at the end of the batch instead of one per shape.  128x128 tiles run as
+// waves, LDS for the largest shape) runs its first tile, then draws from its
+// XCD's queue, then from the shared one (uvt_queues.hpp), and ends when that
+// is empty.  All shapes share the queues, so there is one drain at the end of
+// the batch instead of one per shape.  128x128 tiles run as
 // 4 x 2 waves of 32x64, 64x64 tiles as 2 x 4 waves of 32x16, 128x32 tiles as
 // 4 x 2 waves of 32x16 (the B panel has half as many pieces as threads).  The
 // order of every sum does not depend on the wave layout, so a tile gives the
@@ -115,25 +77,11 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, TileQueues queues, const B
                       F64Cfg<128, 64, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES &&
                       F64Cfg<128, 32, 4, 2>::SMEM_DOUBLES <= F64Cfg<128, 128, 4, 2>::SMEM_DOUBLES,
                   "LDS sized for the largest shape");
-    __shared__ int next, queue;
-    int q = (int)blockIdx.x % kQueues, first = queues.first[q], size = queues.first[q + 1] - first;  // scalar
-    for (;;) {
-        if (threadIdx.x == 0) {
-            int from = q;
-            const int i = atomicAdd(counter + kCounterPad * q, 1);
-            next = i < size ? first + i : draw_elsewhere(from, queues, counter);
-            queue = from;
-        }
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(next);  // uniform: its records load into scalar registers
-        const int from = __builtin_amdgcn_readfirstlane(queue);
-        __syncthreads();  // every thread has read them before they are overwritten
-        if (t < 0) break;
-        if (from != q) {
-            q = from;
-            first = queues.first[q];
-            size = queues.first[q + 1] - first;
-        }
+    __shared__ int next;
+    const int q = (int)blockIdx.x % kQueues, first = queues.first[q], size = queues.first[q + 1] - first;  // scalar
+    const int shared = queues.first[kQueues], rest = queues.first[kQueues + 1] - shared;
+    bool own = size > 0;  // the XCD's queue may hold more
+    for (int t = (int)blockIdx.x;;) {
         const BatchTile bt = tiles[t];
         const BatchProb p = probs[bt.prob];
         // p.pad is always 0, but loaded per tile: the thread index built from
@@ -154,9 +102,28 @@ void k_batch_f64(const BatchTile* __restrict__ tiles, TileQueues queues, const B
         else if (bt.cfg == UVT_CFG_128x64) run(i128, i64, i4, i2);
         else if (bt.cfg == UVT_CFG_128x32) run(i128, i32, i4, i2);
         else run(i128, i128, i4, i2);
+        if (size == 0 && rest == 0) break;
+        if (threadIdx.x == 0) {
+            int x = -1;
+            if (own) {
+                const int i = atomicAdd(counter + kCounterPad * q, 1);
+                if (i < size) x = first + i;
+            }
+            if (x < 0 && rest > 0) {
+                const int i = atomicAdd(counter + kCounterPad * kQueues, 1);
+                if (i < rest) x = shared + i;
+            }
+            next = x;
+        }
         __syncthreads();  // the LDS tile is reused by the next tile
+        t = __builtin_amdgcn_readfirstlane(next);  // uniform: its records load into scalar registers
+        __syncthreads();  // every thread has read it before it is overwritten
+        if (t < 0) break;
+        own = t < shared;
     }
 }
+
+constexpr int kCounters = (kQueues + 1) * kCounterPad;  // of one batch
 
 __global__ void k_zero_ints(int* p, int n)
 {
@@ -179,7 +146,7 @@ int persistent_grid(int cus)
 void launch_persistent(int grid, const BatchTile* tiles, const TileQueues& queues, const BatchProb* probs,
                        int* counter, hipStream_t s)
 {
-    const dim3 g((unsigned)std::max(1, std::min(grid, queues.first[kQueues]))), block(kBatchThreads);
+    const dim3 g((unsigned)std::max(1, std::min(grid, queues.first[kQueues + 1]))), block(kBatchThreads);
     hipLaunchKernelGGL(k_batch_f64, g, block, 0, s, tiles, queues, probs, counter);
 }
 
@@ -276,67 +243,9 @@ void trapezoid_tiles(int prob, int64_t n, int64_t m, int cfg, std::vector<BatchT
         }
 }
 
-// Deals the tiles (in problem order) out to the queues and puts them in queue
-// order.  A queue takes groups of tiles that read the same operands, each
-// whole problem or as many of its row blocks, deepest first, as make up 1/64
-// of the batch's work; the deepest group goes first, to the queue with the
-// least work so far.  Tiles of a group then run side by side on one XCD and
-// find each other's panels in its L2.  Measured on 512 uneven problems, n to
-// 4096, m to 1024: groups of one row block 8.97-9.00 ms, of 256 rows 8.81-8.85,
-// 512 8.65-8.69, 1024 8.59, whole problems 8.34-8.35; 60 problems of 2048 x
-// 1024, where whole problems leave the queues uneven: 4.27-4.30 ms by 1/32 of
-// the work, 4.11-4.12 by 1/64, 4.14 by 1/128, 4.16 by 1/256.
-// The last 128 tiles of a queue (two for each of its XCD's 64 workgroups) go
-// most work first, so that it drains with its smallest: 200 problems of
-// 512 x 512 524 us, 550 without, 531 with 256.
-TileQueues deal_tiles(std::vector<BatchTile>& v)
+int64_t tile_work(const BatchTile& t)
 {
-    constexpr int kGroups = 64, kTail = 128;
-    auto work = [](const BatchTile& t) {
-        return (int64_t)(t.k_hi - t.k_lo) * uvt_cfg_tile_m(t.cfg) * uvt_cfg_tile_n(t.cfg);
-    };
-    struct Group {
-        size_t lo, hi;
-        int64_t top, sum;  // work of its largest tile and of all of them
-    };
-    int64_t total = 0;
-    for (const BatchTile& t : v) total += work(t);
-    std::vector<Group> groups;
-    for (size_t i = 0; i < v.size();) {
-        size_t e = i;
-        while (e < v.size() && v[e].prob == v[i].prob) ++e;
-        std::stable_sort(v.begin() + i, v.begin() + e,
-                         [](const BatchTile& a, const BatchTile& b) { return a.r0 > b.r0; });
-        while (i < e) {
-            Group g{i, i, 0, 0};
-            do {  // one row block
-                for (const int r0 = v[g.hi].r0; g.hi < e && v[g.hi].r0 == r0; ++g.hi) {
-                    g.top = std::max(g.top, work(v[g.hi]));
-                    g.sum += work(v[g.hi]);
-                }
-            } while (g.hi < e && g.sum < total / kGroups);
-            groups.push_back(g);
-            i = g.hi;
-        }
-    }
-    std::stable_sort(groups.begin(), groups.end(), [](const Group& a, const Group& b) { return a.top > b.top; });
-    std::vector<BatchTile> q[kQueues];
-    int64_t load[kQueues] = {0};
-    for (const Group& g : groups) {
-        const int to = (int)(std::min_element(load, load + kQueues) - load);
-        load[to] += g.sum;
-        q[to].insert(q[to].end(), v.begin() + g.lo, v.begin() + g.hi);
-    }
-    TileQueues r;
-    v.clear();
-    for (int j = 0; j < kQueues; ++j) {
-        std::stable_sort(q[j].end() - std::min<size_t>(q[j].size(), kTail), q[j].end(),
-                         [&](const BatchTile& a, const BatchTile& b) { return work(a) > work(b); });
-        r.first[j] = (int32_t)v.size();
-        v.insert(v.end(), q[j].begin(), q[j].end());
-    }
-    r.first[kQueues] = (int32_t)v.size();
-    return r;
+    return (int64_t)(t.k_hi - t.k_lo) * uvt_cfg_tile_m(t.cfg) * uvt_cfg_tile_n(t.cfg);
 }
 
 // Split-class problems whose integer box part is too small to pay for its
@@ -351,7 +260,7 @@ struct uvt_batch_s {
     // FP64 part
     std::vector<int> f64_index;        // problem -> slot in the FP64 table
     std::vector<BatchProb> f64_probs;  // host image
-    std::vector<BatchTile> tiles;  // every tile shape, queue after queue
+    std::vector<BatchTile> tiles;  // every tile shape, in the order of uvt_queues.hpp
     TileQueues queues;
     BatchTile* d_tiles = nullptr;
     BatchProb* d_probs = nullptr;
@@ -481,8 +390,9 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         if (use_int8) b->int8_flops += (double)p.m * (double)p.n * (double)p.n;
         if (use_int8) b->sp.push_back(uvt_split_problem{p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.n, p.m});
     }
+    const int grid = persistent_grid(h->cus);
     if (b->tiles.size() > 0x7FFFFFFF) st = UVT_ERR_SIZE;
-    else b->queues = deal_tiles(b->tiles);
+    else b->queues = deal_tiles(b->tiles, grid, tile_work);
     if (st != UVT_OK) {
         batch_free(b);
         return st;
@@ -505,7 +415,7 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         BATCH_HIP(hipMemcpy(b->d_probs, b->f64_probs.data(), b->f64_probs.size() * sizeof(BatchProb),
                             hipMemcpyHostToDevice));
     }
-    BATCH_HIP(hipMalloc(&b->d_counters, kQueues * kCounterPad * sizeof(int)));
+    BATCH_HIP(hipMalloc(&b->d_counters, kCounters * sizeof(int)));
     // split buffers
     if (!b->sp.empty()) {
         int64_t lut_entries = 0;
@@ -529,14 +439,12 @@ extern "C" uvt_status uvt_batch_create(uvt_handle h, const uvt_problem* probs, i
         }
     }
     // capture (occupancy queries first: nothing but stream work inside the capture)
-    const int grid = persistent_grid(h->cus);
     BATCH_HIP(hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking));
     BATCH_HIP(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
     BATCH_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
     BATCH_HIP(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     BATCH_HIP(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kQueues * kCounterPad), 0, b->cap, b->d_counters,
-                       kQueues * kCounterPad);
+    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kCounters), 0, b->cap, b->d_counters, kCounters);
     // scales and residues of the split problems first: short kernels that
     // would be starved behind the persistent FP64 workgroups
     if (!b->sp.empty())
@@ -684,7 +592,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
     if (hipMalloc(&A, (size_t)nmax * nmax * 8) != hipSuccess ||
         hipMalloc(&B, (size_t)nmax * mmax * 8) != hipSuccess ||
         hipMalloc(&C, c_bytes) != hipSuccess ||
-        hipMalloc(&counter, kQueues * kCounterPad * sizeof(int)) != hipSuccess ||
+        hipMalloc(&counter, kCounters * sizeof(int)) != hipSuccess ||
         hipMalloc(&dprobs, max_copies * sizeof(BatchProb)) != hipSuccess ||
         hipStreamCreate(&s) != hipSuccess || hipEventCreate(&e0) != hipSuccess ||
         hipEventCreate(&e1) != hipSuccess) {
@@ -714,7 +622,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
             for (int cfg = 0; cfg < UVT_NUM_CFGS; ++cfg) {
                 std::vector<BatchTile> tiles;
                 for (int c = 0; c < copies; ++c) trapezoid_tiles(c, n, m, cfg, tiles);
-                const TileQueues queues = deal_tiles(tiles);
+                const TileQueues queues = deal_tiles(tiles, grid, tile_work);
                 if (dtiles) (void)hipFree(dtiles);
                 dtiles = nullptr;
                 if (hipMalloc(&dtiles, tiles.size() * sizeof(BatchTile)) != hipSuccess ||
@@ -724,8 +632,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
                 }
                 float cfg_best = 1e30f;
                 for (int rep = 0; rep < 4; ++rep) {
-                    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kQueues * kCounterPad), 0, s, counter,
-                                       kQueues * kCounterPad);
+                    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kCounters), 0, s, counter, kCounters);
                     (void)hipEventRecord(e0, s);
                     launch_persistent(grid, dtiles, queues, dprobs, counter, s);
                     (void)hipEventRecord(e1, s);
