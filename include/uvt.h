@@ -142,8 +142,9 @@ int32_t uvt_device_cus(uvt_handle h);
  * rows above k in k's 128-row tile through A's structural zeros (0 * Inf =
  * NaN), where a BLAS dtrmm would leave them finite; finite inputs are not
  * affected.  Small products (at most 13000 16x16 tiles of C, under 6e9 to 8e9
- * flops) run as one wave per tile and keep nothing on the device; for others
- * the plan allocates its launch records there on its first use on a device.
+ * flops; of n from 7000 to 27000, under 2e9) run as one wave per tile and
+ * keep nothing on the device; for others the plan allocates its launch records
+ * there on its first use on a device.
  * A plan of at least 2e9 flops whose whole tiles would not finish together
  * (narrow B: few, deep tiles) splits its long reductions and adds the pieces
  * after the first of a tile to C afterwards in k order (results repeat bit for

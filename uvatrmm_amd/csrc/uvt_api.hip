@@ -657,12 +657,13 @@ static void launch_trapezoid(int64_t n, int64_t m, const double* A, int64_t lda,
 //    1600 x 1600     98.4 / 108     91.7   80.0     (10000)
 //    1800 x 1800    127   / 182    159    123       (12769)
 //    2048 x 2048    136   / 202    154    155       (16384)
-// and, deep and narrow, where workgroup tiles cut their reductions:
-//    5000 x 128     106   /  89.0   89.3  184       (3.2e9 flops)
-//    5000 x 250     151   / 198    143    187       (6.2e9)
-//    5000 x 300     169   / 267    186    188       (7.5e9)
-//    4000 x 500     172   / 210    160    156       (8.0e9)
-//    9000 x 250     386   / 711    504    413       (2.0e10)
+// and, deep and narrow, where a plan's workgroup tiles cut their reductions:
+//    3000 x 300      67.1 /  89.3   65.2  116       (2.7e9 flops)
+//    4000 x 250      88.9 / 114     80.2  152       (4.0e9)
+//    5000 x 96       73.7 /  69.6   88.2  187       (2.4e9)
+//    5000 x 160      93.6 / 117     91.2  188       (4.0e9)
+//    5000 x 250     124   / 192    139    190       (6.2e9)
+//    4000 x 400     136   / 183    143    154       (6.4e9)
 // Small tiles share less per load, so each size's waves go from 16x16 to
 // 16x32 to 32x32 as there are enough of them for every SIMD; 32x32 ones need
 // reductions to spread (400 x 8192: 35.3 us in workgroup tiles, 34.4 in
@@ -817,6 +818,29 @@ uvt_status uvt_launch_trapezoid_f64(int32_t cfg, int64_t n, int64_t m, const dou
     return UVT_OK;
 }
 
+// Whether a plan that could run in wave tiles runs in workgroup tiles all the
+// same: one whose reductions those cut (build_launch) and are so deep that a
+// wave alone takes longer over its own.  us, cut workgroup tiles / wave tiles
+// of 16x16 / 16x32:
+//     6000 x 64       57.8 /  73.9 / 102      (2.3e9 flops)
+//     6000 x 96       93.8 /  91.2 / 106      (3.5e9)
+//     6000 x 160     127   / 158   / 122      (5.8e9)
+//     7000 x 48       79.4 /  89.4 / 119      (2.4e9)
+//     7000 x 96      118   / 132   / 123      (4.7e9)
+//     9000 x 31       84.1 / 205   / 210      (2.5e9; uncut before: 153)
+//    12500 x 33      227   / 435   / 321      (5.2e9)
+//    16000 x 16      217   / 308   / 320      (4.1e9)
+//    22000 x 9       413   / 450              (4.4e9)
+//    26000 x 7       562   / 581              (4.7e9)
+//    28000 x 7       653   / 640              (5.5e9; the reads of A bound both)
+// and below 2e9 flops, where nothing is cut:
+//     8000 x 31      406   / 133   / 158
+//    10000 x 16      558   / 177   / 190
+static bool deep_and_narrow(const uvt_plan_s& pl)
+{
+    return pl.n >= 7000 && pl.n < 27000 && pl.flops >= kSplitMinFlops;
+}
+
 extern "C" uvt_status uvt_trmm_f64(uvt_handle h, uvt_plan plan, const double* dA, int64_t lda,
                                    const double* dB, int64_t ldb, double* dC, int64_t ldc,
                                    void* stream)
@@ -825,9 +849,20 @@ extern "C" uvt_status uvt_trmm_f64(uvt_handle h, uvt_plan plan, const double* dA
     if (lda < plan->n || ldb < plan->m || ldc < plan->m) return UVT_ERR_ARG;
     UVT_HIP(hipSetDevice(h->device));
     hipStream_t s = (hipStream_t)stream;
-    if (const int shape = uvt_wave_shape(plan->n, plan->m, lda, ldb))
+    // Wave tiles take no device memory: a deep plan without its records yet
+    // runs in them too where memory cannot be had (none left, or a capture).
+    const int shape = uvt_wave_shape(plan->n, plan->m, lda, ldb);
+    const auto waves = [&] {
         return uvt_launch_waves_f64(shape, plan->n, plan->m, dA, lda, dB, ldb, dC, ldc, h->cus, s);
+    };
+    if (shape && !deep_and_narrow(*plan)) return waves();
+    if (shape && plan->dev_id != h->device) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        UVT_HIP(hipStreamIsCapturing(s, &capture));
+        if (capture != hipStreamCaptureStatusNone) return waves();
+    }
     uvt_status st = plan_upload(h, plan);
+    if (shape && st == UVT_ERR_NOMEM) return waves();
     if (st != UVT_OK) return st;
     double* parts = (double*)plan->dev_parts;
     if (plan->sk_grid > 0)
@@ -850,7 +885,8 @@ extern "C" uvt_status uvt_plan_launch_info(uvt_handle h, uvt_plan plan, int64_t*
                                            int64_t* partial_tiles)
 {
     if (!h || !plan) return UVT_ERR_ARG;
-    if (const int shape = uvt_wave_shape(plan->n, plan->m, plan->n, plan->m)) {
+    const int shape = uvt_wave_shape(plan->n, plan->m, plan->n, plan->m);
+    if (shape && !deep_and_narrow(*plan)) {
         if (workgroups) *workgroups = wave_grid(shape, plan->n, plan->m).launch();
         if (partial_tiles) *partial_tiles = 0;
         return UVT_OK;
