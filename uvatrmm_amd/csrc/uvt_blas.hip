@@ -157,9 +157,19 @@ void launch_walk_waves(Walk g, const double* A, int64_t lda, const double* B, in
 //    1024 x 1024 x 1024    43.6 / 50.6 / 39.1   (4096)
 //    3000 x 500 x 800      57.1 / 62.7 / 48.4   (6016)
 //    1300 x 1300 x 3000   205   / 345  / 289    (6724)
-int gemm_wave_shape(int64_t M, int64_t N)
+// Where C is only written, shallow products that fill the chip are bound by
+// that, and go in workgroup tiles, which write whole lines:
+//    1024 x 1024 x 16      4.9 /  6.5 /  5.5
+//    1024 x 1024 x 64      6.7 /  9.0 /  7.0
+//    3000 x 500 x 32       7.3 /  8.5 /  7.6
+//    1001 x 1203 x 64      8.9 / 10.7 /  8.8
+//    1001 x 1203 x 100    12.5 / 12.8 / 11.5
+//    768 x 768 x 32        5.3 /  5.4 /  5.1    (2304)
+//    1024 x 1024 x 64      8.2 /  9.6 /  8.0    (C read too)
+int gemm_wave_shape(int64_t M, int64_t N, int64_t K, double beta)
 {
     const int64_t tiles = ((M + 15) / 16) * ((N + 15) / 16);
+    if (tiles > 2304 && K <= 64 && beta == 0.0) return 0;
     return tiles <= 1024 ? 11 : tiles <= 6144 ? 12 : 0;
 }
 
@@ -170,7 +180,7 @@ uvt_status launch_blas(int32_t cfg, const Walk& g, const double* A, int64_t lda,
                        double* C, int64_t ldc, const TileEpi& epi, int cus, hipStream_t s)
 {
     constexpr bool kRight = TRI == kTriBLe || TRI == kTriBGe;
-    const int wave = TRI == kTriNone ? gemm_wave_shape(g.M, g.N)
+    const int wave = TRI == kTriNone ? gemm_wave_shape(g.M, g.N, g.K, epi.beta)
                      : kRight        ? uvt_wave_shape(g.K, g.M, ldb, lda)
                                      : uvt_wave_shape(g.K, g.N, lda, ldb);
     if (wave) {
