@@ -38,8 +38,8 @@ struct PartSum {
 };
 
 // PARTS: the records are LaunchTiles (some write partial tiles); else plain
-// uvt_tiles, every one writing C.
-template <int TM, int TN, bool PARTS>
+// uvt_tiles, every one writing C.  WIDE: see TileOpt.
+template <int TM, int TN, bool PARTS, bool WIDE>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__ A, int64_t lda,
@@ -47,18 +47,18 @@ void k_trmm_tiles_f64(const void* __restrict__ tiles, const double* __restrict__
                       int64_t ldc, int64_t m, double* __restrict__ parts)
 {
     using W = TileWaves<TM, TN>;
-    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N>::SMEM_DOUBLES];
+    using Opt = TileOpt<true, false, kTriALe, false, false, true, !PARTS, WIDE>;
+    __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
     if constexpr (PARTS) {
         const LaunchTile lt = static_cast<const LaunchTile*>(tiles)[blockIdx.x];
         const uvt_tile& t = lt.t;
         UVT_GLOBAL double* part = lt.part >= 0 ? gbl(parts) + (int64_t)lt.part * (TM * TN) : nullptr;
-        using Opt = TileOpt<true, false, kTriALe, false, false, true, false>;
         f64_tile<TM, TN, W::M, W::N, Opt>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
                                           ldb, gbl(C), ldc, m, smem, -1, part);
     } else {
         const uvt_tile t = static_cast<const uvt_tile*>(tiles)[blockIdx.x];
-        f64_tile<TM, TN, W::M, W::N>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
-                                     ldb, gbl(C), ldc, m, smem);
+        f64_tile<TM, TN, W::M, W::N, Opt>(TileArgs{t.r0, t.rows, t.c0, t.k_lo, t.k_hi, t.flags}, gbl(A), lda, gbl(B),
+                                          ldb, gbl(C), ldc, m, smem);
     }
 }
 
@@ -138,14 +138,14 @@ __global__ __launch_bounds__(256) void k_trmm_waves_f64(int64_t n, int64_t m, in
 // another, in column tile w % ncg of each piece's row tile when the launch
 // runs column groups; its first piece writes partial tile w if it starts
 // inside its tile, every other piece starts at k = 0 and writes C.
-template <int TM, int TN>
+template <int TM, int TN, bool WIDE>
 __global__ __launch_bounds__((64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N),
                              (TileWaves<TM, TN>::WAVES_PER_EU))
 void k_trmm_sk_f64(SkGeo g, const double* __restrict__ A, int64_t lda, const double* __restrict__ B,
                    int64_t ldb, double* __restrict__ C, int64_t ldc, double* __restrict__ parts)
 {
     using W = TileWaves<TM, TN>;
-    using Opt = TileOpt<true, false, kTriALe, false, false, false, false>;
+    using Opt = TileOpt<true, false, kTriALe, false, false, false, false, WIDE>;
     static_assert(kTileK == kSkPanel, "stream-K panels are the kernel's k panels");
     __shared__ __attribute__((aligned(16))) double smem[F64Cfg<TM, TN, W::M, W::N, Opt>::SMEM_DOUBLES];
     // The piece arithmetic (64-bit divisions) runs in vector registers; its
@@ -491,7 +491,7 @@ void build_launch(const uvt_plan_s& pl, int cus, std::vector<LaunchTile>& launch
         if (total <= 0x7FFFFFFF) w = walk_tile((int)b, (int)total, nct, cus, blocks_per_cu(pl.cfg));  // else not launched
         launch.push_back(LaunchTile{walk[(int64_t)w.outer * nct + w.inner], -1});
     }
-    if (pl.flops < kSplitMinFlops) return;
+    if (pl.flops < kSplitMinFlops || uvt_cfg_tile_n(pl.cfg) >= 128) return;
     int64_t work = 0, deepest = 0;  // k steps, summed over the tiles and the longest
     for (const uvt_tile& w : walk) {
         const int64_t len = (int64_t)w.k_hi - w.k_lo;
@@ -606,18 +606,32 @@ static uvt_status plan_upload(uvt_handle h, uvt_plan plan)
 // FP64 TRMM
 // ---------------------------------------------------------------------
 
+// Whether tiles of this shape have full panels with these leading dimensions
+// (else: TileOpt::WIDE).
+static bool full_panels_fit(int32_t cfg, int64_t lda, int64_t ldb)
+{
+    const int32_t rows = uvt_cfg_tile_m(cfg);
+    return (rows == 256   ? PanelIdx<256, 64, true>::offsets_fit(lda)
+            : rows == 128 ? PanelIdx<128, 64, true>::offsets_fit(lda)
+                          : PanelIdx<64, 64, true>::offsets_fit(lda)) &&
+           PanelIdx<128, 64, false>::offsets_fit(ldb);
+}
+
 // parts == nullptr: dtiles holds uvt_tiles; else LaunchTiles.
-template <int TM, int TN>
+template <int TM, int TN, bool WIDE>
 static void launch_tiles(const void* dtiles, int64_t ntiles, const double* A, int64_t lda, const double* B,
                          int64_t ldb, double* C, int64_t ldc, int64_t m, double* parts, hipStream_t s)
 {
     const dim3 grid((unsigned)ntiles), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    if (parts)
-        hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, true>), grid, block, 0, s, dtiles, A, lda, B, ldb, C, ldc, m,
-                           parts);
-    else
-        hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, false>), grid, block, 0, s, dtiles, A, lda, B, ldb, C, ldc, m,
-                           parts);
+    if constexpr (TN < 128) {  // only these are cut (build_launch)
+        if (parts) {
+            hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, true, WIDE>), grid, block, 0, s, dtiles, A, lda, B, ldb, C,
+                               ldc, m, parts);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_trmm_tiles_f64<TM, TN, false, WIDE>), grid, block, 0, s, dtiles, A, lda, B, ldb, C, ldc, m,
+                       parts);
 }
 
 static uvt_status launch_tiles_f64(int32_t cfg, const void* dtiles, int64_t ntiles,
@@ -626,10 +640,16 @@ static uvt_status launch_tiles_f64(int32_t cfg, const void* dtiles, int64_t ntil
 {
     if (ntiles <= 0) return UVT_OK;
     if (ntiles > 0x7FFFFFFF) return UVT_ERR_SIZE;
-    if (cfg == UVT_CFG_256x128) launch_tiles<256, 128>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
-    else if (cfg == UVT_CFG_64x64) launch_tiles<64, 64>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
-    else if (cfg == UVT_CFG_128x32) launch_tiles<128, 32>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
-    else launch_tiles<128, 128>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+    const auto launch = [&](auto wide) {
+        constexpr bool W = decltype(wide)::value;
+        if (cfg == UVT_CFG_256x128) launch_tiles<256, 128, W>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+        else if (cfg == UVT_CFG_64x64) launch_tiles<64, 64, W>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+        else if (cfg == UVT_CFG_128x32)  // WIDE: an A of 235 GB or more
+            launch_tiles<128, 32, false>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+        else launch_tiles<128, 128, W>(dtiles, ntiles, A, lda, B, ldb, C, ldc, m, parts, s);
+    };
+    if (full_panels_fit(cfg, lda, ldb)) launch(std::false_type{});
+    else launch(std::true_type{});
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }
@@ -673,8 +693,12 @@ int uvt_wave_shape(int64_t n, int64_t m, int64_t lda, int64_t ldb)
     const int64_t tiles = ((n + 15) / 16) * ((m + 15) / 16);
     const double flops = (double)m * (double)n * (double)n;
     if (n > 32768 || tiles > 13000 || flops >= (tiles > 7500 ? 8e9 : 6e9)) return 0;
-    if (!WaveOperand<2, true, false>::fits(lda) || !WaveOperand<2, false, false>::fits(ldb)) return 0;
-    return tiles <= 2500 ? 11 : tiles <= 7500 || n < 512 ? 12 : 22;
+    if (tiles <= 2500) return 11;
+    if (tiles <= 7500 || n < 512) return 12;
+    // Without full panels (rows of 64 MB or longer) 32x32 tiles lose: 1500 x
+    // 1500 220 us, 136 in workgroup tiles; smaller tiles do not: 1024 x 400 40
+    // and 82, 1200 x 1200 79 and 97.
+    return WaveOperand<2, true, false>::fits(lda) && WaveOperand<2, false, false>::fits(ldb) ? 22 : 0;
 }
 
 namespace {
@@ -715,12 +739,12 @@ uvt_status uvt_launch_waves_f64(int shape, int64_t n, int64_t m, const double* A
     return UVT_OK;
 }
 
-template <int TM, int TN>
+template <int TM, int TN, bool WIDE>
 static void launch_trapezoid_sk(const SkGeo& g, const double* A, int64_t lda, const double* B, int64_t ldb,
                                 double* C, int64_t ldc, double* parts, hipStream_t s)
 {
     const dim3 grid((unsigned)sk_launch(g)), block(64 * TileWaves<TM, TN>::M * TileWaves<TM, TN>::N);
-    hipLaunchKernelGGL((k_trmm_sk_f64<TM, TN>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc, parts);
+    hipLaunchKernelGGL((k_trmm_sk_f64<TM, TN, WIDE>), grid, block, 0, s, g, A, lda, B, ldb, C, ldc, parts);
     hipLaunchKernelGGL((k_sk_fixup<TM, TN>), dim3((unsigned)sk_launch(g), 4), dim3(256), 0, s, g, parts, C, ldc);
 }
 
@@ -792,12 +816,11 @@ uvt_status uvt_launch_trapezoid_sk_f64(int32_t cfg, int64_t n, int64_t m, const 
                                        int64_t workgroups, double* parts, hipStream_t s)
 {
     if (n <= 0 || m <= 0 || lda < n || ldb < m || ldc < m || workgroups <= 0 || !parts) return UVT_ERR_ARG;
-    if (cfg == UVT_CFG_256x128) return UVT_ERR_ARG;  // stream-K runs 128x128 tiles (uvt_sk_workgroups)
+    if (cfg != UVT_CFG_128x128) return UVT_ERR_ARG;  // stream-K runs 128x128 tiles (uvt_sk_workgroups)
     if (n > 0x3FFFFFFF || m > 0x3FFFFFFF || workgroups > 0x7FFFFFFF) return UVT_ERR_SIZE;
     const SkGeo g = sk_geometry(n, m, uvt_cfg_tile_m(cfg), uvt_cfg_tile_n(cfg), workgroups, kSkGroupCols);
-    if (cfg == UVT_CFG_64x64) launch_trapezoid_sk<64, 64>(g, A, lda, B, ldb, C, ldc, parts, s);
-    else if (cfg == UVT_CFG_128x32) launch_trapezoid_sk<128, 32>(g, A, lda, B, ldb, C, ldc, parts, s);
-    else launch_trapezoid_sk<128, 128>(g, A, lda, B, ldb, C, ldc, parts, s);
+    if (full_panels_fit(cfg, lda, ldb)) launch_trapezoid_sk<128, 128, false>(g, A, lda, B, ldb, C, ldc, parts, s);
+    else launch_trapezoid_sk<128, 128, true>(g, A, lda, B, ldb, C, ldc, parts, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }

@@ -138,12 +138,22 @@ struct Panel {
     // operand without a triangle loads a panel inside the range as in the
     // steady state, so beside the diagonal only the triangle's own panels go
     // element by element.
-    template <bool TRI, bool GE>
+    template <bool TRI, bool GE, bool WIDE>
     __device__ __forceinline__ void load_masked(int tid, int k0, int k_lo, int k_hi, bool tri)
     {
         if (!(TRI && tri) && Idx::inside(k0, k_lo, k_hi, nx, ld)) {
             seek(k0);
             load(tid);
+            return;
+        }
+        if (WIDE && Idx::whole(k0, k_lo, k_hi, nx) && (!(TRI && tri) || Idx::template clear<GE>(k0, x0, nx))) {
+#pragma unroll
+            for (int q = 0; q < VEC; ++q) {
+                const int v = tid + q * NT;
+                if (PART && v >= PIECES) break;
+                const int64_t x = Idx::full_x(v, nx), k = k0 + Idx::pk(v);
+                r[q] = *reinterpret_cast<const UVT_GLOBAL dbl2u*>(p + (KC ? x * ld + k : k * ld + x));
+            }
             return;
         }
 #pragma unroll
@@ -173,11 +183,11 @@ struct Panel {
 
     // The panel at k0 with zeros outside [k_lo, k_hi) and outside the
     // triangle, and (UNIT) ones on its diagonal.
-    template <bool TRI, bool GE, bool UNIT>
+    template <bool TRI, bool GE, bool UNIT, bool WIDE>
     __device__ __forceinline__ void store_masked(int tid, double* s, int k0, int k_lo, int k_hi, bool tri,
                                                  bool unit) const
     {
-        if (!(TRI && tri) && k0 >= k_lo && k0 + kTileK <= k_hi) {
+        if ((!(TRI && tri) || (WIDE && Idx::template clear<GE>(k0, x0, nx))) && k0 >= k_lo && k0 + kTileK <= k_hi) {
             store(tid, s);
             return;
         }
@@ -219,11 +229,15 @@ enum TriKind {
 // without; 9000 x 250 in cut tiles 395 and 387; 512 problems in a batch, from
 // one queue, 9.08 and 8.95 ms); the plain walks are faster with it (4096^2:
 // 992 us, 1004 without).
+// WIDE: an operand has rows too long for full panels (PanelIdx::offsets_fit);
+// panels that no mask touches are then loaded with 64-bit addresses, not
+// element by element.  A kernel of its own: in the others the extra branch
+// costs registers (short batch tiles 4 % slower, dtrmm on the right 3-5 %).
 template <bool A_KC_ = true, bool B_KC_ = false, TriKind TRI_ = kTriALe, bool UNIT_ = false, bool EPI_ = false,
-          bool EDGE_IDLE_ = true, bool PIPE_MASKED_ = true>
+          bool EDGE_IDLE_ = true, bool PIPE_MASKED_ = true, bool WIDE_ = false>
 struct TileOpt {
     static constexpr bool A_KC = A_KC_, B_KC = B_KC_, UNIT = UNIT_, EPI = EPI_, EDGE_IDLE = EDGE_IDLE_,
-                          PIPE_MASKED = PIPE_MASKED_;
+                          PIPE_MASKED = PIPE_MASKED_, WIDE = WIDE_;
     static constexpr TriKind TRI = TRI_;
     static constexpr bool TRI_A = TRI == kTriALe || TRI == kTriAGe, GE = TRI == kTriAGe || TRI == kTriBGe;
 };
@@ -307,8 +321,8 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
             pa.load(tid);  // panels of the steady state follow each other: see seek()
             pb.load(tid);
         } else {
-            pa.template load_masked<TRI_A, GE>(mtid, k0, k_lo, k_hi, tri);
-            pb.template load_masked<!TRI_A, GE>(mtid, k0, k_lo, k_hi, tri);
+            pa.template load_masked<TRI_A, GE, OPT::WIDE>(mtid, k0, k_lo, k_hi, tri);
+            pb.template load_masked<!TRI_A, GE, OPT::WIDE>(mtid, k0, k_lo, k_hi, tri);
         }
     };
     auto store = [&](int buf, int k0, auto full_tag) {
@@ -318,8 +332,8 @@ __device__ __forceinline__ void f64_tile(const TileArgs& t, const UVT_GLOBAL dou
             pa.store(tid, as);
             pb.store(tid, bs);
         } else {
-            pa.template store_masked<TRI_A, GE, UNIT && TRI_A>(mtid, as, k0, k_lo, k_hi, tri, unit);
-            pb.template store_masked<!TRI_A, GE, UNIT && !TRI_A>(mtid, bs, k0, k_lo, k_hi, tri, unit);
+            pa.template store_masked<TRI_A, GE, UNIT && TRI_A, OPT::WIDE>(mtid, as, k0, k_lo, k_hi, tri, unit);
+            pb.template store_masked<!TRI_A, GE, UNIT && !TRI_A, OPT::WIDE>(mtid, bs, k0, k_lo, k_hi, tri, unit);
         }
     };
 

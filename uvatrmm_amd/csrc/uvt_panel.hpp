@@ -50,10 +50,21 @@ struct PanelIdx {
         return ld <= (int64_t)(0xFFFFFFFFu / (8u * (KC ? X : kTileK))) - 1;
     }
     // Whether the panel at k0 lies wholly inside [k_lo, k_hi) and may be read
-    // as a full one.
+    // as a full one (whole: with 64-bit addresses).
+    static __host__ __device__ bool whole(int k0, int k_lo, int k_hi, int nx)
+    {
+        return k0 >= k_lo && k0 + kTileK <= k_hi - (!KC && (nx & 1) ? 1 : 0);
+    }
     static __host__ __device__ bool inside(int k0, int k_lo, int k_hi, int nx, int64_t ld)
     {
-        return k0 >= k_lo && k0 + kTileK <= k_hi - (!KC && (nx & 1) ? 1 : 0) && offsets_fit(ld);
+        return whole(k0, k_lo, k_hi, nx) && offsets_fit(ld);
+    }
+    // Whether it lies off the diagonal of the triangle (GE: k >= x, else k <=
+    // x) whose x run from x0 on, nx of them.
+    template <bool GE>
+    static __host__ __device__ bool clear(int k0, int x0, int nx)
+    {
+        return GE ? k0 >= x0 + nx : k0 + kTileK <= x0;
     }
 };
 
