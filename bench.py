@@ -459,7 +459,7 @@ def configs_leg(args, h, uvt):
         log(f"config N={n} {mp} {shape} P={p}: {ms:.3f} ms, {tf:.2f} TFLOP/s")
         out.append({"workload": f"trmm_f64 N=M={n} {mp} {shape} P={p}", "ms": round(ms, 4),
                     "tflops": round(tf, 4), "frac": round(tf / FP64_PEAK_TFLOPS, 4),
-                    "phases": plan.phases})
+                    "launches": 2 if h.plan_launch_info(plan)[1] else 1})
         plan.close()
         for b in (dA, dB, dC):
             b.free()
@@ -537,8 +537,8 @@ def main():
     plan = uvt.Plan(n, m, args.bands, args.map, args.shape)
     flops = plan.flops
     h.sync()
-    log(f"plan: {plan.phases} launch(es), tiles={[len(plan.tiles(p)) for p in range(plan.phases)]}, "
-        f"issued/algorithmic={plan.issued_flops / flops:.4f}")
+    wg, parts = h.plan_launch_info(plan)
+    log(f"plan: {wg} workgroups, {parts} partial tiles, issued/algorithmic={plan.issued_flops / flops:.4f}")
     for _ in range(args.warmup):
         h.trmm_f64(plan, dA, n, dB, m, dC, m)
     h.sync()
@@ -622,9 +622,8 @@ def main():
         except Exception as e:  # the baseline is reported, never the measured path
             log("cpu baseline failed:", repr(e))
 
-    # the kernels this plan runs on this GPU (whole tiles, stream-K, or cut reductions)
-    wg, parts = h.plan_launch_info(plan)
-    cfg0 = int(plan.tiles(0)["cfg"][0]) if len(plan.tiles(0)) else 0
+    # the kernels this plan runs on this GPU (whole tiles, stream-K, cut reductions, or waves)
+    cfg0 = int(plan.tiles(0)["cfg"][0])
     tile, waves = {0: ("128,128", "8 waves of 32x64"), 1: ("64,64", "4 waves of 32x32"),
                    2: ("128,32", "4 waves of 32x32"), 4: ("256,128", "16 waves of 32x64")}[cfg0]
     launches = 1
@@ -634,8 +633,10 @@ def main():
     elif parts:
         kernel = f"k_trmm_tiles_f64<{tile}> ({waves}; reductions cut into pieces) + k_add_parts"
         launches = 2
-    else:
+    elif wg == -(-n // plan.tile_shape()[0]) * -(-m // plan.tile_shape()[1]):
         kernel = f"k_trmm_tiles_f64<{tile}> ({waves})"
+    else:
+        kernel = f"k_trmm_waves_f64 ({wg} workgroups of 4 tiles, one wave each)"
     out = {
         "metric": "TRMM TFLOP/s + % MFMA peak at N=32768 (plain FP64 = value; split in 'split')",
         "value": round(value, 4),

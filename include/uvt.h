@@ -123,7 +123,9 @@ uvt_status uvt_plan_get_bands(uvt_plan plan, uvt_range *out, uint32_t cap);
 uvt_status uvt_plan_tile_shape(uvt_plan plan, int32_t *tile_m, int32_t *tile_n);
 /* Algorithmic flops m*n^2 (LAWN 41 count for a left triangular product). */
 double uvt_plan_flops(uvt_plan plan);
-/* MFMA flops actually issued, including masked diagonal tiles and padding. */
+/* MFMA flops a launch issues with operands of ordinary leading dimensions,
+ * including masked diagonal tiles and padding (those of the tiles it runs,
+ * whatever the plan's list). */
 double uvt_plan_issued_flops(uvt_plan plan);
 
 /* ------------------------------------------------------------------ */

@@ -904,6 +904,23 @@ extern "C" uvt_status uvt_trmm_f64(uvt_handle h, uvt_plan plan, const double* dA
     return UVT_OK;
 }
 
+// Of the tiles a launch runs (waves or the trapezoid walk; cut reductions are
+// cut at whole panels), not of the plan's list.
+extern "C" double uvt_plan_issued_flops(uvt_plan plan)
+{
+    if (!plan) return 0.0;
+    const int shape = uvt_wave_shape(plan->n, plan->m, plan->n, plan->m);
+    int64_t tm = uvt_cfg_tile_m(plan->cfg), tn = uvt_cfg_tile_n(plan->cfg);
+    if (shape && !deep_and_narrow(*plan)) {
+        tm = 16 * (shape / 10);
+        tn = 16 * (shape % 10);
+    }
+    double s = 0.0;
+    for (int64_t r0 = 0; r0 < plan->n; r0 += tm)
+        s += (double)((std::min(r0 + tm, plan->n) + kTileK - 1) / kTileK * kTileK);
+    return 2.0 * (double)tm * s * (double)((plan->m + tn - 1) / tn * tn);
+}
+
 extern "C" uvt_status uvt_plan_launch_info(uvt_handle h, uvt_plan plan, int64_t* workgroups,
                                            int64_t* partial_tiles)
 {

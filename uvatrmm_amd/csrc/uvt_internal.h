@@ -36,7 +36,7 @@ struct uvt_plan_s {
     int32_t phases;
     int64_t ntiles[2];
     uvt_tile *tiles[2];
-    double flops, issued;
+    double flops;
     /* device state, owned by the plan, created by the HIP side on first use
      * on a device: the launch's records, and, when tiles write partial
      * products, the partial tiles and the records that add them to C */

@@ -257,19 +257,6 @@ int64_t uvt_plan_trapezoid_tiles(int64_t n, int64_t m, int32_t cfg, uvt_tile *ou
     return c;
 }
 
-static double issued_flops(const uvt_tile *v, int64_t len)
-{
-    double s = 0;
-    for (int64_t i = 0; i < len; i++) {
-        int32_t tm = uvt_cfg_tile_m(v[i].cfg), tn = uvt_cfg_tile_n(v[i].cfg);
-        int64_t klo = v[i].k_lo & ~(int64_t)1; /* the kernels align k down to even */
-        int64_t kl = v[i].k_hi - klo;
-        int64_t kpad = (kl + 15) / 16 * 16; /* 16-deep k panels */
-        s += 2.0 * tm * tn * (double)kpad;
-    }
-    return s;
-}
-
 uvt_status uvt_plan_create(int64_t n, int64_t m, uint32_t p, uvt_map map, uvt_shape shape,
                            uvt_plan *out, int *ref_exit)
 {
@@ -346,7 +333,6 @@ uvt_status uvt_plan_create(int64_t n, int64_t m, uint32_t p, uvt_map map, uvt_sh
         pl->ntiles[ph] = tv[ph].len;
     }
     pl->flops = (double)m * (double)n * (double)n;
-    pl->issued = issued_flops(pl->tiles[0], pl->ntiles[0]) + issued_flops(pl->tiles[1], pl->ntiles[1]);
     *out = pl;
     return UVT_OK;
 }
@@ -396,4 +382,3 @@ uvt_status uvt_plan_tile_shape(uvt_plan plan, int32_t *tile_m, int32_t *tile_n)
 }
 
 double uvt_plan_flops(uvt_plan plan) { return plan ? plan->flops : 0.0; }
-double uvt_plan_issued_flops(uvt_plan plan) { return plan ? plan->issued : 0.0; }
