@@ -271,8 +271,11 @@ uvt_status uvt_batch_create(uvt_handle h, const uvt_problem *probs, int32_t coun
                             const char *tune_table, uvt_batch *out);
 /* One hipGraphLaunch of the whole batch on `stream`. */
 uvt_status uvt_batch_run(uvt_batch b, void *stream);
-/* New pointers for the same shapes and precisions (descriptors live in
- * device memory, so the captured graph picks them up); synchronous. */
+/* New pointers and leading dimensions for the same shapes, precisions and
+ * routes (descriptors live in device memory, so the captured graph picks them
+ * up); synchronous.  A problem whose A and B both lay at 16-byte aligned
+ * addresses with even leading dimensions keeps that, and one whose did not
+ * does not gain it: UVT_ERR_ARG otherwise, and the batch stays as it was. */
 uvt_status uvt_batch_update(uvt_batch b, const uvt_problem *probs, int32_t count);
 /* Algorithmic flops (sum of m n^2), the part of them whose box runs on the
  * int8 path (see uvt_problem.route), FP64 tiles queued, graph nodes.  Any

@@ -48,7 +48,7 @@ struct BatchProb {
     const double* B;
     double* C;
     int64_t lda, ldb, ldc, m;
-    int32_t vec, pad;
+    int32_t pad;  // 0 (see k_batch_f64)
 };
 
 // Persistent FP64 tile kernel for every tile shape: every workgroup (8
@@ -335,10 +335,15 @@ static BatchProb f64_desc(const uvt_problem& p)
     d.ldb = p.ldb;
     d.ldc = p.ldc;
     d.m = p.m;
-    d.vec = ((uintptr_t)p.A % 16 == 0) && ((uintptr_t)p.B % 16 == 0) && p.lda % 2 == 0 &&
-            p.ldb % 2 == 0;
     d.pad = 0;
     return d;
+}
+
+// Whether A and B could be read in aligned 16-byte pairs throughout.  No kernel
+// asks any more; uvt_batch_update holds new operands to it (uvt.h).
+static bool even_aligned(const uvt_problem& p)
+{
+    return (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.B % 16 == 0 && p.lda % 2 == 0 && p.ldb % 2 == 0;
 }
 
 static uvt_status upload_split(uvt_batch b)
@@ -496,8 +501,7 @@ extern "C" uvt_status uvt_batch_update(uvt_batch b, const uvt_problem* probs, in
         if (p.n != q.n || p.m != q.m || p.prec != q.prec || p.route != q.route) return UVT_ERR_ARG;
         uvt_status st = check(p);
         if (st != UVT_OK) return st;
-        // operands keep the alignment they were planned with
-        if (f64_desc(p).vec != b->f64_probs[b->f64_index[i]].vec) return UVT_ERR_ARG;
+        if (even_aligned(p) != even_aligned(q)) return UVT_ERR_ARG;
     }
     UVT_HIP(hipSetDevice(b->h->device));
     UVT_HIP(hipDeviceSynchronize());
