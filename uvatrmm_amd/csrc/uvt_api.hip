@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void k_trmm_waves_f64(int64_t n, int64_t m, in
                                                         double* __restrict__ C, int64_t ldc)
 {
     int b = (int)blockIdx.x;
-    const int g = snake > 0 ? b / snake : 0;
+    const int g = b / snake;
     if (g & 1) b = g * snake + min((g + 1) * snake, (int)gridDim.x) - 1 - b;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int rt = (nrt - 1 - b / nct) * (4 / wn) + wave / wn, ct = b % nct * wn + wave % wn;

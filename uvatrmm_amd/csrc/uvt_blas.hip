@@ -196,8 +196,9 @@ uvt_status launch_blas(int32_t cfg, const Walk& g, const double* A, int64_t lda,
     if (cfg == UVT_CFG_64x64) launch_walk<64, 64, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
     else if (cfg == UVT_CFG_128x32)
         launch_walk<kRight ? 32 : 128, kRight ? 128 : 32, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
-    else if (cfg == UVT_CFG_256x128) launch_walk<256, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
-    else launch_walk<128, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    else if (cfg == UVT_CFG_128x128) launch_walk<128, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
+    else if constexpr (TRI != kTriNone)  // uvt_wide_tiles
+        launch_walk<256, 128, A_KC, B_KC, TRI>(g, A, lda, B, ldb, C, ldc, epi, s);
     UVT_HIP(hipGetLastError());
     return UVT_OK;
 }
