@@ -695,10 +695,10 @@ int uvt_wave_shape(int64_t n, int64_t m, int64_t lda, int64_t ldb)
     if (n > 32768 || tiles > 13000 || flops >= (tiles > 7500 ? 8e9 : 6e9)) return 0;
     if (tiles <= 2500) return 11;
     if (tiles <= 7500 || n < 512) return 12;
-    // Without full panels (rows of 64 MB or longer) 32x32 tiles lose: 1500 x
+    // Without full panels (rows of 128 MB or longer) 32x32 tiles lose: 1500 x
     // 1500 220 us, 136 in workgroup tiles; smaller tiles do not: 1024 x 400 40
     // and 82, 1200 x 1200 79 and 97.
-    return WaveOperand<2, true, false>::fits(lda) && WaveOperand<2, false, false>::fits(ldb) ? 22 : 0;
+    return WaveIdx<2, true>::fits(lda) && WaveIdx<2, false>::fits(ldb) ? 22 : 0;
 }
 
 namespace {

@@ -26,22 +26,18 @@ namespace uvt {
 // F blocks of 16 rows of op(A) (columns of op(B)) as one wave's MFMA operand.
 template <int F, bool KC, bool DOWN>
 struct WaveOperand {
-    static constexpr bool PAIR = !KC && F == 2;  // blocks on alternate columns
-    static constexpr int LOADS = KC ? 2 * F : 4;
-    static constexpr int OFFS = LOADS;
-    static constexpr int PITCH = kTileK + 2;  // LDS row of a k-contiguous operand (see Panel)
-    static constexpr int LDS = KC ? 2 * 16 * F * PITCH : 0;  // doubles: two panels
+    using Idx = WaveIdx<F, KC>;
+    static constexpr bool PAIR = Idx::PAIR;
+    static constexpr int LOADS = Idx::LOADS;
+    static constexpr int SLOT = 16 * F * Idx::PITCH;   // a panel in LDS
+    static constexpr int LDS = KC ? 2 * SLOT : 0;      // doubles: two panels
 
     const UVT_GLOBAL double* p;  // element (x0, k = 0)
     int64_t ld;
     int nx, x0, lane;
     double* lds;
     const UVT_GLOBAL char* at;  // the full panel load() reads next
-    uint32_t off[OFFS];         // byte offsets of this lane's loads in it
-
-    // Offsets fit 32 bits: else (rows of 128 MB or longer) there are no full
-    // panels, and the host takes workgroup tiles where it can.
-    static __host__ __device__ bool fits(int64_t ld) { return ld < (int64_t)(0xFFFFFFFFu / (8u * 16 * F)) - 16; }
+    uint32_t off[LOADS];        // byte offsets of this lane's loads in it
 
     __device__ __forceinline__ void init(const UVT_GLOBAL double* p_, int64_t ld_, int nx_, int x0_, double* lds_)
     {
@@ -52,22 +48,13 @@ struct WaveOperand {
         lds = lds_;
         lane = threadIdx.x & 63;
 #pragma unroll
-        for (int q = 0; q < OFFS; ++q) {
-            uint32_t x, k;
-            if (KC) {
-                const int row = 8 * q + (lane >> 3);
-                x = (uint32_t)(row < nx ? row : nx - 1);
-                k = 2 * (lane & 7);
-            } else {
-                const int col = PAIR ? 2 * (lane & 15) : lane & 15, last = PAIR ? (nx - 1) & ~1 : nx - 1;
-                x = (uint32_t)(col < last ? col : last);
-                k = 4 * (lane >> 4) + q;
-            }
+        for (int q = 0; q < LOADS; ++q) {
+            const uint32_t x = (uint32_t)Idx::load_x(q, lane, nx), k = (uint32_t)Idx::load_k(q, lane);
             off[q] = 8u * (KC ? x * (uint32_t)ld + k : k * (uint32_t)ld + x);
         }
     }
     // This lane's row (column) of block f.
-    __device__ __forceinline__ int row(int f) const { return PAIR ? 2 * (lane & 15) + f : 16 * f + (lane & 15); }
+    __device__ __forceinline__ int row(int f) const { return Idx::row(f, lane); }
     __device__ __forceinline__ void seek(int k0)
     {
         at = reinterpret_cast<const UVT_GLOBAL char*>(KC ? p + k0 : p + (int64_t)k0 * ld);
@@ -96,19 +83,17 @@ struct WaveOperand {
     __device__ __forceinline__ void fragments(const double (&r)[4 * F], int slot, double (&v)[F][4])
     {
         if constexpr (KC) {
-            double* s = lds + slot * (16 * F * PITCH);
+            double* s = lds + slot * SLOT;
 #pragma unroll
-            for (int q = 0; q < 2 * F; ++q)
-                *reinterpret_cast<dbl2*>(&s[(8 * q + (lane >> 3)) * PITCH + 2 * (lane & 7)]) =
-                    dbl2{r[2 * q], r[2 * q + 1]};
+            for (int q = 0; q < LOADS; ++q)
+                *reinterpret_cast<dbl2*>(&s[Idx::lds_write(q, lane)]) = dbl2{r[2 * q], r[2 * q + 1]};
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int f = 0; f < F; ++f)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const dbl2 w =
-                        *reinterpret_cast<const dbl2*>(&s[(16 * f + (lane & 15)) * PITCH + 4 * (lane >> 4) + 2 * h]);
+                    const dbl2 w = *reinterpret_cast<const dbl2*>(&s[Idx::lds_read(f, h, lane)]);
                     v[f][2 * h] = w.x;
                     v[f][2 * h + 1] = w.y;
                 }
@@ -181,7 +166,7 @@ __device__ __forceinline__ void f64_wave(const TileArgs& t, const UVT_GLOBAL dou
     const int tx0 = TRI_A ? t.r0 : t.c0, tx1 = tx0 + (TRI_A ? t.rows : cols) - 1;
     const bool odd = (OA::PAIR && (t.rows & 1)) || (OB::PAIR && (cols & 1));
     const FullPanels fp = full_panels<GE>(k_lo, k_hi, tri, unit, tx0, tx1, odd);
-    const int f0 = fp.f0, f1 = fp.f1 > f0 && OA::fits(lda) && OB::fits(ldb) ? fp.f1 : f0;
+    const int f0 = fp.f0, f1 = fp.f1 > f0 && OA::Idx::fits(lda) && OB::Idx::fits(ldb) ? fp.f1 : f0;
 
     OA pa;
     OB pb;

@@ -68,6 +68,37 @@ struct PanelIdx {
     }
 };
 
+// The same for the tile of a single wave (uvt_f64_wave.hpp), whose operand is F
+// blocks of 16 rows (columns).  A load of a full panel takes a pair along k (KC:
+// 8 lanes on the 128 bytes of a row), a pair along x (PAIR: two blocks on
+// alternate columns) or one element; the pairs along k are turned round through
+// LDS rows of PITCH doubles.  Lane l's fragment of block f for MFMA step s is row
+// row(f, l), k = 4 (l / 16) + s.
+template <int F, bool KC>
+struct WaveIdx {
+    static constexpr bool PAIR = !KC && F == 2;
+    static constexpr int LOADS = KC ? 2 * F : 4;
+    static constexpr int PITCH = kTileK + 2;
+    // x and k of load q (of its first element), with nx rows inside the matrix.
+    static __host__ __device__ int load_x(int q, int lane, int nx)
+    {
+        const int x = KC ? 8 * q + (lane >> 3) : PAIR ? 2 * (lane & 15) : lane & 15;
+        const int last = PAIR ? (nx - 1) & ~1 : nx - 1;
+        return x < last ? x : last;
+    }
+    static __host__ __device__ int load_k(int q, int lane) { return KC ? 2 * (lane & 7) : 4 * (lane >> 4) + q; }
+    static __host__ __device__ int row(int f, int lane) { return PAIR ? 2 * (lane & 15) + f : 16 * f + (lane & 15); }
+    // Where in LDS load q's pair goes, and pair h of block f's fragment lies (KC).
+    static __host__ __device__ int lds_write(int q, int lane) { return (8 * q + (lane >> 3)) * PITCH + 2 * (lane & 7); }
+    static __host__ __device__ int lds_read(int f, int h, int lane)
+    {
+        return (16 * f + (lane & 15)) * PITCH + 4 * (lane >> 4) + 2 * h;
+    }
+    // Offsets of a full panel fit 32 bits for every matrix but one whose rows
+    // are 256 MB (F = 2: 128 MB) or longer; such a tile has no full panels.
+    static __host__ __device__ bool fits(int64_t ld) { return ld < (int64_t)(0xFFFFFFFFu / (8u * 16 * F)) - 16; }
+};
+
 // The k another panel reads element (x, k) at, x inside the matrix: the
 // nearest below k_hi and, with tri, in the triangle (GE: k >= x, else k <= x).
 template <bool GE>
