@@ -39,6 +39,66 @@ def run(gpu, uvt, n, m, shape, pads):
     return launch
 
 
+def waves(n, m, tm, tn):
+    """Workgroups of four one-wave tiles, two along the columns where there are
+    two."""
+    rt, ct = -(-n // tm), -(-m // tn)
+    wn = 2 if ct > 1 else 1
+    return -(-rt // (4 // wn)) * -(-ct // wn)
+
+
+@pytest.mark.parametrize("n,m,shape,form,tm,tn", [
+    (1023, 31, "boxes", "waves", 16, 16),
+    (1023, 701, "trapezoid", "waves", 16, 32),
+    (1301, 2003, "boxes", "waves", 32, 32),
+    (769, 4001, "trapezoid", "waves", 32, 32),
+    (2049, 1999, "boxes", "tiles", 64, 64),
+    (2177, 2111, "trapezoid", "tiles", 64, 64),
+    (5001, 301, "boxes", "cut", 64, 64),
+    (9001, 33, "trapezoid", "cut", 128, 32),
+    (1301, 8001, "boxes", "tiles", 128, 128),
+    (5001, 1711, "boxes", "stream-k", 128, 128),
+])
+def test_each_form_with_poisoned_surroundings(gpu, uvt, n, m, shape, form, tm, tn):
+    wg, parts = run(gpu, uvt, n, m, shape, ((0, 0), (1, 1), (2, 3)) if n < 4000 else ((1, 1),))
+    if form == "waves":
+        assert (wg, parts) == (waves(n, m, tm, tn), 0)
+    elif form == "tiles":
+        assert (wg, parts) == (tiles(n, m, tm, tn), 0)
+    elif form == "cut":
+        assert parts > 0 and wg == tiles(n, m, tm, tn) + parts
+    else:
+        assert parts > 0 and wg <= 2 * gpu.cus and wg > 2 * gpu.cus - tiles(1, m, tm, tn)
+
+
+def test_whole_narrow_tiles(gpu, uvt):
+    """128x32 tiles are run whole only past n = 32768 and under 2e9 flops: a
+    triangle of 8.7 GB, zero but for some rows, with NaN above their diagonal."""
+    n, m, ld = 33001, 1, 33003
+    rng = np.random.default_rng(9)
+    rows = np.unique(np.concatenate([[0, 1, 15, 16, 127, 128, 129, n - 129, n - 2, n - 1], rng.integers(0, n, 60)]))
+    B = rng.integers(-2, 3, (n, m)).astype(np.float64)
+    want = np.zeros((n, m))
+    dA, dB, dC = gpu.alloc(n * ld * 8), gpu.array(B), gpu.array(np.full((n, m), np.nan))
+    dA.zero()
+    L = uvt.lib()
+    for r in rows:
+        a = np.full(ld, np.nan)
+        a[:r + 1] = rng.integers(-2, 3, r + 1)
+        want[r] = a[:r + 1] @ B[:r + 1]
+        assert L.uvt_memcpy(gpu.ptr, dA.ptr + int(r) * ld * 8, a.ctypes.data, ld * 8, 0) == 0
+    plan = uvt.Plan(n, m)
+    print("[gpu-plan-forms]", n, m, gpu.plan_launch_info(plan), flush=True)
+    assert gpu.plan_launch_info(plan) == (tiles(n, m, 128, 32), 0)
+    gpu.trmm_f64(plan, dA, ld, dB, m, dC, m)
+    gpu.sync()
+    got = dC.download((n, m))
+    plan.close()
+    for b in (dA, dB, dC):
+        b.free()
+    np.testing.assert_array_equal(got, want)
+
+
 @pytest.mark.parametrize("n,m", [(7000, 19), (7001, 41), (9000, 31), (7003, 101), (27000, 3)])
 def test_deep_narrow_plans_cut_their_reductions(gpu, uvt, n, m):
     """From n = 7000 to 27000, of 2e9 flops or more (m > 40 at n = 7000): else
