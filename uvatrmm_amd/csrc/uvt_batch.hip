@@ -566,17 +566,22 @@ extern "C" uvt_status uvt_tune_choice(const char* tune_table, int64_t n, int64_t
 
 // ---- autotuner -----------------------------------------------------------------
 
-// For every (n, m) bucket, a batch of copies of one problem at the bucket's
-// upper edge (enough to fill the GPU, as a mixed batch does) is timed with
-// each tile shape (persistent kernel, best of three runs); the fastest shape
-// is the bucket's entry.
+// For every (n, m) bucket, a batch of problems of the bucket's upper edge (enough
+// to fill the GPU, as a mixed batch does) is timed with each tile shape
+// (persistent kernel, best of three runs); the fastest shape is the bucket's
+// entry.  Every problem has a B and a C of its own, and the triangles take
+// turns over kTunePool bytes, so that none is read from a cache because another
+// problem has just used it: narrow problems are bound by those reads (4096 of
+// 512 x 16 take 0.62 ms with one A and one B for all, 1.13 ms with their own).
+// Up to 32 columns 128x128 makes the same tiles as 128x32, which is timed for
+// both.
+constexpr size_t kTunePool = (size_t)4 << 30;
 extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
 {
     if (!h || !out_path) return UVT_ERR_ARG;
     UVT_HIP(hipSetDevice(h->device));
     const int64_t ns[] = {64, 128, 256, 512, 1024, 2048, 4096};
     const int64_t ms[] = {16, 32, 64, 128, 256, 512, 1024};
-    const int64_t nmax = 4096, mmax = 1024;
     double *A = nullptr, *B = nullptr, *C = nullptr;
     int* counter = nullptr;
     BatchProb* dprobs = nullptr;
@@ -584,17 +589,17 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
     hipStream_t s = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     // Enough copies of a bucket's problem to keep every CU busy the way a
-    // mixed batch does (~1.2e11 flops), within a 1 GiB C buffer.
+    // mixed batch does (~1.2e11 flops), within 1 GiB of B and of C.
     const int max_copies = 4096;
     const size_t c_bytes = (size_t)1 << 30;
+    const int64_t pool = (int64_t)(kTunePool / sizeof(double)), cn = (int64_t)(c_bytes / sizeof(double));
     uvt_status st = UVT_OK;
     std::string json = "{\n  \"version\": 1,\n  \"device\": \"gfx950\",\n  \"what\": \"FP64 tile shape per (n, m) bucket, chosen by timing\",\n  \"table\": [\n";
     auto fail = [&](uvt_status e) {
         st = e;
         return e;
     };
-    if (hipMalloc(&A, (size_t)nmax * nmax * 8) != hipSuccess ||
-        hipMalloc(&B, (size_t)nmax * mmax * 8) != hipSuccess ||
+    if (hipMalloc(&A, kTunePool) != hipSuccess || hipMalloc(&B, c_bytes) != hipSuccess ||
         hipMalloc(&C, c_bytes) != hipSuccess ||
         hipMalloc(&counter, kCounters * sizeof(int)) != hipSuccess ||
         hipMalloc(&dprobs, max_copies * sizeof(BatchProb)) != hipSuccess ||
@@ -603,7 +608,9 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
         (void)hipGetLastError();
         fail(UVT_ERR_NOMEM);
     }
-    if (st == UVT_OK) st = uvt_fill_seeded(h, nmax, mmax, 7, 0, A, nmax, B, mmax, s);
+    // filled as wide matrices of B values: nothing is above a diagonal
+    if (st == UVT_OK) st = uvt_fill_seeded(h, pool >> 15, 1 << 15, 7, 0, nullptr, 0, A, 1 << 15, s);
+    if (st == UVT_OK) st = uvt_fill_seeded(h, cn >> 15, 1 << 15, 8, 0, nullptr, 0, B, 1 << 15, s);
     bool first = true;
     for (int64_t n : ns) {
         for (int64_t m : ms) {
@@ -612,7 +619,9 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
             while (copies > 1 && (size_t)copies * n * m * 8 > c_bytes) --copies;
             std::vector<BatchProb> hp(copies);
             for (int c = 0; c < copies; ++c) {
-                uvt_problem p = {A, nmax, B, mmax, C + (size_t)c * n * m, m, n, m, UVT_PREC_F64, 0};
+                const size_t own = (size_t)c * n * m;
+                uvt_problem p = {A + (size_t)(c % (pool / (n * n))) * n * n, n, B + own, m, C + own, m, n, m,
+                                 UVT_PREC_F64, 0};
                 hp[c] = f64_desc(p);
             }
             if (hipMemcpy(dprobs, hp.data(), copies * sizeof(BatchProb), hipMemcpyHostToDevice) != hipSuccess) {
@@ -624,6 +633,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
             float best_ms = 1e30f;
             float per_cfg[UVT_NUM_CFGS] = {0, 0, 0};
             for (int cfg = 0; cfg < UVT_NUM_CFGS; ++cfg) {
+                if (cfg == UVT_CFG_128x128 && m <= 32) continue;
                 std::vector<BatchTile> tiles;
                 for (int c = 0; c < copies; ++c) trapezoid_tiles(c, n, m, cfg, tiles);
                 const TileQueues queues = deal_tiles(tiles, grid, tile_work);
@@ -654,6 +664,7 @@ extern "C" uvt_status uvt_autotune_f64(uvt_handle h, const char* out_path)
                 }
             }
             if (st != UVT_OK) break;
+            if (m <= 32) per_cfg[UVT_CFG_128x128] = per_cfg[UVT_CFG_128x32];
             char line[512];
             const double fl = (double)m * n * n * copies;
             snprintf(line, sizeof line,
