@@ -106,7 +106,8 @@ typedef struct {
 } uvt_tile;
 #define UVT_TILE_256x128 4 /* 256 x 128 tiles (not selectable per batch problem) */
 #define UVT_TILE_LOWER 1 /* A[i][k] is treated as 0 for k > i */
-#define UVT_TILE_ACCUM 2 /* C += product (else C = product) */
+#define UVT_TILE_ACCUM 2 /* in a boxes plan's list: the triangle's part of a row the box
+                          * part came before; no launch accumulates into C */
 
 /* Plans C = tril(A) * B for an n x n A and n x m B over p bands of the given
  * mapping and shape.  Errors as uvt_plan_bands. */
@@ -141,9 +142,9 @@ int32_t uvt_device_cus(uvt_handle h);
  * written; C is fully overwritten on rows [0, n) x columns [0, m)).  Entries
  * of A above the diagonal are never read.  The kernels multiply whole
  * 16-deep k panels of B, so a NaN or infinity in B[k][j] also reaches the
- * rows above k in k's 128-row tile through A's structural zeros (0 * Inf =
- * NaN), where a BLAS dtrmm would leave them finite; finite inputs are not
- * affected.  Small products (at most 13000 16x16 tiles of C, under 6e9 to 8e9
+ * rows above k in the row tile the product runs in (16 to 256 rows, by size)
+ * through A's structural zeros (0 * Inf = NaN), where a BLAS dtrmm would
+ * leave them finite; finite inputs are not affected.  Small products (at most 13000 16x16 tiles of C, under 6e9 to 8e9
  * flops; of n from 7000 to 27000, under 2e9) run as one wave per tile and
  * keep nothing on the device; for others the plan allocates its launch records
  * there on its first use on a device.
@@ -261,8 +262,8 @@ enum { UVT_ROUTE_AUTO = 0, UVT_ROUTE_INT8 = 1, UVT_ROUTE_FP64 = 2 };
 
 typedef struct uvt_batch_s *uvt_batch;
 
-/* Plans a batch: the tiles of the FP64 problems become one queue per XCD,
- * drained by a persistent kernel (tile shape per problem from the tuning
+/* Plans a batch: the tiles of the FP64 problems become one queue per XCD and
+ * one that all share, drained by a persistent kernel (tile shape per problem from the tuning
  * table: a file written by uvt_autotune_f64, or NULL for the built-in one);
  * the split problems run through batched split stages with `slices` moduli.
  * Everything is captured once into a hipGraph on the handle's device.  Each

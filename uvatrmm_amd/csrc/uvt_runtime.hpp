@@ -14,7 +14,7 @@ struct uvt_handle_s {
     int device;
     int cus;
     size_t vram;
-    void* work;        // grows on demand (dtrmm's copy of B)
+    void* work;        // grows on demand (dtrmm's copy of B, dgemm's C where operands overlap)
     size_t work_bytes;
     std::mutex norm_mu; // uvt_inf_norm, one call at a time: its partial maxima
     double* norm_part;  // and their counter (device) and its result (pinned
